@@ -2699,9 +2699,9 @@ __device__ __forceinline__ void persist_barrier(PersistCtl* ctl, unsigned& sense
     __syncthreads();
     if (threadIdx.x == 0) {
         sense ^= 1u;
-        __atomic_thread_fence(__ATOMIC_RELEASE);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         const unsigned arrived =
-            __hip_atomic_fetch_add(&ctl->count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+            __hip_atomic_fetch_add(&ctl->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
         if (arrived == gridDim.x) {
             __hip_atomic_store(&ctl->q[ended], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (ended == 0) __hip_atomic_store(&ctl->q[PERSIST_PHASES - 1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2709,7 +2709,7 @@ __device__ __forceinline__ void persist_barrier(PersistCtl* ctl, unsigned& sense
             __hip_atomic_store(&ctl->sense, sense, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
         } else {
             uint32_t spins = 0;
-            while (__hip_atomic_load(&ctl->sense, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) != sense) {
+            while (__hip_atomic_load(&ctl->sense, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != sense) {
                 if (++spins > (1u << 22)) {
                     atomicOr(&ctl->err, 1u);
                     break;
@@ -2717,7 +2717,7 @@ __device__ __forceinline__ void persist_barrier(PersistCtl* ctl, unsigned& sense
                 __builtin_amdgcn_s_sleep(2);
             }
         }
-        __atomic_thread_fence(__ATOMIC_ACQUIRE);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
 }
