@@ -707,9 +707,35 @@ template <int NX, int CAP = BAND_CAP> constexpr size_t band_lds(unsigned threads
     return (threads / 64) * sizeof(Band<NX, CAP>);
 }
 
+/* Which models take the sweeps split by rows (k_*_rows; three cells per axis, the row-structured
+ * grid). us per launch by particles, nine wavefronts per 64 particles / three / one lane each (the
+ * bonded tissue drifting off the cell faces; in brackets the fluid without bonds):
+ *   pressure   32,768: 17.5 /  29.0 /  66.6;  46,656: 27.4 / 30.5 / 66.4;  54,872: 35.5 / 30.8 / 66.4;
+ *              110,592: 55 / 40 / 68;  262,144: 112 / 68 / 92;  512,000: 237 / 142 / 183
+ *   force      32,768: 15.7 / 21.6 / 45.6;  110,592: 43 / 53 / 53;  140,608: 53 / 66 / 59;
+ *              175,616: 67 / 80 / 63;  262,144: 101 / 110 / 73
+ *             [46,656: 25 / 21 / 41;  64,000: 32 / 22 / 42;  110,592: 50 / 37 / 41;  140,608: 63 / 48 / 47]
+ * Nine wavefronts win while the chip has wavefront slots to spare (49,152 particles are three
+ * workgroups per CU); beyond, three rows per wavefront keep more of the chip busy per byte of
+ * LDS, until the one-lane form fills it too. The force with bonds has no use for three: its two
+ * bond wavefronts then idle longer than the rows take. */
+const int kPressureRows9 = 49152;
+const int kForceRows9 = 147456, kForceRows9NoBonds = 40960, kForceRows3NoBonds = 131072;
+
+bool rows_of_three(const mg_handle* h, const DS& d) { return d.rows && h->g.srch == RS_CELLS; }
+
 /* the pressure and force launches for the handle's SPH kernels */
 void launch_pressure(mg_handle* h, unsigned nb, const DS& d)
 {
+    const bool poly6 = h->sph == MG_SPH_POLY6_SPIKY;
+    auto rows = [&](auto kernel, unsigned waves) {
+        hipLaunchKernelGGL(kernel, dim3(nblk(h->N, 64)), dim3(64 * waves), 0, h->st, d, h->p, h->g);
+    };
+    if (rows_of_three(h, d)) {
+        if (h->N <= kPressureRows9)
+            return poly6 ? rows(k_pressure_rows<MG_SPH_POLY6_SPIKY, 9>, 9) : rows(k_pressure_rows<MG_SPH_REFERENCE, 9>, 9);
+        return poly6 ? rows(k_pressure_rows<MG_SPH_POLY6_SPIKY, 3>, 3) : rows(k_pressure_rows<MG_SPH_REFERENCE, 3>, 3);
+    }
     if (h->sph == MG_SPH_POLY6_SPIKY)
         hipLaunchKernelGGL(k_pressure<MG_SPH_POLY6_SPIKY>, dim3(nb), dim3(256), band_lds<0>(256), h->st, d, h->p, h->g);
     else
@@ -724,6 +750,32 @@ void launch_force(mg_handle* h, unsigned nb, const DS& d, int accumulate)
     else
         hipLaunchKernelGGL(k_force<MG_SPH_REFERENCE>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p, h->g,
                            accumulate);
+}
+
+void launch_force_advance(mg_handle* h, unsigned nb, const DS& d, float dt, int special, float zoff)
+{
+    const bool poly6 = h->sph == MG_SPH_POLY6_SPIKY;
+    auto rows = [&](auto kernel, unsigned waves) {
+        hipLaunchKernelGGL(kernel, dim3(nblk(h->N, 64)), dim3(64 * waves), 0, h->st, d, h->p, h->g, dt, special, zoff);
+    };
+    if (rows_of_three(h, d)) {
+        /* split by rows the bonds come as records only */
+        if (h->B > 0 && d.ETR && h->N <= kForceRows9)
+            return poly6 ? rows(k_force_advance_rows<MG_SPH_POLY6_SPIKY, 1, 9>, 11)
+                         : rows(k_force_advance_rows<MG_SPH_REFERENCE, 1, 9>, 11);
+        if (h->B == 0 && h->N <= kForceRows9NoBonds)
+            return poly6 ? rows(k_force_advance_rows<MG_SPH_POLY6_SPIKY, 0, 9>, 9)
+                         : rows(k_force_advance_rows<MG_SPH_REFERENCE, 0, 9>, 9);
+        if (h->B == 0 && h->N <= kForceRows3NoBonds)
+            return poly6 ? rows(k_force_advance_rows<MG_SPH_POLY6_SPIKY, 0, 3>, 3)
+                         : rows(k_force_advance_rows<MG_SPH_REFERENCE, 0, 3>, 3);
+    }
+    if (poly6)
+        hipLaunchKernelGGL(k_force_advance<MG_SPH_POLY6_SPIKY>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p,
+                           h->g, dt, special, zoff);
+    else
+        hipLaunchKernelGGL(k_force_advance<MG_SPH_REFERENCE>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p,
+                           h->g, dt, special, zoff);
 }
 
 /* The FCONC float4 groups the diffusion sweep reads and the per-TF coefficients
@@ -976,12 +1028,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
         DS d = make_ds(h);
         d.HMR = hm;
         d.ETR = bond_records(h, hm);
-        if (h->sph == MG_SPH_POLY6_SPIKY)
-            hipLaunchKernelGGL(k_force_advance<MG_SPH_POLY6_SPIKY>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d,
-                               h->p, h->g, dt, special, zoff);
-        else
-            hipLaunchKernelGGL(k_force_advance<MG_SPH_REFERENCE>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d,
-                               h->p, h->g, dt, special, zoff);
+        launch_force_advance(h, nb, d, dt, special, zoff);
     }
     {
         PhaseScope ps(h, MG_PH_DIFFUSION);

@@ -660,21 +660,29 @@ __device__ __forceinline__ float axis_gap(float fr, int o, float inv_delta)
 template <int NX, int CAP = BAND_CAP>
 struct Band {
     float4 p[CAP + BAND_PAD];
-    float4 x[NX > 0 ? NX : 1][CAP + BAND_PAD];
+    float4 x[NX > 0 ? NX : 1][NX > 0 ? CAP + BAND_PAD : 1];
 };
 
 
+/* Minimum / maximum over the 64 lanes, wavefront-uniform: DPP shifts inside the 16-lane rows,
+ * then the two row broadcasts, so no step goes through the LDS crossbar (six of its round trips
+ * cost a wavefront about 0.3 us, twice per sweep). Every lane must be active. */
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_min(uint32_t v)
+{
+    return min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, ROWS, 0xF, false));
+}
 __device__ __forceinline__ uint32_t wave_min(uint32_t v)
 {
-    for (int o = 32; o > 0; o >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, o));
-    return __builtin_amdgcn_readfirstlane(v);
+    v = dpp_min<0x111, 0xF>(v); /* row_shr:1, 2, 4, 8: lane 15 of a row holds its minimum */
+    v = dpp_min<0x112, 0xF>(v);
+    v = dpp_min<0x114, 0xF>(v);
+    v = dpp_min<0x118, 0xF>(v);
+    v = dpp_min<0x142, 0xA>(v); /* row_bcast:15 into rows 1 and 3 */
+    v = dpp_min<0x143, 0xC>(v); /* row_bcast:31 into rows 2 and 3 */
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
-
-__device__ __forceinline__ uint32_t wave_max(uint32_t v)
-{
-    for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o));
-    return __builtin_amdgcn_readfirstlane(v);
-}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) { return ~wave_min(~v); }
 
 /* The candidates of one cell, slots [lo, hi), K at a time. getp(j) / getx(j, q) fetch the
  * position / extra field q of slot j; extras are fetched for the hits of a batch only. */
@@ -735,13 +743,12 @@ __device__ __forceinline__ void sweep(const DS& d, const MgGrid& g, Band<NX, CAP
     /* position of x_i inside its own cell (cell units) and cell sizes, for the culling */
     f3 fr = mk3(0.f, 0.f, 0.f), inv = mk3(0.f, 0.f, 0.f);
     if (cull && valid) {
-        const uint32_t own = gc0 + (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
-        const uint32_t cx = own % (uint32_t)g.res[0];
-        const uint32_t cz = (own / (uint32_t)g.res[0]) % (uint32_t)g.res[2];
-        const uint32_t cy = own / ((uint32_t)g.res[0] * (uint32_t)g.res[2]);
-        fr = mk3((pi.x - g.gmin[0]) * g.delta[0] - (float)cx, (pi.y - g.gmin[1]) * g.delta[1] - (float)cy,
-                 (pi.z - g.gmin[2]) * g.delta[2] - (float)cz);
-        inv = mk3(1.0f / g.delta[0], 1.0f / g.delta[1], 1.0f / g.delta[2]);
+        /* the binning's own expressions (insert_one): the slot's cell is their integer part */
+        const float gx = (pi.x - g.gmin[0]) * g.delta[0], gy = (pi.y - g.gmin[1]) * g.delta[1],
+                    gz = (pi.z - g.gmin[2]) * g.delta[2];
+        fr = mk3(gx - truncf(gx), gy - truncf(gy), gz - truncf(gz));
+        /* an ulp of 1 / delta is far below the shrink of the box distance */
+        inv = mk3(__builtin_amdgcn_rcpf(g.delta[0]), __builtin_amdgcn_rcpf(g.delta[1]), __builtin_amdgcn_rcpf(g.delta[2]));
     }
 
     /* band of segment s (wave-uniform); fits == false selects the global path */
@@ -1000,6 +1007,15 @@ __device__ __forceinline__ void sweep(const DS& d, const MgGrid& g, Band<NX, CAP
     }
 }
 
+/* The record (DS::ETW) of a bond the force does not skip: term, strain, break flag */
+__device__ __forceinline__ float4 bond_record(f3 ipos, f3 ivev, float4 pj, float4 vj, float4 bp, float pmass)
+{
+    float strain, abs_dist;
+    const f3 eterm = bond_term(ipos, ivev, xyz(pj), xyz(vj), bp, pmass, &strain, &abs_dist);
+    const uint32_t brk = abs_dist >= bp.x ? 0x80000000u : 0u;
+    return make_float4(eterm.x, eterm.y, eterm.z, __uint_as_float(__float_as_uint(strain) | brk));
+}
+
 /* The bond terms of active slot i's live bond slots, each as the owner's force pass would
  * evaluate it (same operands: the step's positions and veval), recorded for that pass
  * (d.ETW; the record layout is described at DS::ETW). Slots in groups of 4, ascending, the
@@ -1037,15 +1053,47 @@ __device__ __forceinline__ void record_bond_terms(const DS& d, const MgParams& p
         for (int k = 0; k < 4; k++) {
             if (!(g4 & (1u << k))) continue;
             float4 r = make_float4(0.f, 0.f, 0.f, __builtin_nanf(""));
-            if (use[k]) {
-                float strain, abs_dist;
-                const f3 eterm = bond_term(ipos, ivev, xyz(pj[k]), xyz(vj[k]), bp[k], p.pmass, &strain, &abs_dist);
-                const uint32_t brk = abs_dist >= bp[k].x ? 0x80000000u : 0u;
-                r = make_float4(eterm.x, eterm.y, eterm.z, __uint_as_float(__float_as_uint(strain) | brk));
-            }
+            if (use[k]) r = bond_record(ipos, ivev, pj[k], vj[k], bp[k], p.pmass);
             d.ETW[(size_t)(q + k) * N + h] = r;
         }
     }
+}
+
+/* A hit's density term added to csum: the Wendland-C2 kernel of the reference, or the poly6 sum it
+ * keeps in comments (src/fluid_system_cuda.cu:668-672, 695). r / sr for a power-of-two sr is
+ * r * (1 / sr) exactly (a scaling by 2^-k), so that case (inv_sr != 0) skips the correctly rounded
+ * division; the sums are the same bits either way. */
+template <int MODE>
+__device__ __forceinline__ float pressure_inv_sr(const MgParams& p)
+{
+    const uint32_t srb = __float_as_uint(p.psmoothradius);
+    const bool pow2 = (srb & 0x007FFFFFu) == 0u && ((srb >> 23) & 0xFFu) != 0u && ((srb >> 23) & 0xFFu) != 0xFFu;
+    return MODE == MG_SPH_REFERENCE && pow2 ? 1.0f / p.psmoothradius : 0.0f;
+}
+template <int MODE, bool POW2>
+__device__ __forceinline__ void pressure_visit(const MgParams& p, float inv_sr, float dsq, float& csum)
+{
+    if (MODE == MG_SPH_POLY6_SPIKY) {
+        const float c = (p.r2 - dsq) * p.d2;
+        csum += c * c * c;
+        return;
+    }
+    const float r = sqrt_rn(dsq);
+    const float q = POW2 ? r * inv_sr : r / p.psmoothradius;
+    float b = 1.0f - q;
+    b *= b;
+    b *= b;
+    csum += b * (4.0f * q + 1.0f);
+}
+
+/* FPRESS into P.w and FDENSITY (= 1/density) into V.w */
+template <int MODE>
+__device__ __forceinline__ void pressure_store(const DS& d, const MgParams& p, uint32_t i, float sum)
+{
+    sum = sum * p.pmass * (MODE == MG_SPH_POLY6_SPIKY ? p.poly6kern : p.wendlandC2kern);
+    if (sum == 0.0f) sum = 1.0f;
+    ((float*)&d.P[i])[3] = (sum - p.prest_dens) * p.pintstiff;
+    ((float*)&d.V[i])[3] = 1.0f / sum;
 }
 
 /* ------------------------------------------------------------ pressure (a9)
@@ -1067,58 +1115,26 @@ __device__ __forceinline__ void pressure_body(const DS& d, const MgParams& p, co
     const bool valid = gc != MG_GRID_UNDEF;
     gc -= (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
     const f3 pi = valid ? xyz(d.P[i]) : mk3(0.f, 0.f, 0.f);
-    const float sr = p.psmoothradius;
     float sum = 0.0f, csum = 0.0f;
     auto flush = [&]() {
         sum += csum;
         csum = 0.0f;
     };
     auto none = [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); };
-    /* r / sr for a power-of-two sr is r * (1 / sr) exactly (a scaling by 2^-k), so that case
-     * skips the correctly rounded division; the sums are the same bits either way */
-    const uint32_t srb = __float_as_uint(sr);
-    const bool sr_pow2 = (srb & 0x007FFFFFu) == 0u && ((srb >> 23) & 0xFFu) != 0u && ((srb >> 23) & 0xFFu) != 0xFFu;
-    if (MODE == MG_SPH_POLY6_SPIKY) {
-        /* the poly6 sum the reference keeps in comments (src/fluid_system_cuda.cu:668-672, 695) */
-        const float r2 = p.r2, d2 = p.d2;
+    const float inv_sr = pressure_inv_sr<MODE>(p);
+    if (inv_sr != 0.0f) {
         sweep<K, 0, 1, CAP>(
             d, g, bands[threadIdx.x >> 6], valid, gc, pi, p.r2, none,
-            [&](uint32_t, float4, f3, float dsq, const float4*) {
-                const float c = (r2 - dsq) * d2;
-                csum += c * c * c;
-            },
-            flush, i, MG_SKIN_LIM);
-    } else if (sr_pow2) {
-        const float inv_sr = 1.0f / sr;
-        sweep<K, 0, 1, CAP>(
-            d, g, bands[threadIdx.x >> 6], valid, gc, pi, p.r2, none,
-            [&](uint32_t, float4, f3, float dsq, const float4*) {
-                float r = sqrt_rn(dsq);
-                float q = r * inv_sr;
-                float b = 1.0f - q;
-                b *= b;
-                b *= b;
-                csum += b * (4.0f * q + 1.0f);
-            },
+            [&](uint32_t, float4, f3, float dsq, const float4*) { pressure_visit<MODE, true>(p, inv_sr, dsq, csum); },
             flush, i, MG_SKIN_LIM);
     } else {
         sweep<K, 0, 1, CAP>(
             d, g, bands[threadIdx.x >> 6], valid, gc, pi, p.r2, none,
-            [&](uint32_t, float4, f3, float dsq, const float4*) {
-                float r = sqrt_rn(dsq);
-                float q = r / sr;
-                float b = 1.0f - q;
-                b *= b;
-                b *= b;
-                csum += b * (4.0f * q + 1.0f);
-            },
+            [&](uint32_t, float4, f3, float dsq, const float4*) { pressure_visit<MODE, false>(p, inv_sr, dsq, csum); },
             flush, i, MG_SKIN_LIM);
     }
     if (!valid) return;
-    sum = sum * p.pmass * (MODE == MG_SPH_POLY6_SPIKY ? p.poly6kern : p.wendlandC2kern);
-    if (sum == 0.0f) sum = 1.0f;
-    ((float*)&d.P[i])[3] = (sum - p.prest_dens) * p.pintstiff;
-    ((float*)&d.V[i])[3] = 1.0f / sum;
+    pressure_store<MODE>(d, p, i, sum);
     if (d.ETW) record_bond_terms(d, p, i);
 }
 
@@ -1129,6 +1145,353 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_pressure(DS d, MgParams p, MgGrid g)
 {
     extern __shared__ float4 mg_lds[];
     pressure_body<8, BAND_CAP, MODE>(d, p, g, (Band<0>*)mg_lds, xcd_block(), gridDim.x);
+}
+
+/* ---------------------------------------------------- split by rows: small models
+ * A sweep kernel with one lane per particle lasts as long as one wavefront's walk through its
+ * nine rows: below about one wavefront per SIMD (65,536 particles) the chip waits for serial
+ * chains, and 512 particles take as long as 30,000. These kernels give the same 64 particles to
+ * nine wavefronts, one row of the neighbourhood each, in one workgroup. A row leaves its cells'
+ * partial sums in LDS (at most three per row, in cell order; a cell that is not flushed adds +0)
+ * and one wavefront then adds all 27 in the order of the one-lane walk, so the sums keep their
+ * bits. They need the row-structured neighbourhood of three cells per axis. With W = 3 each
+ * wavefront takes three rows in turn. A row's candidates are tested into a mask first and the
+ * mask's bits visited then: half the registers of the one-lane sweep (51 against 102 in the
+ * pressure), so twice the wavefronts per SIMD hide each other's latency. The 512-particle tissue's
+ * pressure 40 -> 12 us and force 32 -> 10 us, at 29,667 particles 63 -> 16 and 44 -> 14; the
+ * host chooses W by size (launch_pressure, launch_force_advance). */
+#define RS_ROWS 9
+#define RS_CELLS 3 /* cells per row */
+#define RS_OCC 5   /* wavefronts per SIMD: at most 96 VGPRs */
+
+/* A row of the neighbourhood seen by a wavefront: the lane's cells [b[k], b[k + 1]) and the
+ * wavefront's slot band [blo, blo + n) in LDS (staged = 0: the band is wider than the stage and
+ * the candidates are read from global memory). */
+struct RsRow {
+    uint32_t b[RS_CELLS + 1];
+    uint32_t blo;
+    bool staged;
+};
+
+/* Row s for the lanes with cell offset gc0 (valid), the band's positions and NX extra fields
+ * staged into `wb`. Called by whole wavefronts; returns false when no lane sweeps. */
+template <int NX, class XLoad>
+__device__ __forceinline__ bool rs_stage(const DS& d, const MgGrid& g, Band<NX>& wb, bool valid, uint32_t gc0, int s,
+                                         XLoad xload, RsRow& r)
+{
+    const uint32_t cmin = wave_min(valid ? gc0 : 0xFFFFFFFFu);
+    const uint32_t cmax = wave_max(valid ? gc0 : 0u);
+    if (cmin == 0xFFFFFFFFu) return false;
+    const uint32_t N = (uint32_t)d.N, lane = __lane_id(), a = (uint32_t)g.adj[s * RS_CELLS];
+    const uint32_t c0 = (valid ? gc0 : cmin) + a;
+    const uint32_t blo = min(d.OFF[cmin + a], N), bhi = min(d.OFF[cmax + a + RS_CELLS], N);
+#pragma unroll
+    for (int k = 0; k <= RS_CELLS; k++) r.b[k] = min(d.OFF[c0 + (uint32_t)k], N);
+    r.blo = blo;
+    r.staged = bhi >= blo && bhi - blo <= (uint32_t)BAND_CAP;
+    if (r.staged) {
+#pragma unroll
+        for (int q = 0; q < BAND_CAP / 64; q++) {
+            const uint32_t j = blo + lane + 64u * (uint32_t)q;
+            if (j < bhi) {
+                wb.p[j - blo] = d.P[j];
+#pragma unroll
+                for (int x = 0; x < NX; x++) wb.x[x][j - blo] = xload(j, x);
+            }
+        }
+        wave_lds_sync();
+    }
+    return true;
+}
+
+/* The candidates [lo, hi) (at most 64) of point pi with 0 < dsq < lim, bit k = slot lo + k */
+template <class GetP>
+__device__ __forceinline__ uint64_t rs_test(uint32_t lo, uint32_t hi, f3 pi, float lim, GetP getp)
+{
+    uint64_t m = 0ull;
+    for (uint32_t j0 = lo; j0 < hi; j0 += 4) {
+        float4 pj[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) pj[q] = getp(j0 + (uint32_t)q);
+        uint32_t nib = 0u;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const f3 dist = pi - xyz(pj[q]);
+            const float dsq = dot3(dist, dist);
+            if (j0 + (uint32_t)q < hi && dsq < lim && dsq > 0.0f) nib |= 1u << q;
+        }
+        m |= (uint64_t)nib << (j0 - lo);
+    }
+    return m;
+}
+
+/* Visits the hits (0 < dsq < lim) of a staged row in ascending slots: `given` (bit k = slot
+ * b[0] + k, a superset of the hits; ~0: none) or the candidates of [flo, fhi) within tlim, 64
+ * slots at a time. end_cell() is called between hits of different cells (at most twice) and
+ * after the last. Returns the recorded superset for slots b[0] .. b[0] + 63 (tested rows). */
+template <int NX, class GetP, class GetX, class Visit, class EndCell>
+__device__ __forceinline__ uint64_t rs_walk(const RsRow& r, uint64_t given, uint32_t flo, uint32_t fhi, f3 pi,
+                                            float lim, float tlim, GetP getp, GetX getx, Visit visit, EndCell end_cell)
+{
+    auto next_bound = [&](uint32_t j) -> uint32_t {
+        uint32_t c = 0xFFFFFFFFu;
+#pragma unroll
+        for (int k = RS_CELLS; k >= 1; k--)
+            if (j < r.b[k]) c = r.b[k];
+        return c;
+    };
+    uint64_t rec = 0ull;
+    uint32_t cnext = next_bound(r.b[0]);
+    const bool test = given == ~0ull;
+    uint32_t base = r.b[0];
+    do {
+        uint64_t m = given;
+        if (test) {
+            const uint32_t lo = max(base, flo), hi = min(base + 64u, fhi);
+            m = lo < hi ? rs_test(lo, hi, pi, tlim, getp) << (lo - base) : 0ull;
+            if (base == r.b[0]) rec = m;
+        }
+        while (m != 0ull) {
+            const uint32_t j = base + (uint32_t)__builtin_ctzll(m);
+            m &= m - 1ull;
+            if (j >= cnext) {
+                end_cell();
+                cnext = next_bound(j);
+            }
+            const float4 pj = getp(j);
+            float4 ex[NX > 0 ? NX : 1];
+#pragma unroll
+            for (int x = 0; x < NX; x++) ex[x] = getx(j, x);
+            const f3 dist = pi - xyz(pj);
+            const float dsq = dot3(dist, dist);
+            if (dsq < lim && dsq > 0.0f) visit(pj, dist, dsq, ex);
+        }
+        base += 64u;
+    } while (test && base < fhi);
+    end_cell();
+    return rec;
+}
+
+/* The candidate range of a row that a culled sweep has to test (the cells within reach of x_i;
+ * `sweep` gives the rule), [b[0], b[3]) when nothing is culled */
+__device__ __forceinline__ void rs_live_range(const DS& d, const MgGrid& g, const RsRow& r, int s, f3 pi, float tlim,
+                                              uint32_t& flo, uint32_t& fhi)
+{
+    flo = r.b[0];
+    fhi = max(r.b[RS_CELLS], r.b[0]);
+    if (!d.cull) return;
+    const float gx = (pi.x - g.gmin[0]) * g.delta[0], gy = (pi.y - g.gmin[1]) * g.delta[1],
+                gz = (pi.z - g.gmin[2]) * g.delta[2];
+    const f3 inv = mk3(__builtin_amdgcn_rcpf(g.delta[0]), __builtin_amdgcn_rcpf(g.delta[1]), __builtin_amdgcn_rcpf(g.delta[2]));
+    const float ay = axis_gap(gy - truncf(gy), s / RS_CELLS - 1, inv.y);
+    const float az = axis_gap(gz - truncf(gz), s % RS_CELLS - 1, inv.z);
+    const float fx = gx - truncf(gx), gyz = ay * ay + az * az;
+    const float xl = axis_gap(fx, -1, inv.x), xr = axis_gap(fx, 1, inv.x);
+    if (!(gyz + xl * xl < tlim)) flo = r.b[1];
+    if (!(gyz + xr * xr < tlim)) fhi = max(r.b[2], flo);
+    if (!(gyz < tlim)) fhi = flo; /* the own column is out of reach, and the others lie farther */
+}
+
+/* the slots a of a 64-bit live mask with a mod W == w (W = 9 or 3) */
+template <int W>
+__device__ __forceinline__ uint64_t rs_share(uint64_t live, uint32_t w)
+{
+    static_assert(W == 9 || W == 3, "rows per wavefront");
+    return live & ((W == 9 ? 0x8040201008040201ull : 0x9249249249249249ull) << w);
+}
+
+/* record_bond_terms for wavefront w's share of slot i's live bond slots, two at a time */
+template <int W>
+__device__ __forceinline__ void rs_record_bonds(const DS& d, const MgParams& p, uint32_t i, uint32_t w)
+{
+    const uint32_t N = (uint32_t)d.N, na = d.ctr[MG_C_ACTIVE];
+    const uint32_t h = d.HOME[i];
+    uint64_t live = rs_share<W>(d.LIVE[h], w);
+    if (live == 0ull) return;
+    const f3 ipos = xyz(d.P[i]), ivev = xyz(d.V[i]);
+    while (live) {
+        uint32_t jc[2];
+        size_t bi[2];
+        float4 bp[2], pj[2], vj[2];
+        bool has[2], use[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            has[k] = live != 0ull;
+            bi[k] = (size_t)(has[k] ? __builtin_ctzll(live) : 0) * N + h;
+            live &= live - 1ull;
+            jc[k] = has[k] ? d.SLOT[d.BPARTNER[bi[k]]] : MG_NONE;
+            bp[k] = has[k] ? d.BPAR[bi[k]] : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            use[k] = jc[k] < na && !((double)bp[k].y < 0.000000001);
+            pj[k] = vj[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (use[k]) {
+                pj[k] = d.P[jc[k]];
+                vj[k] = d.V[jc[k]];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            if (!has[k]) continue;
+            float4 r = make_float4(0.f, 0.f, 0.f, __builtin_nanf(""));
+            if (use[k]) r = bond_record(ipos, ivev, pj[k], vj[k], bp[k], p.pmass);
+            d.ETW[bi[k]] = r;
+        }
+    }
+}
+
+/* contributePressure / computePressure split by rows; writes what k_pressure writes */
+template <int MODE, int W>
+__global__ __launch_bounds__(64 * W, RS_OCC) void k_pressure_rows(DS d, MgParams p, MgGrid g)
+{
+    constexpr int PER = RS_ROWS / W; /* rows per wavefront */
+    __shared__ Band<0> bands[W];
+    __shared__ float part[RS_ROWS * RS_CELLS][64];
+    const uint32_t bid = xcd_block(), lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (d.ZERO)
+        for (uint32_t z = bid * blockDim.x + threadIdx.x; z < d.zero_n; z += gridDim.x * blockDim.x) d.ZERO[z] = 0u;
+    if (d.HMW && bid == 0 && threadIdx.x == 0) d.ctr[MG_C_SKIN] = 0u;
+    const uint32_t i = bid * 64u + lane;
+    uint32_t gc = (i < d.ctr[MG_C_ACTIVE]) ? d.GCELL[i] : MG_GRID_UNDEF;
+    const bool valid = gc != MG_GRID_UNDEF;
+    gc -= (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
+    const f3 pi = valid ? xyz(d.P[i]) : mk3(0.f, 0.f, 0.f);
+    const float inv_sr = pressure_inv_sr<MODE>(p), tlim = d.HMW ? fmaxf(MG_SKIN_LIM, p.r2) : p.r2;
+    auto none = [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); };
+    for (int q = 0; q < PER; q++) {
+        const int s = (int)w * PER + q;
+#pragma unroll
+        for (int k = 0; k < RS_CELLS; k++) part[s * RS_CELLS + k][lane] = 0.0f;
+        RsRow r;
+        if (q > 0) wave_lds_sync(); /* the previous row's reads are done */
+        if (!rs_stage<0>(d, g, bands[w], valid, gc, s, none, r) || !valid) continue;
+        uint32_t flo, fhi, nflush = 0u;
+        rs_live_range(d, g, r, s, pi, tlim, flo, fhi);
+        float csum = 0.0f;
+        auto visit = [&](float4, f3, float dsq, const float4*) {
+            if (inv_sr != 0.0f) pressure_visit<MODE, true>(p, inv_sr, dsq, csum);
+            else pressure_visit<MODE, false>(p, inv_sr, dsq, csum);
+        };
+        auto end_cell = [&]() {
+            if (nflush < RS_CELLS) part[s * RS_CELLS + nflush][lane] = csum;
+            nflush++;
+            csum = 0.0f;
+        };
+        uint64_t rec;
+        if (r.staged)
+            rec = rs_walk<0>(r, ~0ull, flo, fhi, pi, p.r2, tlim, [&](uint32_t j) { return bands[w].p[j - r.blo]; }, none,
+                             visit, end_cell);
+        else
+            rec = rs_walk<0>(r, ~0ull, flo, fhi, pi, p.r2, tlim, [&](uint32_t j) { return d.P[j]; }, none, visit,
+                             end_cell);
+        if (d.HMW) d.HMW[(size_t)s * d.N + i] = r.b[RS_CELLS] - r.b[0] > 64u ? ~0ull : rec;
+    }
+    if (valid && d.ETW) rs_record_bonds<W>(d, p, i, w);
+    __syncthreads();
+    if (w != 0u || !valid) return;
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < RS_ROWS * RS_CELLS; k++) sum += part[k][lane];
+    pressure_store<MODE>(d, p, i, sum);
+}
+
+/* A hit's fluid force added to cf (P_i, V_i the particle, Pj, Vj the neighbour) */
+template <int MODE>
+__device__ __forceinline__ void force_visit(const MgParams& p, float4 P_i, float4 V_i, float4 Pj, float4 Vj, f3 dist,
+                                            float dsq, f3& cf)
+{
+    if (MODE == MG_SPH_POLY6_SPIKY) {
+        cf = cf + fluid_term_poly6(dist, dsq, p, P_i.w, Pj.w, V_i.w, Vj.w, xyz(V_i), xyz(Vj));
+    } else {
+        float r, inv_r;
+        sqrt_rcp_rn(dsq, r, inv_r);
+        cf = cf + fluid_term(dist, r, inv_r, p.psmoothradius, P_i.w, Pj.w, V_i.w, Vj.w, xyz(V_i), xyz(Vj), p.psurface_t);
+    }
+}
+/* the reference's force tests dsq < 1 (src/fluid_system_cuda.cu:3203); the Mueller kernels have
+ * the smoothing radius as support */
+template <int MODE>
+__device__ __forceinline__ float force_lim(const MgParams& p)
+{
+    return MODE == MG_SPH_POLY6_SPIKY ? p.r2 : 1.0f;
+}
+
+/* The own live slots' bond records of home h, written by the pressure pass of the same positions:
+ * integrators, force and breaking in slot order, with the operations of the evaluation. Groups
+ * of 4 slots, their records loaded together. Returns minus the sum of the terms. */
+__device__ __forceinline__ f3 own_records(const DS& d, const MgParams& p, uint32_t h, uint64_t live)
+{
+    const int N = d.N;
+    const bool freeze = p.freeze != 0;
+    f3 force = mk3(0.0f, 0.0f, 0.0f);
+    while (live) {
+        const int q = (__ffsll((long long)live) - 1) & ~3;
+        const uint32_t g4 = (uint32_t)(live >> q) & 0xFu;
+        live &= ~(0xFull << q);
+        float4 r[4];
+        float2 inc[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            r[k] = make_float4(0.f, 0.f, 0.f, __builtin_nanf(""));
+            inc[k] = make_float2(0.f, 0.f);
+            if (g4 & (1u << k)) {
+                const size_t bi = (size_t)(q + k) * N + h;
+                r[k] = d.ETR[bi];
+                inc[k] = d.BINT[bi];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (r[k].w != r[k].w) continue; /* not a live slot, or one the force skips */
+            const size_t bi = (size_t)(q + k) * N + h;
+            const uint32_t wbits = __float_as_uint(r[k].w);
+            const float strain = __uint_as_float(wbits & 0x7FFFFFFFu);
+            if (!d.dry) {
+                float2 v = inc[k];
+                v.x = v.x + strain * strain;
+                v.y = v.y + strain;
+                d.BINT[bi] = v;
+            }
+            const f3 eterm = mk3(r[k].x, r[k].y, r[k].z);
+            if (!has_nan3(eterm)) force = force - eterm;
+            if ((wbits >> 31) && !freeze && !d.dry) ((float*)&d.BPAR[bi])[1] = 0.0f;
+        }
+    }
+    return force;
+}
+
+/* F plus the owners' records of the incoming bonds e0 .. e1 - 1 in order (an inactive owner's
+ * record is stale: its slot decides, as in the evaluation); `first`, when given, holds the first
+ * four entries of INC. */
+__device__ __forceinline__ f3 incoming_records(const DS& d, uint32_t na, uint32_t e0, uint32_t e1, f3 F,
+                                               const uint32_t* first = nullptr)
+{
+    const int N = d.N, B = d.B;
+    uint32_t packed[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) packed[k] = first ? first[k] : d.INC[min(e0 + (uint32_t)k, e1 - 1u)];
+    for (uint32_t e = e0; e < e1; e += 4) {
+        uint32_t ks[4];
+        float4 r[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t kh = packed[k] / (uint32_t)B, b = packed[k] - kh * (uint32_t)B;
+            ks[k] = d.SLOT[kh];
+            r[k] = d.ETR[(size_t)b * N + kh];
+        }
+        if (e + 4u < e1)
+#pragma unroll
+            for (int k = 0; k < 4; k++) packed[k] = d.INC[min(e + 4u + (uint32_t)k, e1 - 1u)];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (!(e + (uint32_t)k < e1 && ks[k] < na && r[k].w == r[k].w)) continue;
+            const f3 eterm = mk3(r[k].x, r[k].y, r[k].z);
+            if (!has_nan3(eterm)) F = F + eterm;
+        }
+    }
+    return F;
 }
 
 /* --------------------------------------------------------------- force (a10)
@@ -1159,7 +1522,6 @@ __device__ __forceinline__ f3 force_one(const DS& d, const MgParams& p, const Mg
         V_i = d.V[i];
     }
     const f3 ipos = xyz(P_i), ivev = xyz(V_i);
-    const float ipress = P_i.w, idens = V_i.w;
     const bool freeze = p.freeze != 0;
 
     f3 force = mk3(0.0f, 0.0f, 0.0f);
@@ -1167,7 +1529,7 @@ __device__ __forceinline__ f3 force_one(const DS& d, const MgParams& p, const Mg
      * while the previous group's partner positions load (software pipeline). The own bond
      * terms are summed after the fluid sweep (into their own total, as before it), and the
      * first group's partner slots are fetched before the sweep. */
-    uint64_t live = valid ? d.LIVE[h] : 0ull;
+    uint64_t live = valid && !d.ETR ? d.LIVE[h] : 0ull;
     int q = 0;
     uint32_t g4 = 0, j[4];
     auto next_group = [&]() {
@@ -1177,7 +1539,6 @@ __device__ __forceinline__ f3 force_one(const DS& d, const MgParams& p, const Mg
             g4 = (uint32_t)(live >> q) & 0xFu;
             live &= ~(0xFull << q);
         }
-        if (d.ETR) return; /* the records replace the partners' positions */
 #pragma unroll
         for (int k = 0; k < 4; k++) j[k] = (g4 & (1u << k)) ? d.SLOT[d.BPARTNER[(size_t)(q + k) * N + h]] : MG_NONE;
     };
@@ -1188,22 +1549,11 @@ __device__ __forceinline__ f3 force_one(const DS& d, const MgParams& p, const Mg
 #pragma unroll
         for (int k = 0; k < 4; k++) first[k] = d.INC[min(e0 + (uint32_t)k, e1 - 1u)];
     /* fluid terms: per-cell sums added in gridAdj order */
-    const float sr = p.psmoothradius, st = p.psurface_t;
     f3 fsum = mk3(0.0f, 0.0f, 0.0f), cf = mk3(0.0f, 0.0f, 0.0f);
-    /* the reference's force tests dsq < 1 (src/fluid_system_cuda.cu:3203); the Mueller kernels
-     * have the smoothing radius as support */
-    const float flim = MODE == MG_SPH_POLY6_SPIKY ? p.r2 : 1.0f;
     sweep<4, 1, 2>(
-        d, g, wb, valid, gc, ipos, flim, [&](uint32_t j, int) { return d.V[j]; },
+        d, g, wb, valid, gc, ipos, force_lim<MODE>(p), [&](uint32_t j, int) { return d.V[j]; },
         [&](uint32_t, float4 Pj, f3 dist, float dsq, const float4* x) {
-            const float4 Vj = x[0];
-            if (MODE == MG_SPH_POLY6_SPIKY) {
-                cf = cf + fluid_term_poly6(dist, dsq, p, ipress, Pj.w, idens, Vj.w, ivev, xyz(Vj));
-            } else {
-                float r, inv_r;
-                sqrt_rcp_rn(dsq, r, inv_r);
-                cf = cf + fluid_term(dist, r, inv_r, sr, ipress, Pj.w, idens, Vj.w, ivev, xyz(Vj), st);
-            }
+            force_visit<MODE>(p, P_i, V_i, Pj, x[0], dist, dsq, cf);
         },
         [&]() {
             fsum = fsum + cf;
@@ -1214,41 +1564,8 @@ __device__ __forceinline__ f3 force_one(const DS& d, const MgParams& p, const Mg
     float4 bp[4];
     float2 in[4];
     if (d.ETR) {
-        /* the pressure pass's records of the own live slots: integrators, force, breaking in
-         * the order below (the same operations on the same values as the evaluation) */
-        while (g4) {
-            const int qc = q;
-            const uint32_t gc4 = g4;
-            float4 r[4];
-            float2 inc[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                r[k] = make_float4(0.f, 0.f, 0.f, __builtin_nanf(""));
-                inc[k] = make_float2(0.f, 0.f);
-                if (gc4 & (1u << k)) {
-                    const size_t bi = (size_t)(qc + k) * N + h;
-                    r[k] = d.ETR[bi];
-                    inc[k] = d.BINT[bi];
-                }
-            }
-            next_group();
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if (r[k].w != r[k].w) continue; /* not a live slot, or one the force skips */
-                const size_t bi = (size_t)(qc + k) * N + h;
-                const uint32_t wbits = __float_as_uint(r[k].w);
-                const float strain = __uint_as_float(wbits & 0x7FFFFFFFu);
-                if (!d.dry) {
-                    float2 v = inc[k];
-                    v.x = v.x + strain * strain;
-                    v.y = v.y + strain;
-                    d.BINT[bi] = v;
-                }
-                const f3 eterm = mk3(r[k].x, r[k].y, r[k].z);
-                if (!has_nan3(eterm)) force = force - eterm;
-                if ((wbits >> 31) && !freeze && !d.dry) ((float*)&d.BPAR[bi])[1] = 0.0f;
-            }
-        }
+        if (valid) force = own_records(d, p, h, d.LIVE[h]);
+        g4 = 0;
     }
     auto records = [&]() {
 #pragma unroll
@@ -1318,29 +1635,7 @@ __device__ __forceinline__ f3 force_one(const DS& d, const MgParams& p, const Mg
 #pragma unroll
         for (int k = 0; k < 4; k++) packed[k] = d.INC[min(e + (uint32_t)k, e1 - 1u)];
     };
-    if (d.ETR) {
-        /* the owners' records of the incoming bonds (an inactive owner's record is stale: its
-         * slot decides, as in the evaluation) */
-        uint32_t packed[4] = {first[0], first[1], first[2], first[3]};
-        for (uint32_t e = e0; valid && e < e1; e += 4) {
-            uint32_t ks[4];
-            float4 r[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t kh = packed[k] / (uint32_t)B, b = packed[k] - kh * (uint32_t)B;
-                ks[k] = d.SLOT[kh];
-                r[k] = d.ETR[(size_t)b * N + kh];
-            }
-            if (e + 4u < e1) entries(e + 4u, packed);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if (!(e + (uint32_t)k < e1 && ks[k] < na && r[k].w == r[k].w)) continue;
-                const f3 eterm = mk3(r[k].x, r[k].y, r[k].z);
-                if (!has_nan3(eterm)) F = F + eterm;
-            }
-        }
-        return F;
-    }
+    if (d.ETR) return valid && e0 < e1 ? incoming_records(d, na, e0, e1, F, first) : F;
     if (valid && e0 < e1) fetch_in(first);
     for (uint32_t e = e0; valid && e < e1; e += 4) {
         bool use[4];
@@ -1575,6 +1870,130 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_force_advance(DS d, MgParams p, MgGrid g, 
 {
     extern __shared__ float4 mg_lds[];
     force_advance_body<MODE>(d, p, g, (Band<1>*)mg_lds, dt, xcd_block(), special, zoff);
+}
+
+/* ------------------------------------------------- force + advance split by rows
+ * k_force_advance for 64 particles per workgroup: a wavefront per row of the neighbourhood (see
+ * RS_ROWS) and, with bonds, two more: wavefront 9 sums the own bonds' records and updates their
+ * integrators, wavefront 10 fetches the incoming bonds' records (the first RS_INC of each
+ * particle into registers) while the rows are swept, then adds everything up in force_one's
+ * order and advances. Bonds come as the pressure pass's records only (d.ETR). */
+#define RS_INC 12
+template <int MODE, int BONDS, int W>
+__global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? RS_OCC : 3) void k_force_advance_rows(DS d, MgParams p, MgGrid g, float dt,
+                                                                                   int special, float zoff)
+{
+    constexpr int PER = RS_ROWS / W; /* rows per wavefront */
+    __shared__ Band<1> bands[W];
+    __shared__ float part[RS_ROWS * RS_CELLS][3][64];
+    __shared__ float own[3][64];
+    const uint32_t bid = xcd_block(), lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t i = bid * 64u + lane, N = (uint32_t)d.N, B = (uint32_t)d.B;
+    const uint32_t na = d.ctr[MG_C_ACTIVE];
+    const uint32_t gc = (i < na) ? d.GCELL[i] : MG_GRID_UNDEF;
+    const bool valid = gc != MG_GRID_UNDEF;
+    const uint32_t last = BONDS ? W + 1u : 0u; /* the wavefront that adds up and advances */
+    uint32_t e0 = 0, e1 = 0;
+    f3 in[BONDS ? RS_INC : 1];
+    if (w < (uint32_t)W) {
+        const uint32_t gc0 = gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
+        float4 P_i = make_float4(0.f, 0.f, 0.f, 0.f), V_i = P_i;
+        if (valid) {
+            P_i = d.P[i];
+            V_i = d.V[i];
+        }
+        const f3 pi = xyz(P_i);
+        const float lim = force_lim<MODE>(p);
+        auto getv = [&](uint32_t j, int) { return d.V[j]; };
+        for (int q = 0; q < PER; q++) {
+            const int s = (int)w * PER + q;
+            uint64_t hm = ~0ull;
+            if (valid && d.HMR) hm = d.HMR[(size_t)s * N + i];
+#pragma unroll
+            for (int k = 0; k < RS_CELLS; k++)
+#pragma unroll
+                for (int c = 0; c < 3; c++) part[s * RS_CELLS + k][c][lane] = 0.0f;
+            RsRow r;
+            if (q > 0) wave_lds_sync(); /* the previous row's reads are done */
+            if (!rs_stage<1>(d, g, bands[w], valid, gc0, s, getv, r) || !valid) continue;
+            uint32_t flo, fhi, nflush = 0u;
+            rs_live_range(d, g, r, s, pi, lim, flo, fhi);
+            f3 cf = mk3(0.0f, 0.0f, 0.0f);
+            auto visit = [&](float4 Pj, f3 dist, float dsq, const float4* x) {
+                force_visit<MODE>(p, P_i, V_i, Pj, x[0], dist, dsq, cf);
+            };
+            auto end_cell = [&]() {
+                if (nflush < RS_CELLS) {
+                    part[s * RS_CELLS + nflush][0][lane] = cf.x;
+                    part[s * RS_CELLS + nflush][1][lane] = cf.y;
+                    part[s * RS_CELLS + nflush][2][lane] = cf.z;
+                }
+                nflush++;
+                cf = mk3(0.0f, 0.0f, 0.0f);
+            };
+            if (r.staged)
+                rs_walk<1>(r, hm, flo, fhi, pi, lim, lim, [&](uint32_t j) { return bands[w].p[j - r.blo]; },
+                           [&](uint32_t j, int x) { return bands[w].x[x][j - r.blo]; }, visit, end_cell);
+            else
+                rs_walk<1>(r, hm, flo, fhi, pi, lim, lim, [&](uint32_t j) { return d.P[j]; }, getv, visit, end_cell);
+        }
+    } else if (BONDS && w == (uint32_t)W) {
+        f3 force = mk3(0.0f, 0.0f, 0.0f);
+        if (valid) {
+            const uint32_t h = d.HOME[i];
+            force = own_records(d, p, h, d.LIVE[h]);
+        }
+        own[0][lane] = force.x;
+        own[1][lane] = force.y;
+        own[2][lane] = force.z;
+    } else if (BONDS) {
+        if (valid) {
+            const uint32_t h = d.HOME[i];
+            e0 = d.INC_OFF[h];
+            e1 = d.INC_OFF[h + 1];
+        }
+#pragma unroll
+        for (int k = 0; k < RS_INC; k++) in[k] = mk3(0.0f, 0.0f, 0.0f);
+        if (e0 < e1) {
+            uint32_t packed[RS_INC], ks[RS_INC];
+            float4 r[RS_INC];
+#pragma unroll
+            for (int k = 0; k < RS_INC; k++) packed[k] = d.INC[min(e0 + (uint32_t)k, e1 - 1u)];
+#pragma unroll
+            for (int k = 0; k < RS_INC; k++) {
+                const uint32_t kh = packed[k] / B, b = packed[k] - kh * B;
+                ks[k] = d.SLOT[kh];
+                r[k] = d.ETR[(size_t)b * N + kh];
+            }
+            /* a term that force_one leaves out adds +0 here: FFORCE is a sum that starts at +0,
+             * so it is never -0 and keeps its bits */
+#pragma unroll
+            for (int k = 0; k < RS_INC; k++) {
+                const f3 t = mk3(r[k].x, r[k].y, r[k].z);
+                if (e0 + (uint32_t)k < e1 && ks[k] < na && r[k].w == r[k].w && !has_nan3(t)) in[k] = t;
+            }
+        }
+    }
+    __syncthreads();
+    if (w != last) return;
+    f3 F = mk3(0.0f, 0.0f, 0.0f);
+    if (valid) {
+        f3 fsum = mk3(0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (int k = 0; k < RS_ROWS * RS_CELLS; k++)
+            fsum = fsum + mk3(part[k][0][lane], part[k][1][lane], part[k][2][lane]);
+        f3 force = mk3(0.0f, 0.0f, 0.0f);
+        if (BONDS) force = mk3(own[0][lane], own[1][lane], own[2][lane]);
+        force = force + fsum * p.pmass;
+        F = mk3(0.0f, 0.0f, 0.0f) + force;
+        if (BONDS) {
+#pragma unroll
+            for (int k = 0; k < RS_INC; k++) F = F + in[k];
+            if (e0 + RS_INC < e1) F = incoming_records(d, na, e0 + RS_INC, e1, F);
+        }
+    }
+    if (i < N) advance_other_half(d, p, dt, i, valid, F, special, zoff);
 }
 
 /* ----------------------------------------------------------- diffusion (a12)
