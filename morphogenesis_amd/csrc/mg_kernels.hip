@@ -2248,6 +2248,266 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_diffuse_genes_insert(DS d, MgParams p, MgG
     diffuse_genes_insert_body<NG>(d, p, g, gen, dp, genes, (Band<NG>*)mg_lds, xcd_block());
 }
 
+/* ---------------------------------- diffusion, genes and insert split by rows
+ * The fused k_diffuse_genes_insert (PART = RS_DIFFUSE | RS_GENES | RS_INSERT), or one of its phase
+ * kernels (RS_DIFFUSE, RS_GENES), for 64 particles per workgroup of nine wavefronts.
+ *
+ * Diffusion adds its terms hit by hit, without per-cell sums, so the rows cannot be summed apart.
+ * The wavefronts find the hits of a row each instead and write them (weight, slot) into the
+ * particle's list in LDS, in visit order (the rows' counts give each its place; a recorded
+ * candidate that is not a hit is marked and skipped; more than RS_LIST entries take several
+ * rounds). One wavefront per float4 group of FCONC then walks the list: no search in its loop,
+ * loads four entries ahead, and a wavefront's time is its busiest lane's total, not the sum over
+ * the rows of each row's busiest lane.
+ *
+ * Genes: a wavefront sums the activity of genes w and w + 9 and counts their activations; then
+ * four wavefronts add the secretions of four TFs each, genes in order, while wavefront 8 counts
+ * the epigenetic states down and stores them. Wavefront 7 bins the particle.
+ *
+ * 512 particles 34 -> 19 us, 29,667 46 -> 20 (a lane per particle was one serial chain: sweep,
+ * then every gene in turn); with the chip full it loses, as most wavefronts wait while few
+ * work (64,000 particles 50 -> 54 us), so larger models keep a lane per particle. */
+#define RS_DIFFUSE 1
+#define RS_GENES 2
+#define RS_INSERT 4
+#define RS_LIST 48
+template <int PART>
+__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_rows(DS d, MgParams p, MgGrid g, MgGenome gen,
+                                                                       DiffPlan dp)
+{
+    union Stage {
+        struct {
+            Band<0> bands[RS_ROWS];
+            uint2 list[RS_LIST][64]; /* (weight, slot); NaN: recorded, not a hit */
+        } a;
+        struct {
+            float act[MG_NUM_GENES][64];
+            uint32_t depi[MG_NUM_GENES][64];
+        } b;
+    };
+    __shared__ Stage sh;
+    __shared__ uint32_t cnt[RS_ROWS][64];
+    __shared__ float conc[MG_NUM_TF][64];
+    const uint32_t bid = xcd_block(), lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t i = bid * 64u + lane, N = (uint32_t)d.N;
+    const uint32_t na = d.ctr[MG_C_ACTIVE], nump = d.ctr[MG_C_NUM_POINTS];
+    const uint32_t gc = (i < na) ? d.GCELL[i] : MG_GRID_UNDEF;
+    const bool valid = gc != MG_GRID_UNDEF;
+
+    /* wavefronts 0 .. 3 own a float4 group of FCONC each, the first dp.ng of them the plan's */
+    uint32_t grp = 0;
+    if (w < 4u) {
+        uint32_t unused = 0xFu;
+        for (int q = 0; q < dp.ng; q++) unused &= ~(1u << dp.grp[q]);
+        if ((int)w < dp.ng) {
+            grp = (uint32_t)dp.grp[w];
+        } else {
+            for (uint32_t q = (uint32_t)dp.ng; q < w; q++) unused &= unused - 1u;
+            grp = (uint32_t)__builtin_ctz(unused);
+        }
+    }
+    const float4* C4 = (const float4*)d.CONC;
+    float4 cur = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (w < 4u && i < N) cur = C4[(size_t)i * 4u + grp];
+
+    if (PART & RS_DIFFUSE) {
+        const float d2 = p.psimscale * p.psimscale, r2 = p.r2 / d2;
+        const bool hm_ok = d.HMR != nullptr && d.ctr[MG_C_SKIN] == 0u && r2 == 1.0f;
+        f3 pi = mk3(0.f, 0.f, 0.f);
+        uint64_t m = 0ull;
+        if (valid) {
+            pi = xyz(d.P[i]);
+            m = hm_ok ? d.HMR[(size_t)w * N + i] : ~0ull;
+        }
+        RsRow r;
+        const bool any = dp.ng > 0 && rs_stage<0>(d, g, sh.a.bands[w], valid,
+                                                  gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1), (int)w,
+                                                  [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); }, r);
+        const bool test = m == ~0ull; /* the row's candidates have to be tested, 64 slots at a time */
+        auto getp_band = [&](uint32_t j) { return sh.a.bands[w].p[j - r.blo]; };
+        auto getp_global = [&](uint32_t j) { return d.P[j]; };
+        uint32_t n = 0u;
+        if (any && valid) {
+            if (test) {
+                for (uint32_t b = r.b[0]; b < r.b[RS_CELLS]; b += 64u) {
+                    const uint32_t hi = min(b + 64u, r.b[RS_CELLS]);
+                    m = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
+                    n += (uint32_t)__builtin_popcountll(m);
+                }
+            } else {
+                n = (uint32_t)__builtin_popcountll(m);
+            }
+        }
+        cnt[w][lane] = n;
+        __syncthreads();
+        uint32_t at = 0u, tot = 0u;
+#pragma unroll
+        for (uint32_t q = 0; q < RS_ROWS; q++) {
+            const uint32_t c = cnt[q][lane];
+            if (q < w) at += c;
+            tot += c;
+        }
+        const uint32_t most = wave_max(tot);
+        float nw[4] = {0.f, 0.f, 0.f, 0.f};
+        const bool adds = (int)w < dp.ng;
+        for (uint32_t base = 0u; base < most; base += RS_LIST) {
+            if (any && valid && n != 0u) {
+                uint32_t k = at;
+                uint32_t b = r.b[0];
+                do {
+                    uint64_t mm = m;
+                    /* a row of one window keeps the mask of the count */
+                    if (test && r.b[RS_CELLS] - r.b[0] > 64u) {
+                        const uint32_t hi = min(b + 64u, r.b[RS_CELLS]);
+                        mm = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
+                    }
+                    while (mm != 0ull) {
+                        const uint32_t j = b + (uint32_t)__builtin_ctzll(mm);
+                        mm &= mm - 1ull;
+                        const uint32_t e = k - base; /* wraps below the round's entries */
+                        k++;
+                        if (e >= RS_LIST) continue;
+                        const float4 pj = r.staged ? getp_band(j) : getp_global(j);
+                        const f3 dist = pi - xyz(pj);
+                        const float dsq = dot3(dist, dist);
+                        const float cc = dsq < r2 && dsq > 0.0f ? (r2 - dsq) * d2 : __builtin_nanf("");
+                        sh.a.list[e][lane] = make_uint2(__float_as_uint(cc), j);
+                    }
+                    b += 64u;
+                } while (test && b < r.b[RS_CELLS]);
+            }
+            __syncthreads();
+            if (adds) {
+                const uint32_t ne = tot > base ? min(tot - base, (uint32_t)RS_LIST) : 0u;
+                for (uint32_t e0 = 0; e0 < ne; e0 += 4) {
+                    uint2 en[4];
+                    float4 cn[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) en[q] = sh.a.list[min(e0 + (uint32_t)q, ne - 1u)][lane];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) cn[q] = C4[(size_t)en[q].y * 4u + grp];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const float cc = __uint_as_float(en[q].x);
+                        if (!(e0 + (uint32_t)q < ne && cc == cc)) continue;
+                        const float c4[4] = {cn[q].x, cn[q].y, cn[q].z, cn[q].w};
+                        const float u4[4] = {cur.x, cur.y, cur.z, cur.w};
+#pragma unroll
+                        for (int t = 0; t < 4; t++)
+                            if (dp.dm & (1u << (4u * w + (uint32_t)t))) nw[t] += dp.D[4u * w + (uint32_t)t] * cc * (c4[t] - u4[t]);
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (valid && w < 4u) {
+            cur.x = (float)gen.tf_breakdown_rate[4u * grp + 0u] * (cur.x + nw[0]);
+            cur.y = (float)gen.tf_breakdown_rate[4u * grp + 1u] * (cur.y + nw[1]);
+            cur.z = (float)gen.tf_breakdown_rate[4u * grp + 2u] * (cur.z + nw[2]);
+            cur.w = (float)gen.tf_breakdown_rate[4u * grp + 3u] * (cur.w + nw[3]);
+        }
+    }
+    if (!(PART & RS_GENES)) {
+        if (w < 4u && i < N) ((float4*)d.CONC2)[(size_t)i * 4u + grp] = cur;
+        return;
+    }
+
+    /* genes: the membership of the last sort */
+    const bool listed = d.ctr[MG_C_LISTS] != 0u && i < nump;
+    const uint32_t m = listed ? d.GMASK[i] : 0u;
+    const bool tally = (m & 4u) && i < na;
+    if (w < 4u) {
+        conc[4u * grp + 0u][lane] = cur.x;
+        conc[4u * grp + 1u][lane] = cur.y;
+        conc[4u * grp + 2u][lane] = cur.z;
+        conc[4u * grp + 3u][lane] = cur.w;
+    }
+    for (uint32_t q = w; q < MG_NUM_GENES; q += RS_ROWS) sh.b.depi[q][lane] = 0u;
+    /* lane q < 16: gene q's secretion and activation counts and first entries */
+    const uint32_t gq = lane & 15u;
+    const int nsec = gen.secrete[gq][2 * MG_NUM_TF], sec_tf = gen.secrete[gq][0], sec_rate = gen.secrete[gq][1];
+    const int nact = gen.activate[gq][2 * MG_NUM_GENES], act_to = gen.activate[gq][0], act_thr = gen.activate[gq][1];
+    uint32_t h = 0u, epi[MG_NUM_GENES], was[MG_NUM_GENES];
+    if (w == RS_ROWS - 1u && i < nump) {
+        h = d.HOME[i];
+#pragma unroll
+        for (int k = 0; k < MG_NUM_GENES; k++) epi[k] = d.EPIGEN[(size_t)k * N + h];
+    }
+    __syncthreads();
+    {
+        float c[MG_NUM_TF];
+#pragma unroll
+        for (int t = 0; t < MG_NUM_TF; t++) c[t] = conc[t][lane];
+        for (uint32_t gene = w; gene < MG_NUM_GENES; gene += RS_ROWS) {
+            float activity = 0.0f;
+#pragma unroll
+            for (int tf = 0; tf < MG_NUM_TF; tf++)
+                if (gen.sensitivity[gene][tf] != 0u) activity += (float)gen.sensitivity[gene][tf] * c[tf];
+            sh.b.act[gene][lane] = activity;
+            const int numL = __builtin_amdgcn_readlane(nact, (int)gene);
+            for (int j = 0; j < numL && j < MG_NUM_GENES; j++) {
+                const int other = j == 0 ? __builtin_amdgcn_readlane(act_to, (int)gene) : gen.activate[gene][j * 2];
+                const int threshold = j == 0 ? __builtin_amdgcn_readlane(act_thr, (int)gene) : gen.activate[gene][j * 2 + 1];
+                if (other < 0 || other >= MG_NUM_GENES) continue;
+                if ((m & (1u << gene)) && (float)threshold < activity) atomicAdd(&sh.b.depi[other][lane], 1u);
+            }
+        }
+    }
+    __syncthreads();
+    if (w < 4u) {
+        float dc[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int gene = 0; gene < MG_NUM_GENES; gene++) {
+            const int numTF = __builtin_amdgcn_readlane(nsec, gene);
+            for (int j = 0; j < numTF && j < MG_NUM_TF; j++) {
+                const int tf = j == 0 ? __builtin_amdgcn_readlane(sec_tf, gene) : gen.secrete[gene][j * 2];
+                const int rate = j == 0 ? __builtin_amdgcn_readlane(sec_rate, gene) : gen.secrete[gene][j * 2 + 1];
+                if (tf < 0 || tf >= MG_NUM_TF || (uint32_t)tf >> 2 != grp) continue;
+                const float add = ((float)rate * sh.b.act[gene][lane]) * p.secrete_scale;
+                if (m & (1u << gene)) {
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+                        if ((tf & 3) == t) dc[t] += add;
+                }
+            }
+        }
+        if (tally) {
+            cur.x = cur.x + dc[0];
+            cur.y = cur.y + dc[1];
+            cur.z = cur.z + dc[2];
+            cur.w = cur.w + dc[3];
+        }
+        float4* out = (float4*)((PART & RS_DIFFUSE) ? d.CONC2 : d.CONC);
+        if (i < N && ((PART & RS_DIFFUSE) || tally)) out[(size_t)i * 4u + grp] = cur;
+    } else if (w == RS_ROWS - 1u) {
+        uint32_t mnext = 0u;
+        if (i < nump) {
+#pragma unroll
+            for (int k = 0; k < MG_NUM_GENES; k++) was[k] = epi[k];
+#pragma unroll
+            for (int k = 0; k < MG_NUM_GENES; k++) {
+                const int delay = (int)epi[k];
+                if ((m & (1u << k)) && 0 < delay && delay < MG_INT_MAX) {
+                    epi[k]--;
+                    if (delay == 1 && k + 1 < MG_NUM_GENES && epi[k + 1 < MG_NUM_GENES ? k + 1 : k])
+                        epi[k + 1 < MG_NUM_GENES ? k + 1 : k] = gen.delay[k + 1 < MG_NUM_GENES ? k + 1 : k];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < MG_NUM_GENES; k++) {
+                if (tally) epi[k] += sh.b.depi[k][lane];
+                /* most states do not change in a step: store only those that did */
+                if (epi[k] != was[k]) d.EPIGEN[(size_t)k * N + h] = epi[k];
+                if (epi[k] > 0u) mnext |= 1u << k;
+            }
+        }
+        if ((PART & RS_INSERT) && i < N) d.GMN[i] = mnext;
+    } else if ((PART & RS_INSERT) && w == RS_ROWS - 2u) {
+        /* binning rewrites GCELL, which every wavefront has read before the barriers above */
+        insert_one(d, g, i, i < N, i < N ? d.P[i] : make_float4(0.f, 0.f, 0.f, 0.f), d.CNTN, nullptr);
+    }
+}
+
 /* -------------------------------------------------------- bond formation
  * contribFindBonds (src/fluid_system_cuda.cu:1938-1976) over the cells gc + gridAdj[c] for one
  * bond slot of the particle at slot i (home h), seen from the point x (the particle's position

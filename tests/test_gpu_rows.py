@@ -1,7 +1,8 @@
 """The sweeps split by rows (nine or three wavefronts per 64 particles, `launch_pressure`,
-`launch_force_advance`) against the FP32 oracle, bit for bit, at the sizes
+`launch_force_advance`, `launch_diffuse_rows`) against the FP32 oracle, bit for bit, at the sizes
 where they can go wrong: workgroups of one, 63, 64 and 65 particles; cells so full that a row has
-more than 64 candidates, a wavefront's band exceeds its stage; particles with more incoming bonds than the force keeps in registers; and both
+more than 64 candidates, a wavefront's band exceeds its stage and a particle's hit list takes
+several rounds; particles with more incoming bonds than the force keeps in registers; and both
 sides of each size at which the split changes."""
 import sys
 
@@ -34,7 +35,7 @@ def scene(dims, b, genes=True, spacing=0.5, drift=0.0, seed=5):
     ((4, 4, 4), 32, True, 0.5, 5.0, 8),       # 64
     ((5, 13, 1), 0, False, 0.5, 5.0, 8),      # 65, no bonds
     ((9, 10, 11), 6, True, 0.22, 0.0, 6),     # ~94 particles per cell: wide rows, unstaged bands
-    ((9, 9, 9), 32, True, 0.3, 50.0, 6), 
+    ((9, 9, 9), 32, True, 0.3, 50.0, 6),      # fast: diffusion tests its candidates itself
     ((10, 10, 10), 0, False, 0.22, 50.0, 6),
 ])
 def test_small_models_match_oracle(built, dims, b, genes, spacing, drift, steps):
@@ -76,6 +77,7 @@ def test_many_incoming_bonds(built):
 @pytest.mark.parametrize("dims,b,genes,sph", [
     ((32, 32, 40), 0, False, 0), ((32, 32, 41), 0, False, 1),   # force without bonds: nine, three
     ((32, 32, 48), 6, True, 0), ((32, 32, 49), 6, True, 1),     # pressure: nine, three
+    ((32, 32, 56), 6, True, 0), ((32, 32, 57), 6, True, 0),     # diffusion: by rows, a lane each
     ((48, 48, 56), 0, False, 0), ((48, 48, 57), 0, False, 0),   # force without bonds: three, a lane each
     ((48, 48, 64), 6, True, 0), ((48, 48, 65), 6, True, 0),     # force with bonds: nine, a lane each
 ])
