@@ -20,7 +20,8 @@ struct mg_net {
     hipStream_t st = nullptr;
     MlpDev* dev = nullptr;
     float *params = nullptr, *grads = nullptr, *m = nullptr, *v = nullptr;
-    __bf16* wb = nullptr; /* bf16 copy of the whole parameter vector (only the W parts are read) */
+    __bf16* wb = nullptr; /* bf16 copy of the parameter vector (the backward pass reads W2 and W3) */
+    __bf16* wt = nullptr; /* its matrices in [out][in] order (the forward pass) */
     int adam_t = 0;
     uint64_t version = 1; /* bumped on every parameter / normalisation change */
     float mu[MLP_IN], inv_sigma[MLP_IN];
@@ -32,12 +33,12 @@ struct mg_net {
     std::vector<uint64_t> used_prefix; /* rows with a nonzero mask before each row (rows + 1) */
     float* loss_dev = nullptr;         /* per-step losses of mg_net_train, downloaded at its end */
     size_t loss_cap = 0;
-    /* work buffers for minibatches of up to cap rows */
+    /* work buffers of a training pass over up to cap rows */
     size_t cap = 0;
-    __bf16 *Xn = nullptr, *A1b = nullptr, *A2b = nullptr, *dYb = nullptr, *dZ2b = nullptr, *dZ1b = nullptr;
-    float *Z1 = nullptr, *Z2 = nullptr, *Y = nullptr, *dY = nullptr, *dA2 = nullptr, *dZ2 = nullptr;
-    float *dA1 = nullptr, *dZ1 = nullptr, *part = nullptr, *lpart = nullptr;
-    size_t part_cap = 0;
+    NetOps ops = {};
+    float *lpart = nullptr, *part = nullptr, *bpart = nullptr;
+    float* Y = nullptr;                      /* mg_net_forward's outputs */
+    size_t y_cap = 0;
     std::vector<void*> allocs;
 };
 
@@ -57,7 +58,7 @@ unsigned gblk(size_t n) { return (unsigned)((n + 255) / 256); }
 /* bf16 copies and packed inference parameters from the fp32 master weights */
 int net_sync(mg_net* n)
 {
-    hipLaunchKernelGGL(k_to_bf16, dim3(gblk(kNParams)), dim3(256), 0, n->st, n->params, n->wb, kNParams);
+    hipLaunchKernelGGL(k_net_weights, dim3(gblk(kNParams)), dim3(256), 0, n->st, n->params, n->wb, n->wt);
     /* W1 in input order; W2 and W3 in the order the previous layer's results sit in registers */
     hipLaunchKernelGGL(k_pack_frag, dim3(gblk(MLP_IN * MLP_H)), dim3(256), 0, n->st, n->params + kOffW1, MLP_IN,
                        MLP_H, n->dev->w1f, 0);
@@ -78,112 +79,69 @@ int net_sync(mg_net* n)
     return MG_OK;
 }
 
-int net_reserve(mg_net* n, size_t S)
+unsigned net_blocks(size_t rows) { return (unsigned)((rows + NET_ROWS - 1) / NET_ROWS); }
+
+/* splits of the sum over rows in the weight gradients, at most 64, of about 1,024 rows or more */
+const int kNetSplits = 64;
+void net_splits(size_t rows, int* splits, int* kper)
 {
-    if (S <= n->cap) return MG_OK;
-    CHK(nalloc(n, &n->Xn, S * MLP_IN));
-    CHK(nalloc(n, &n->A1b, S * MLP_H));
-    CHK(nalloc(n, &n->A2b, S * MLP_H));
-    CHK(nalloc(n, &n->dYb, S * MLP_OUT));
-    CHK(nalloc(n, &n->dZ2b, S * MLP_H));
-    CHK(nalloc(n, &n->dZ1b, S * MLP_H));
-    CHK(nalloc(n, &n->Z1, S * MLP_H));
-    CHK(nalloc(n, &n->Z2, S * MLP_H));
-    CHK(nalloc(n, &n->Y, S * MLP_OUT));
-    CHK(nalloc(n, &n->dY, S * MLP_OUT));
-    CHK(nalloc(n, &n->dA2, S * MLP_H));
-    CHK(nalloc(n, &n->dZ2, S * MLP_H));
-    CHK(nalloc(n, &n->dA1, S * MLP_H));
-    CHK(nalloc(n, &n->dZ1, S * MLP_H));
-    CHK(nalloc(n, &n->lpart, gblk(S)));
+    const int chunks = (int)((rows + 31) / 32);
+    const int n = std::min(chunks, (int)std::min<size_t>(kNetSplits, std::max<size_t>(1, rows / 1024)));
+    *kper = (int)(((rows + n - 1) / n + 31) / 32) * 32;
+    *splits = (int)((rows + *kper - 1) / *kper);
+}
+
+int net_reserve(mg_net* n, size_t rows)
+{
+    if (rows <= n->cap) return MG_OK;
+    const size_t S = (size_t)net_blocks(rows) * NET_ROWS;
+    CHK(nalloc(n, &n->ops.x, S * MLP_IN));
+    CHK(nalloc(n, &n->ops.a1, S * MLP_H));
+    CHK(nalloc(n, &n->ops.a2, S * MLP_H));
+    CHK(nalloc(n, &n->ops.dz1, S * MLP_H));
+    CHK(nalloc(n, &n->ops.dz2, S * MLP_H));
+    CHK(nalloc(n, &n->ops.dy, S * MLP_OUT));
+    CHK(nalloc(n, &n->ops.fz1, S * MLP_H));
+    CHK(nalloc(n, &n->ops.fz2, S * MLP_H));
+    CHK(nalloc(n, &n->ops.fy, S * MLP_OUT));
+    CHK(nalloc(n, &n->lpart, S / NET_ROWS));
+    if (!n->part) {
+        CHK(nalloc(n, &n->part, kNetSplits * kNParams));
+        CHK(nalloc(n, &n->bpart, 256 * NET_BIASES));
+    }
     n->cap = S;
     return MG_OK;
 }
 
-/* C[M x N] = A(m,k) B(k,n), K split into `splits` chunks reduced in order */
-int gemm(mg_net* n, int M, int N, int K, const __bf16* A, long sam, long sak, const __bf16* B, long sbk, long sbn,
-         float* C, int splits)
+NetWeights net_weights(const mg_net* n)
 {
-    splits = std::max(1, std::min(splits, (K + 31) / 32));
-    const int kper = ((K + splits - 1) / splits + 31) / 32 * 32;
-    splits = (K + kper - 1) / kper;
-    const size_t mn = (size_t)M * N;
-    if (splits > 1 && mn * splits > n->part_cap) {
-        CHK(nalloc(n, &n->part, mn * splits));
-        n->part_cap = mn * splits;
-    }
-    float* out = splits > 1 ? n->part : C;
-    hipLaunchKernelGGL(k_gemm_bf16, dim3((N + 63) / 64, (M + 63) / 64, splits), dim3(256), 0, n->st, M, N, K, A, sam,
-                       sak, B, sbk, sbn, out, kper);
-    if (splits > 1) hipLaunchKernelGGL(k_gemm_reduce, dim3(gblk(mn)), dim3(256), 0, n->st, n->part, splits, mn, C);
-    HIPCHK(hipGetLastError());
-    return MG_OK;
+    NetWeights W;
+    W.w1t = n->wt + kOffW1; W.w2t = n->wt + kOffW2; W.w3t = n->wt + kOffW3;
+    W.w2 = n->wb + kOffW2; W.w3 = n->wb + kOffW3;
+    W.b1 = n->params + kOffB1; W.b2 = n->params + kOffB2; W.b3 = n->params + kOffB3;
+    W.mu = n->dev->mu; W.inv_sigma = n->dev->inv_sigma;
+    return W;
 }
 
-/* forward (and with grads, backward) over rows [r0, r0 + S) of the training set */
-/* one thread: the blocks' loss partials summed in order in double, as a float (the host's
- * sum of the same partials gives the same bits) */
-__global__ void k_sum_partials(const float* __restrict__ part, unsigned count, float* __restrict__ out)
+/* forward and backward over rows [r0, r0 + S) of the training set: gradients into n->grads and,
+ * where `loss` (device) is given, the mean loss; with adam.update the weights are updated */
+int net_backward(mg_net* n, size_t r0, size_t S, float* loss, const AdamStep& adam)
 {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double s = 0.0;
-    for (unsigned k = 0; k < count; k++) s += part[k];
-    *out = (float)s;
-}
-
-/* forward (and backward) over rows [r0, r0 + S); the mean loss goes to the host (loss_host)
- * or stays on the device (loss_dev), either may be null */
-int net_pass(mg_net* n, size_t r0, size_t S, bool backward, float* loss_host, float* loss_dev = nullptr)
-{
-    CHK(net_reserve(n, S));
-    const float* X = n->X + r0 * MLP_IN;
-    float *mu_d = n->dev->mu, *is_d = n->dev->inv_sigma;
-    const __bf16 *W1 = n->wb + kOffW1, *W2 = n->wb + kOffW2, *W3 = n->wb + kOffW3;
-    hipLaunchKernelGGL(k_normalize_rows, dim3(gblk(S * MLP_IN)), dim3(256), 0, n->st, X, mu_d, is_d, n->Xn, S);
-    CHK(gemm(n, (int)S, MLP_H, MLP_IN, n->Xn, MLP_IN, 1, W1, MLP_H, 1, n->Z1, 1));
-    hipLaunchKernelGGL(k_bias_silu, dim3(gblk(S * MLP_H)), dim3(256), 0, n->st, n->Z1, n->params + kOffB1, MLP_H, S,
-                       n->A1b, 1);
-    CHK(gemm(n, (int)S, MLP_H, MLP_H, n->A1b, MLP_H, 1, W2, MLP_H, 1, n->Z2, 1));
-    hipLaunchKernelGGL(k_bias_silu, dim3(gblk(S * MLP_H)), dim3(256), 0, n->st, n->Z2, n->params + kOffB2, MLP_H, S,
-                       n->A2b, 1);
-    CHK(gemm(n, (int)S, MLP_OUT, MLP_H, n->A2b, MLP_H, 1, W3, MLP_OUT, 1, n->Y, 1));
-    hipLaunchKernelGGL(k_bias_silu, dim3(gblk(S * MLP_OUT)), dim3(256), 0, n->st, n->Y, n->params + kOffB3, MLP_OUT,
-                       S, (__bf16*)nullptr, 0);
-    if (!backward) return MG_OK;
-    /* count of masked rows in this window, for the mean (from the prefix taken at load) */
+    /* rows with a nonzero mask in this window, for the mean (from the prefix taken at load) */
     const double cnt = (double)(n->used_prefix[r0 + S] - n->used_prefix[r0]);
     const float inv = cnt > 0 ? (float)(1.0 / cnt) : 0.f;
-    const unsigned lb = gblk(S);
-    hipLaunchKernelGGL(k_mse, dim3(lb), dim3(256), 0, n->st, n->Y, n->T + r0 * MLP_OUT_REAL, n->mask + r0, S, inv, n->dY,
-                       n->dYb, n->lpart);
-    float* g = n->grads;
-    const int ks = (int)std::min<size_t>(64, std::max<size_t>(1, S / 1024));
-    /* layer 3 */
-    CHK(gemm(n, MLP_H, MLP_OUT, (int)S, n->A2b, 1, MLP_H, n->dYb, MLP_OUT, 1, g + kOffW3, ks));
-    hipLaunchKernelGGL(k_colsum, dim3(MLP_OUT), dim3(256), 0, n->st, n->dY, S, MLP_OUT, g + kOffB3);
-    CHK(gemm(n, (int)S, MLP_H, MLP_OUT, n->dYb, MLP_OUT, 1, W3, 1, MLP_OUT, n->dA2, 1));
-    hipLaunchKernelGGL(k_silu_back, dim3(gblk(S * MLP_H)), dim3(256), 0, n->st, n->dA2, n->Z2, S * MLP_H, n->dZ2, n->dZ2b);
-    /* layer 2 */
-    CHK(gemm(n, MLP_H, MLP_H, (int)S, n->A1b, 1, MLP_H, n->dZ2b, MLP_H, 1, g + kOffW2, ks));
-    hipLaunchKernelGGL(k_colsum, dim3(MLP_H), dim3(256), 0, n->st, n->dZ2, S, MLP_H, g + kOffB2);
-    CHK(gemm(n, (int)S, MLP_H, MLP_H, n->dZ2b, MLP_H, 1, W2, 1, MLP_H, n->dA1, 1));
-    hipLaunchKernelGGL(k_silu_back, dim3(gblk(S * MLP_H)), dim3(256), 0, n->st, n->dA1, n->Z1, S * MLP_H, n->dZ1, n->dZ1b);
-    /* layer 1 */
-    CHK(gemm(n, MLP_IN, MLP_H, (int)S, n->Xn, 1, MLP_IN, n->dZ1b, MLP_H, 1, g + kOffW1, ks));
-    hipLaunchKernelGGL(k_colsum, dim3(MLP_H), dim3(256), 0, n->st, n->dZ1, S, MLP_H, g + kOffB1);
+    CHK(net_reserve(n, S));
+    int splits = 1, kper = 32;
+    net_splits(S, &splits, &kper);
+    const unsigned blocks = net_blocks(S);
+    hipLaunchKernelGGL(k_net_pass<true>, dim3(blocks), dim3(256), sizeof(NetLds), n->st, net_weights(n),
+                       n->X + r0 * MLP_IN, n->T + r0 * MLP_OUT_REAL, n->mask + r0, S, inv, n->ops, n->lpart,
+                       (float*)nullptr);
+    hipLaunchKernelGGL(k_net_grad, dim3((unsigned)(splits * NET_TASKS / 4 + NET_BIAS_BLOCKS)), dim3(256), 0, n->st,
+                       n->ops, S, splits, kper, n->part, n->bpart);
+    hipLaunchKernelGGL(k_net_reduce, dim3((unsigned)(gblk(kNParams) + NET_BIASES)), dim3(256), 0, n->st, n->part, splits,
+                       n->bpart, n->lpart, (int)blocks, n->grads, loss, adam, n->params, n->m, n->v, n->wb, n->wt);
     HIPCHK(hipGetLastError());
-    if (loss_dev) {
-        hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(64), 0, n->st, n->lpart, lb, loss_dev);
-        HIPCHK(hipGetLastError());
-    }
-    if (loss_host) {
-        std::vector<float> lp(lb);
-        HIPCHK(hipMemcpyAsync(lp.data(), n->lpart, lb * 4, hipMemcpyDeviceToHost, n->st));
-        HIPCHK(hipStreamSynchronize(n->st));
-        double s = 0;
-        for (float x : lp) s += x;
-        *loss_host = (float)s;
-    }
     return MG_OK;
 }
 
@@ -267,12 +225,22 @@ int mg_net_create(mg_net** out, uint64_t seed)
     if (r == MG_OK) r = nalloc(n, &n->m, kNParams);
     if (r == MG_OK) r = nalloc(n, &n->v, kNParams);
     if (r == MG_OK) r = nalloc(n, &n->wb, kNParams);
+    if (r == MG_OK) r = nalloc(n, &n->wt, kNParams);
+    if (r == MG_OK) r = nalloc(n, &n->loss_dev, 1);
     if (r != MG_OK) return fail(r);
     if (hipFuncSetAttribute((const void*)k_mlp_apply, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)sizeof(MlpLds)) != hipSuccess) {
         set_err("mg_net_create: the inference kernel's LDS (%zu bytes) is not available", sizeof(MlpLds));
         return fail(MG_ERR_HIP);
     }
+    if (hipFuncSetAttribute((const void*)k_net_pass<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)sizeof(NetLds)) != hipSuccess ||
+        hipFuncSetAttribute((const void*)k_net_pass<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)sizeof(NetLds)) != hipSuccess) {
+        set_err("mg_net_create: the training kernel's LDS (%zu bytes) is not available", sizeof(NetLds));
+        return fail(MG_ERR_HIP);
+    }
+    n->loss_cap = 1;
     /* Xavier-uniform (Glorot & Bengio, 2010) over the real fan-in / fan-out; padding zero */
     std::vector<float> p(kNParams, 0.f);
     uint64_t s = seed;
@@ -357,10 +325,9 @@ int mg_net_load_data(mg_net* n, const float* X, const float* T, const float* mas
 int mg_net_grad(mg_net* n, size_t row0, size_t rows, float* grads_out, float* loss_out)
 {
     if (!n || rows == 0 || row0 + rows > n->rows) { set_err("mg_net_grad: rows outside the data"); return MG_ERR_ARG; }
-    CHK(net_pass(n, row0, rows, true, loss_out));
-    if (grads_out) {
-        HIPCHK(hipMemcpyAsync(grads_out, n->grads, kNParams * 4, hipMemcpyDeviceToHost, n->st));
-    }
+    CHK(net_backward(n, row0, rows, n->loss_dev, AdamStep{}));
+    if (grads_out) HIPCHK(hipMemcpyAsync(grads_out, n->grads, kNParams * 4, hipMemcpyDeviceToHost, n->st));
+    if (loss_out) HIPCHK(hipMemcpyAsync(loss_out, n->loss_dev, 4, hipMemcpyDeviceToHost, n->st));
     HIPCHK(hipStreamSynchronize(n->st));
     return MG_OK;
 }
@@ -369,7 +336,14 @@ int mg_net_grad(mg_net* n, size_t row0, size_t rows, float* grads_out, float* lo
 int mg_net_forward(mg_net* n, size_t row0, size_t rows, float* y_out)
 {
     if (!n || !y_out || rows == 0 || row0 + rows > n->rows) { set_err("mg_net_forward: rows outside the data"); return MG_ERR_ARG; }
-    CHK(net_pass(n, row0, rows, false, nullptr));
+    if (rows > n->y_cap) {
+        CHK(nalloc(n, &n->Y, rows * MLP_OUT));
+        n->y_cap = rows;
+    }
+    hipLaunchKernelGGL(k_net_pass<false>, dim3(net_blocks(rows)), dim3(256), sizeof(NetLds), n->st, net_weights(n),
+                       n->X + row0 * MLP_IN, (const float*)nullptr, (const float*)nullptr, rows, 0.0f, NetOps{},
+                       (float*)nullptr, n->Y);
+    HIPCHK(hipGetLastError());
     std::vector<float> y(rows * MLP_OUT);
     HIPCHK(hipMemcpyAsync(y.data(), n->Y, rows * MLP_OUT * 4, hipMemcpyDeviceToHost, n->st));
     HIPCHK(hipStreamSynchronize(n->st));
@@ -396,13 +370,9 @@ int mg_net_train(mg_net* n, int steps, size_t batch, float lr, uint64_t seed, fl
     for (int k = 0; k < steps; k++) {
         const size_t r0 = (w % std::max<size_t>(windows, 1)) * batch;
         w++;
-        CHK(net_pass(n, r0, batch, true, nullptr, loss_out ? n->loss_dev + k : nullptr));
         n->adam_t++;
         const float c1 = 1.0f - std::pow(b1, (float)n->adam_t), c2 = 1.0f - std::pow(b2, (float)n->adam_t);
-        hipLaunchKernelGGL(k_adam, dim3(gblk(kNParams)), dim3(256), 0, n->st, n->params, n->grads, n->m, n->v,
-                           kNParams, lr, b1, b2, eps, c1, c2);
-        hipLaunchKernelGGL(k_to_bf16, dim3(gblk(kNParams)), dim3(256), 0, n->st, n->params, n->wb, kNParams);
-        HIPCHK(hipGetLastError());
+        CHK(net_backward(n, r0, batch, loss_out ? n->loss_dev + k : nullptr, AdamStep{1, lr, b1, b2, eps, c1, c2}));
     }
     if (loss_out && steps > 0)
         HIPCHK(hipMemcpyAsync(loss_out, n->loss_dev, (size_t)steps * 4, hipMemcpyDeviceToHost, n->st));

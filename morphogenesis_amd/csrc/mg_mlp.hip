@@ -22,8 +22,9 @@
  * B[8 (l / 16) + e][l % 16] (e = 0..7), and the 16 x 16 fp32 result lane l holds
  * D[4 (l / 16) + r][l % 16] (r = 0..3).
  *
- * Training uses a generic bf16 GEMM with split-K partials reduced in a fixed order, and
- * fp32 Adam on fp32 master weights; inference is one fused kernel per step.
+ * Training runs a minibatch forward and backward in one kernel (bf16 operands, fp32
+ * accumulation, gradient partials reduced in a fixed order) with fp32 Adam on fp32 master
+ * weights; inference is two kernels per step.
  */
 
 #define MLP_IN 64
@@ -382,224 +383,410 @@ __global__ __launch_bounds__(256) void k_mlp_apply(const MlpDev* __restrict__ ne
     if (l == 0 && nfall) atomicAdd(fallbacks, nfall);
 }
 
-/* ------------------------------------------------------------ training GEMM
- * C[s][m][n] = sum over k in split s of A(m, k) * B(k, n), A(m, k) = A[m * sam + k * sak],
- * B(k, n) = B[k * sbk + n * sbn] (bf16), fp32 partials per split; k_gemm_reduce adds the
- * splits in order (deterministic). 64 x 64 block tile, four 32 x 32 wave tiles, K step 32. */
-__global__ __launch_bounds__(256) void k_gemm_bf16(int M, int N, int K, const __bf16* __restrict__ A, long sam,
-                                                   long sak, const __bf16* __restrict__ Bm, long sbk, long sbn,
-                                                   float* __restrict__ C, int kper)
+/* ------------------------------------------------------------ training
+ * A step of Adam is three launches: k_net_pass takes a minibatch forward and backward, k_net_grad
+ * multiplies out the gradients, k_net_reduce adds their partials and updates the weights. (The
+ * layer-by-layer form they replaced, a GEMM with elementwise and column-sum kernels over
+ * intermediates in memory, took 21 launches and 316 us per step of 16,384 rows; its sums over
+ * rows are kept in their order, because a last-bit difference in a gradient grows, through the
+ * bf16 rounding of the weights, to 1e-4 of them within 60 steps.) Now 22 + 14 + 7 us at 16,384
+ * rows, 2.6 GFLOP: the pass is bound by its chain of six layers with a barrier each (one workgroup
+ * of four wavefronts per CU), the other two by the 55 MB of operands and partials.
+ *
+ * k_net_pass: a workgroup takes 64 rows through all layers, the activations in LDS and the
+ * pre-activations in registers. Products are transposed, D[neuron][row] = W^T[neuron][k]
+ * X^T[k][row], so wavefront w owns the 32 neurons from 32 w of each hidden layer for all 64 rows:
+ * the weights are read once per workgroup, straight from memory in fragments of 16 contiguous
+ * bytes per lane ([out][in] order forward, [in][out] backward), the rows' operands from LDS. The
+ * weight gradients sum over rows, so their operands are kept transposed ([neuron][row]) and leave
+ * in tiles of 16 neurons by 32 rows (1 KB), which k_net_grad reads whole. */
+#define NET_ROWS 64
+#define NET_LD(k) ((k) + 8) /* row stride of an LDS operand with k columns (bf16) */
+struct NetLds {
+    __bf16 Xr[NET_ROWS][NET_LD(MLP_IN)];
+    __bf16 XT[MLP_IN][NET_LD(NET_ROWS)];
+    union {
+        __bf16 A1r[NET_ROWS][NET_LD(MLP_H)];   /* dead after layer 2 */
+        __bf16 dZ1T[MLP_H][NET_LD(NET_ROWS)];
+    };
+    __bf16 A1T[MLP_H][NET_LD(NET_ROWS)];
+    union {
+        __bf16 A2r[NET_ROWS][NET_LD(MLP_H)];   /* dead after layer 3 */
+        __bf16 dZ2r[NET_ROWS][NET_LD(MLP_H)];
+    };
+    __bf16 A2T[MLP_H][NET_LD(NET_ROWS)];
+    __bf16 dZ2T[MLP_H][NET_LD(NET_ROWS)];
+    __bf16 dYr[NET_ROWS][NET_LD(32)];          /* columns 16 .. 31 zero (K padding) */
+    __bf16 dYT[MLP_OUT][NET_LD(NET_ROWS)];
+    float loss[4];
+};
+
+/* What a pass leaves for the gradients: operand tiles [row chunk][neuron tile][16][32] in bf16, and
+ * dZ1, dZ2 [rows][128], dY [rows][16] in fp32 for the bias gradients */
+struct NetOps {
+    __bf16 *x, *a1, *a2, *dz1, *dz2, *dy;
+    float *fz1, *fz2, *fy;
+};
+
+/* bf16 weights of a pass: [out][in] (forward) and [in][out] (backward) */
+struct NetWeights {
+    const __bf16 *w1t, *w2t, *w3t; /* [128][64], [128][128], [16][128] */
+    const __bf16 *w2, *w3;         /* [128][128], [128][16] */
+    const float *b1, *b2, *b3;
+    const float *mu, *inv_sigma;
+};
+
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4_t;
+
+/* four neurons n .. n + 3 of a row into the row-major and the transposed operand */
+template <int KR, int KT>
+__device__ __forceinline__ void net_put(__bf16 (*rows)[KR], __bf16 (*cols)[KT], int row, int n, const float v[4])
 {
-    __shared__ __bf16 As[64][32 + 8];
-    __shared__ __bf16 Bs[64][32 + 8]; /* transposed: Bs[n][k] */
-    const int t = threadIdx.x, w = t >> 6, l = t & 63;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const int k_lo = blockIdx.z * kper, k_hi = min(K, k_lo + kper);
-    const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-    f32x4_t acc[2][2];
+    bf16x4_t b;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int r = 0; r < 4; r++) b[r] = to_bf16(v[r]);
+    if (rows) *(bf16x4_t*)&rows[row][n] = b;
 #pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    /* each thread stages one 8-element chunk of A and one of B per K step: 8 consecutive k of
-     * a row when the operand is contiguous in k, else 8 consecutive m (n) of a k when it is
-     * contiguous in m (n), with one 16-byte load when the chunk is in range and aligned */
-    const bool a_k = sak == 1, a_m = !a_k && sam == 1;
-    const bool b_k = sbk == 1, b_n = !b_k && sbn == 1;
-    auto aligned = [](const __bf16* q) { return ((uintptr_t)q & 15u) == 0u; };
-    for (int k0 = k_lo; k0 < k_hi; k0 += 32) {
-        if (a_k || a_m) {
-            const int r = a_k ? t >> 2 : (t & 7) * 8, c = a_k ? (t & 3) * 8 : t >> 3;
-            const int m = m0 + r, k = k0 + c;
-            const __bf16* q = A + (long)m * sam + (long)k * sak;
-            const bool full = a_k ? (m < M && k + 8 <= k_hi) : (k < k_hi && m + 8 <= M);
-            if (full && aligned(q)) {
-                const bf16x8_t v = *(const bf16x8_t*)q;
+    for (int r = 0; r < 4; r++) cols[n + r][row] = b[r];
+}
+
+/* the block's operand tiles (TILES x 16 neurons, 64 rows: two chunks of 32) to memory */
+template <int TILES>
+__device__ __forceinline__ void net_tiles(const __bf16 (*T)[NET_LD(NET_ROWS)], __bf16* __restrict__ out, size_t blk, int t)
+{
+    uint4* o = (uint4*)out + blk * (size_t)(2 * TILES * 64);
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    if (a_k) As[r][c + e] = v[e];
-                    else As[r + e][c] = v[e];
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int mm = a_k ? m : m + e, kk = a_k ? k + e : k;
-                    As[a_k ? r : r + e][a_k ? c + e : c] =
-                        (mm < M && kk < k_hi) ? A[(long)mm * sam + (long)kk * sak] : to_bf16(0.0f);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int idx = t * 8 + e;
-                const int r = idx >> 5, c = idx & 31;
-                const int m = m0 + r, k = k0 + c;
-                As[r][c] = (m < M && k < k_hi) ? A[(long)m * sam + (long)k * sak] : to_bf16(0.0f);
-            }
-        }
-        if (b_k || b_n) {
-            const int r = b_k ? t >> 2 : (t & 7) * 8, c = b_k ? (t & 3) * 8 : t >> 3;
-            const int n = n0 + r, k = k0 + c;
-            const __bf16* q = Bm + (long)k * sbk + (long)n * sbn;
-            const bool full = b_k ? (n < N && k + 8 <= k_hi) : (k < k_hi && n + 8 <= N);
-            if (full && aligned(q)) {
-                const bf16x8_t v = *(const bf16x8_t*)q;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    if (b_k) Bs[r][c + e] = v[e];
-                    else Bs[r + e][c] = v[e];
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int nn = b_k ? n : n + e, kk = b_k ? k + e : k;
-                    Bs[b_k ? r : r + e][b_k ? c + e : c] =
-                        (nn < N && kk < k_hi) ? Bm[(long)kk * sbk + (long)nn * sbn] : to_bf16(0.0f);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const int idx = t * 8 + e;
-                const int r = idx >> 5, c = idx & 31;
-                const int n = n0 + r, k = k0 + c;
-                Bs[r][c] = (n < N && k < k_hi) ? Bm[(long)k * sbk + (long)n * sbn] : to_bf16(0.0f);
-            }
-        }
-        __syncthreads();
-        const int row = l & 15, kq = l >> 4;
-#pragma unroll
-        for (int a = 0; a < 2; a++)
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const bf16x8_t av = lds8(&As[wm + a * 16 + row][8 * kq]);
-                const bf16x8_t bv = lds8(&Bs[wn + b * 16 + row][8 * kq]);
-                acc[a][b] = mfma16(av, bv, acc[a][b]);
-            }
-        __syncthreads();
+    for (int k = t; k < 2 * TILES * 64; k += 256) {
+        const int l = k & 63, nt = (k >> 6) % TILES, kc = (k >> 6) / TILES;
+        o[k] = *(const uint4*)&T[16 * nt + (l & 15)][32 * kc + 8 * (l >> 4)];
     }
-    float* Cs = C + (size_t)blockIdx.z * M * N;
-    const int kq = l >> 4;
+}
+
+/* offsets of the parameter vector: W1 b1 W2 b2 W3 b3 */
+#define NET_W1 0
+#define NET_B1 (NET_W1 + MLP_IN * MLP_H)
+#define NET_W2 (NET_B1 + MLP_H)
+#define NET_B2 (NET_W2 + MLP_H * MLP_H)
+#define NET_W3 (NET_B2 + MLP_H)
+#define NET_B3 (NET_W3 + MLP_H * MLP_OUT)
+#define NET_PARAMS (NET_B3 + MLP_OUT)
+
+/* BACK: the operands of the gradients into O and the loss into lpart[block] (times inv_count);
+ * else the outputs into Y [rows][16] */
+template <bool BACK>
+__global__ __launch_bounds__(256, 1) void k_net_pass(NetWeights W, const float* __restrict__ X,
+                                                     const float* __restrict__ T, const float* __restrict__ mask,
+                                                     size_t rows, float inv_count, NetOps O, float* __restrict__ lpart,
+                                                     float* __restrict__ Y)
+{
+    extern __shared__ float4 mg_lds[];
+    NetLds& L = *(NetLds*)mg_lds;
+    const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63, q = l >> 4, col = l & 15;
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    float lsum = 0.0f;
+    if (BACK)
+        for (int k = t; k < NET_ROWS * 16; k += 256) L.dYr[k >> 4][16 + (k & 15)] = to_bf16(0.0f);
+    const size_t blk = blockIdx.x, r0 = blk * NET_ROWS;
+    /* inputs: chunk c of 4 columns of row c / 16 */
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int k = 0; k < 4; k++) {
+        const int c = t + 256 * k, row = c >> 4, k0 = 4 * (c & 15);
+        float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+        const bool in = r0 + (size_t)row < rows;
+        if (in) x = *(const float4*)(X + (r0 + (size_t)row) * MLP_IN + k0);
+        const float4 m = *(const float4*)(W.mu + k0), s = *(const float4*)(W.inv_sigma + k0);
+        const float v[4] = {in ? (x.x - m.x) * s.x : 0.f, in ? (x.y - m.y) * s.y : 0.f,
+                            in ? (x.z - m.z) * s.z : 0.f, in ? (x.w - m.w) * s.w : 0.f};
+        net_put(L.Xr, L.XT, row, k0, v);
+    }
+    __syncthreads();
+    /* layer 1 */
+    f32x4_t z1[2][4], z2[2][4];
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+    for (int a = 0; a < 2; a++) {
+        const int mt = 2 * w + a;
+        bf16x8_t wf[2];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm + a * 16 + 4 * kq + r, n = n0 + wn + b * 16 + (l & 15);
-                if (m < M && n < N) Cs[(size_t)m * N + n] = acc[a][b][r];
+        for (int kc = 0; kc < 2; kc++) wf[kc] = lds8(W.w1t + (size_t)(16 * mt + col) * MLP_IN + 32 * kc + 8 * q);
+        const float4 bias = *(const float4*)(W.b1 + 16 * mt + 4 * q);
+#pragma unroll
+        for (int rt = 0; rt < 4; rt++) {
+            f32x4_t acc = zero;
+#pragma unroll
+            for (int kc = 0; kc < 2; kc++) acc = mfma16(wf[kc], lds8(&L.Xr[16 * rt + col][32 * kc + 8 * q]), acc);
+            acc[0] += bias.x; acc[1] += bias.y; acc[2] += bias.z; acc[3] += bias.w;
+            z1[a][rt] = acc;
+            const float v[4] = {silu(acc[0]), silu(acc[1]), silu(acc[2]), silu(acc[3])};
+            net_put(L.A1r, L.A1T, 16 * rt + col, 16 * mt + 4 * q, v);
+        }
+    }
+    __syncthreads();
+    /* layer 2 */
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const int mt = 2 * w + a;
+        bf16x8_t wf[4];
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++) wf[kc] = lds8(W.w2t + (size_t)(16 * mt + col) * MLP_H + 32 * kc + 8 * q);
+        const float4 bias = *(const float4*)(W.b2 + 16 * mt + 4 * q);
+#pragma unroll
+        for (int rt = 0; rt < 4; rt++) {
+            f32x4_t acc = zero;
+#pragma unroll
+            for (int kc = 0; kc < 4; kc++) acc = mfma16(wf[kc], lds8(&L.A1r[16 * rt + col][32 * kc + 8 * q]), acc);
+            acc[0] += bias.x; acc[1] += bias.y; acc[2] += bias.z; acc[3] += bias.w;
+            z2[a][rt] = acc;
+            const float v[4] = {silu(acc[0]), silu(acc[1]), silu(acc[2]), silu(acc[3])};
+            net_put(L.A2r, L.A2T, 16 * rt + col, 16 * mt + 4 * q, v);
+        }
+    }
+    __syncthreads();
+    /* layer 3: wavefront w the rows 16 w .. 16 w + 15, lane outputs 4 q .. 4 q + 3 */
+    {
+        f32x4_t y = zero;
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++)
+            y = mfma16(lds8(W.w3t + (size_t)col * MLP_H + 32 * kc + 8 * q), lds8(&L.A2r[16 * w + col][32 * kc + 8 * q]), y);
+        const float4 bias = *(const float4*)(W.b3 + 4 * q);
+        y[0] += bias.x; y[1] += bias.y; y[2] += bias.z; y[3] += bias.w;
+        const size_t row = r0 + (size_t)(16 * w + col);
+        const bool in = row < rows;
+        if (!BACK) {
+            if (in) *(float4*)(Y + row * MLP_OUT + 4 * q) = make_float4(y[0], y[1], y[2], y[3]);
+        } else {
+            /* loss = sum over masked-in rows of |Y - T|^2 / count; dY = 2 (Y - T) / count */
+            float g[4] = {0.f, 0.f, 0.f, 0.f};
+            if (in && mask[row] != 0.f) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int c = 4 * q + r;
+                    if (c >= MLP_OUT_REAL) continue;
+                    const float e = y[r] - T[row * MLP_OUT_REAL + c];
+                    lsum += e * e;
+                    g[r] = 2.0f * e * inv_count;
+                }
             }
+            if (in) *(float4*)(O.fy + row * MLP_OUT + 4 * q) = make_float4(g[0], g[1], g[2], g[3]);
+            net_put(L.dYr, L.dYT, 16 * w + col, 4 * q, g);
+        }
+    }
+    if (!BACK) return;
+    __syncthreads();
+    /* dZ2 = (W3 dY) silu'(Z2); K = 16 outputs, padded to 32 with zeros */
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const int mt = 2 * w + a;
+        bf16x8_t wf = __builtin_bit_cast(bf16x8_t, make_uint4(0u, 0u, 0u, 0u));
+        if (q < 2) wf = lds8(W.w3 + (size_t)(16 * mt + col) * MLP_OUT + 8 * q);
+#pragma unroll
+        for (int rt = 0; rt < 4; rt++) {
+            const f32x4_t acc = mfma16(wf, lds8(&L.dYr[16 * rt + col][8 * q]), zero);
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = acc[r] * silu_grad(z2[a][rt][r]);
+            const size_t row = r0 + (size_t)(16 * rt + col);
+            if (row < rows) *(float4*)(O.fz2 + row * MLP_H + 16 * mt + 4 * q) = make_float4(v[0], v[1], v[2], v[3]);
+            net_put(L.dZ2r, L.dZ2T, 16 * rt + col, 16 * mt + 4 * q, v);
+        }
+    }
+    __syncthreads();
+    /* dZ1 = (W2 dZ2) silu'(Z1) */
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const int mt = 2 * w + a;
+        bf16x8_t wf[4];
+#pragma unroll
+        for (int kc = 0; kc < 4; kc++) wf[kc] = lds8(W.w2 + (size_t)(16 * mt + col) * MLP_H + 32 * kc + 8 * q);
+#pragma unroll
+        for (int rt = 0; rt < 4; rt++) {
+            f32x4_t acc = zero;
+#pragma unroll
+            for (int kc = 0; kc < 4; kc++) acc = mfma16(wf[kc], lds8(&L.dZ2r[16 * rt + col][32 * kc + 8 * q]), acc);
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = acc[r] * silu_grad(z1[a][rt][r]);
+            const size_t row = r0 + (size_t)(16 * rt + col);
+            if (row < rows) *(float4*)(O.fz1 + row * MLP_H + 16 * mt + 4 * q) = make_float4(v[0], v[1], v[2], v[3]);
+            net_put((__bf16(*)[NET_LD(MLP_H)]) nullptr, L.dZ1T, 16 * rt + col, 16 * mt + 4 * q, v);
+        }
+    }
+    __syncthreads();
+    net_tiles<MLP_IN / 16>(L.XT, O.x, blk, t);
+    net_tiles<MLP_H / 16>(L.A1T, O.a1, blk, t);
+    net_tiles<MLP_H / 16>(L.A2T, O.a2, blk, t);
+    net_tiles<MLP_H / 16>(L.dZ1T, O.dz1, blk, t);
+    net_tiles<MLP_H / 16>(L.dZ2T, O.dz2, blk, t);
+    net_tiles<MLP_OUT / 16>(L.dYT, O.dy, blk, t);
+    for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
+    if (l == 0) L.loss[w] = lsum;
+    __syncthreads();
+    if (t == 0) lpart[blk] = (((L.loss[0] + L.loss[1]) + L.loss[2]) + L.loss[3]) * inv_count;
 }
 
-__global__ LAUNCH_BOUNDS_256 void k_gemm_reduce(const float* __restrict__ part, int splits, size_t mn,
-                                                float* __restrict__ C)
+/* Gradients of the weights, W[m][n] = sum over rows of A[row][m] dZ[row][n], in splits of `kper`
+ * rows (a multiple of 32) that k_net_reduce adds in order, into part[split][NET_PARAMS]. One
+ * wavefront per (split, 16-row tile of W, four column tiles): a chain of MFMAs over the split's
+ * rows, 32 at a time, its operand tiles read whole from memory (1 KB per load) four chunks ahead.
+ * Tasks of a split: W2 8 x 2, W1 4 x 2, W3 8. The blocks past the splits' tasks sum the bias
+ * gradients' columns, rows t, t + 256, ... for each of 256 values of t, into bpart[t][272]
+ * (b1, b2, b3); k_net_reduce adds the 256. */
+#define NET_TASKS 32
+#define NET_BIASES (2 * MLP_H + MLP_OUT)
+#define NET_BIAS_BLOCKS (2 * 2 * 64 + 16)
+__global__ LAUNCH_BOUNDS_256 void k_net_grad(NetOps O, size_t rows, int splits, int kper, float* __restrict__ part,
+                                             float* __restrict__ bpart)
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= mn) return;
-    float s = part[i];
-    for (int k = 1; k < splits; k++) s += part[(size_t)k * mn + i];
-    C[i] = s;
+    const int t = threadIdx.x, l = t & 63, q = l >> 4, col = l & 15;
+    const int tasks = (splits * NET_TASKS) / 4; /* blocks of four wavefronts */
+    if ((int)blockIdx.x >= tasks) {
+        int b = (int)blockIdx.x - tasks;
+        const float* G;
+        int cols, c, tt, to;
+        if (b < 256) { /* 64 columns x 4 values of t */
+            G = b < 128 ? O.fz1 : O.fz2;
+            to = b < 128 ? 0 : MLP_H;
+            b &= 127;
+            cols = MLP_H;
+            c = (b & 1) * 64 + l;
+            tt = (b >> 1) * 4 + (t >> 6);
+        } else { /* 16 columns x 16 values of t */
+            G = O.fy;
+            to = 2 * MLP_H;
+            cols = MLP_OUT;
+            c = t & 15;
+            tt = (b - 256) * 16 + (t >> 4);
+        }
+        float s = 0.0f;
+        size_t r = (size_t)tt;
+        for (; r + 7 * 256 < rows; r += 8 * 256) {
+            float x[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) x[k] = G[(r + (size_t)k * 256) * cols + c];
+#pragma unroll
+            for (int k = 0; k < 8; k++) s += x[k];
+        }
+        for (; r < rows; r += 256) s += G[r * cols + c];
+        bpart[(size_t)tt * NET_BIASES + to + c] = s;
+        return;
+    }
+    const int task = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (t >> 6));
+    const int split = task / NET_TASKS, k = task % NET_TASKS;
+    const bf16x8_t *A, *B;
+    int ta, tb, mt, nt, nn, off, ld; /* tiles per chunk of A and B, the task's tiles, W's offset and row */
+    if (k < 16) {
+        A = (const bf16x8_t*)O.a1; B = (const bf16x8_t*)O.dz2;
+        ta = tb = MLP_H / 16; mt = k >> 1; nt = (k & 1) * 4; nn = 4; off = NET_W2; ld = MLP_H;
+    } else if (k < 24) {
+        A = (const bf16x8_t*)O.x; B = (const bf16x8_t*)O.dz1;
+        ta = MLP_IN / 16; tb = MLP_H / 16; mt = (k - 16) >> 1; nt = (k & 1) * 4; nn = 4; off = NET_W1; ld = MLP_H;
+    } else {
+        A = (const bf16x8_t*)O.a2; B = (const bf16x8_t*)O.dy;
+        ta = MLP_H / 16; tb = 1; mt = k - 24; nt = 0; nn = 1; off = NET_W3; ld = MLP_OUT;
+    }
+    const size_t c0 = (size_t)split * (kper / 32), c1 = min(c0 + (size_t)(kper / 32), (rows + 31) / 32);
+    A += (size_t)mt * 64 + l;
+    B += (size_t)nt * 64 + l;
+    f32x4_t acc[4];
+#pragma unroll
+    for (int n = 0; n < 4; n++) acc[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (size_t c = c0; c < c1; c += 4) {
+        bf16x8_t a[4], b[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const size_t cu = min(c + (size_t)u, c1 - 1);
+            a[u] = A[cu * ta * 64];
+#pragma unroll
+            for (int n = 0; n < 4; n++)
+                if (n < nn) b[u][n] = B[(cu * tb + n) * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (c + (size_t)u < c1)
+#pragma unroll
+                for (int n = 0; n < 4; n++)
+                    if (n < nn) acc[n] = mfma16(a[u], b[u][n], acc[n]);
+    }
+    float* out = part + (size_t)split * NET_PARAMS + off;
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+        if (n < nn)
+#pragma unroll
+            for (int r = 0; r < 4; r++) out[(16 * mt + 4 * q + r) * ld + 16 * (nt + n) + col] = acc[n][r];
 }
 
-/* ---------------------------------------------------------- elementwise steps */
-__global__ LAUNCH_BOUNDS_256 void k_to_bf16(const float* __restrict__ x, __bf16* __restrict__ y, size_t n)
+/* Adam's constants of one step (Kingma & Ba, 2015); update = 0: gradients only */
+struct AdamStep {
+    int update;
+    float lr, b1, b2, eps, c1, c2;
+};
+
+/* the [out][in] index of parameter i, or -1 where no bf16 [out][in] copy is kept (biases) */
+__device__ __forceinline__ int net_transposed(int i)
 {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = to_bf16(x[i]);
+    if (i < NET_B1) return NET_W1 + (i % MLP_H) * MLP_IN + i / MLP_H;
+    if (i >= NET_W2 && i < NET_B2) return NET_W2 + ((i - NET_W2) % MLP_H) * MLP_H + (i - NET_W2) / MLP_H;
+    if (i >= NET_W3 && i < NET_B3) return NET_W3 + ((i - NET_W3) % MLP_OUT) * MLP_H + (i - NET_W3) / MLP_OUT;
+    return -1;
 }
 
-/* rows of X (raw features) normalised and converted to bf16 */
-__global__ LAUNCH_BOUNDS_256 void k_normalize_rows(const float* __restrict__ X, const float* __restrict__ mu,
-                                                   const float* __restrict__ inv_sigma, __bf16* __restrict__ Xn,
-                                                   size_t rows)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * MLP_IN) return;
-    const int k = (int)(i % MLP_IN);
-    Xn[i] = to_bf16((X[i] - mu[k]) * inv_sigma[k]);
-}
-
-/* Z += bias (per column); A = silu(Z) in fp32 and bf16 */
-__global__ LAUNCH_BOUNDS_256 void k_bias_silu(float* __restrict__ Z, const float* __restrict__ bias, int cols,
-                                              size_t rows, __bf16* __restrict__ Ab, int apply_silu)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * cols) return;
-    const float z = Z[i] + bias[i % cols];
-    Z[i] = z;
-    if (Ab) Ab[i] = to_bf16(apply_silu ? silu(z) : z);
-}
-
-/* loss = sum over rows with mask of |Y[:, :3] - T|^2 / count; dY = 2 (Y - T) / count */
-__global__ LAUNCH_BOUNDS_256 void k_mse(const float* __restrict__ Y, const float* __restrict__ T,
-                                        const float* __restrict__ mask, size_t rows, float inv_count,
-                                        float* __restrict__ dY, __bf16* __restrict__ dYb, float* __restrict__ lpart)
+/* Gradients: a weight's is its splits' partials added in order (blocks of 256 weights), a bias's
+ * the tree sum of its 256 columns' sums (a block each, after those); with a.update the Adam update
+ * of fp32 master weights w and their bf16 copies. Block 0 also adds the loss partials (in double). */
+__global__ LAUNCH_BOUNDS_256 void k_net_reduce(const float* __restrict__ part, int splits,
+                                               const float* __restrict__ bpart, const float* __restrict__ lpart,
+                                               int lparts, float* __restrict__ grads, float* __restrict__ loss,
+                                               AdamStep a, float* __restrict__ w, float* __restrict__ m,
+                                               float* __restrict__ v, __bf16* __restrict__ wb, __bf16* __restrict__ wt)
 {
     __shared__ float red[256];
-    const size_t r = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    float l = 0.f;
-    if (r < rows) {
-        const float mk = mask[r];
-        for (int c = 0; c < MLP_OUT; c++) {
-            float g = 0.f;
-            if (c < MLP_OUT_REAL && mk != 0.f) {
-                const float e = Y[r * MLP_OUT + c] - T[r * MLP_OUT_REAL + c];
-                l += e * e;
-                g = 2.0f * e * inv_count;
-            }
-            dY[r * MLP_OUT + c] = g;
-            dYb[r * MLP_OUT + c] = to_bf16(g);
+    const int t = threadIdx.x, nw = (NET_PARAMS + 255) / 256;
+    int i = (int)blockIdx.x * 256 + t;
+    float gi;
+    if ((int)blockIdx.x < nw) {
+        if (blockIdx.x == 0 && t < 64 && loss) {
+            double d = 0.0;
+            for (int p = t; p < lparts; p += 64) d += lpart[p];
+            for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o);
+            if (t == 0) *loss = (float)d;
         }
-    }
-    red[threadIdx.x] = l;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+        const bool bias = (i >= NET_B1 && i < NET_W2) || (i >= NET_B2 && i < NET_W3) || i >= NET_B3;
+        if (bias) return;
+        gi = part[i];
+        for (int p = 1; p < splits; p++) gi += part[(size_t)p * NET_PARAMS + i];
+    } else {
+        const int b = (int)blockIdx.x - nw;
+        red[t] = bpart[(size_t)t * NET_BIASES + b];
         __syncthreads();
+        for (int k = 128; k > 0; k >>= 1) {
+            if (t < k) red[t] += red[t + k];
+            __syncthreads();
+        }
+        if (t != 0) return;
+        gi = red[0];
+        i = b < MLP_H ? NET_B1 + b : b < 2 * MLP_H ? NET_B2 + b - MLP_H : NET_B3 + b - 2 * MLP_H;
     }
-    if (threadIdx.x == 0) lpart[blockIdx.x] = red[0] * inv_count;
-}
-
-/* dZ = dA * silu'(Z) (fp32 and bf16) */
-__global__ LAUNCH_BOUNDS_256 void k_silu_back(const float* __restrict__ dA, const float* __restrict__ Z, size_t n,
-                                              float* __restrict__ dZ, __bf16* __restrict__ dZb)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float g = dA[i] * silu_grad(Z[i]);
-    dZ[i] = g;
-    dZb[i] = to_bf16(g);
-}
-
-/* column sums of G [rows x cols], one block per column, fixed-order tree: deterministic */
-__global__ LAUNCH_BOUNDS_256 void k_colsum(const float* __restrict__ G, size_t rows, int cols, float* __restrict__ out)
-{
-    __shared__ float red[256];
-    const int c = blockIdx.x;
-    float s = 0.f;
-    for (size_t r = threadIdx.x; r < rows; r += 256) s += G[r * cols + c];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = red[0];
-}
-
-/* Adam (Kingma & Ba, 2015) on fp32 master weights */
-__global__ LAUNCH_BOUNDS_256 void k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                                         float* __restrict__ v, size_t n, float lr, float b1, float b2, float eps,
-                                         float c1, float c2)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
+    grads[i] = gi;
+    if (!a.update) return;
+    const float mi = a.b1 * m[i] + (1.0f - a.b1) * gi;
+    const float vi = a.b2 * v[i] + (1.0f - a.b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float x = w[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+    w[i] = x;
+    wb[i] = to_bf16(x);
+    const int j = net_transposed(i);
+    if (j >= 0) wt[j] = to_bf16(x);
+}
+
+/* the bf16 copies of the fp32 weights: wb as they are, wt the matrices in [out][in] order */
+__global__ LAUNCH_BOUNDS_256 void k_net_weights(const float* __restrict__ w, __bf16* __restrict__ wb,
+                                                __bf16* __restrict__ wt)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= NET_PARAMS) return;
+    wb[i] = to_bf16(w[i]);
+    const int j = net_transposed(i);
+    if (j >= 0) wt[j] = to_bf16(w[i]);
 }
 
 /* W [K x N] fp32 row-major -> fragment layout (ntile, kchunk, col, k) in bf16 */
