@@ -182,7 +182,8 @@ int mg_debug_set_scan_ticket(mg_handle* h, uint64_t ticket);
 
 /* ---- batched instances (no counterpart in the reference, which steps one FluidSystem) ----
  * A batch steps many independent handles (each with its own buffers, grid, parameters and
- * genome) together: by default one persistent launch per step covers every phase of every
+ * genome) together: by default one launch per phase over every instance, for batches of more
+ * than 4,194,304 particles one persistent launch per step that covers every phase of every
  * instance (resident workgroups, per-phase work queues, grid barriers); the alternative
  * dispatch form runs one launch per phase and size class. Every instance evolves bit for bit
  * as under mg_step. While a handle belongs to a batch its work
@@ -205,8 +206,9 @@ int mg_batch_classes(mg_batch* b, int* nclass, int* members, unsigned* threads);
  * per size class, the one with the least kernel time (threads_out, one entry per class, may be
  * null, receives it); then, at those block sizes, the pressure sweep's tile shape per class
  * (candidates tested at a time 8 or 4, staged band of 128 or 64 slots per wavefront) with the
- * least pressure time; then times `steps` whole steps of that dispatch form and of the
- * persistent form at each workgroup count per CU that stays resident, and keeps the fastest.
+ * least pressure time; then times `steps` whole steps of that dispatch form, of the persistent
+ * form at each workgroup count per CU that stays resident and of the form with one launch per
+ * phase over every instance, and keeps the fastest.
  * The steps are real steps of the batch. */
 int mg_batch_autotune(mg_batch* b, int steps, float dt, unsigned flags, unsigned* threads_out);
 /* The dispatch form's configuration of size class cls (0 .. nclass - 1): its instances, block
@@ -217,7 +219,7 @@ int mg_batch_class_config(mg_batch* b, int cls, int* instances, unsigned* thread
  * band_cap 128 or 64 (MG_ERR_ARG otherwise). Every shape gives the same bits. */
 int mg_batch_set_tile_shape(mg_batch* b, int cls, int cand_batch, int band_cap);
 /* The launch form in use: *persistent = 1 for one persistent launch per step (with
- * *workgroups workgroups of 256 threads), 0 for the dispatch form. Either may be null. */
+ * *workgroups workgroups of 256 threads), 0 for a form of launches per phase. Either may be null. */
 int mg_batch_launch_config(mg_batch* b, int* persistent, unsigned* workgroups);
 /* Chooses the form: on = 1 persistent (workgroups_per_cu workgroups on each CU, 0 = all that
  * stay resident; batches whose instances exceed 65,535 blocks of 256 use the dispatch form),

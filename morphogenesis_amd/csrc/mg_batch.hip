@@ -1,17 +1,21 @@
 /*
  * mg_batch.hip — many independent handles stepped together (included by mg_capi.hip).
  *
- * A step of every instance is one persistent launch (kb_step): resident workgroups walk the
- * six phases of the fused step (pressure, force + advance, diffusion + genes + insert,
- * scan, place, rank + gather) over per-phase queues of (instance, block) items, with grid
- * barriers between phases. The alternative is the dispatch form: instances grouped into
- * size classes by particle count, each class running the six phases as launches that cover
- * all of its instances (6 x classes dispatches per step). Both look up their instance in a
- * device table (BatchInst) built from each handle exactly as its own fused step builds its
- * kernel arguments, so every instance evolves bit for bit as it would alone. Tables cover the
- * two buffer parities of consecutive steps; two consecutive steps are captured into one
- * hipGraph and replayed. mg_batch_autotune measures the dispatch form at each block size per
- * class and the persistent form at each workgroup count per CU, and keeps the fastest.
+ * A step of every instance takes one of three forms:
+ *   merged      six launches per step (pressure, force + advance, diffusion + genes + insert, scan,
+ *               place, rank + gather), each over every instance in blocks of 64 particles, the
+ *               sweeps split by rows as a single model's: the default up to kBatchMerged particles;
+ *   persistent  one launch (kb_step), whose resident workgroups walk the six phases over per-phase
+ *               queues of (instance, block) items, with grid barriers between phases: the default
+ *               of larger batches;
+ *   dispatch    instances grouped into size classes by particle count, each class running the six
+ *               phases as launches that cover its instances (6 x classes dispatches per step).
+ * All look up their instance in a device table (BatchInst) built from each handle exactly as its
+ * own fused step builds its kernel arguments, so every instance evolves bit for bit as it would
+ * alone. Tables cover the two buffer parities of consecutive steps; two consecutive steps are
+ * captured into one hipGraph and replayed. mg_batch_autotune measures the dispatch form at each block size per
+ * class, the persistent form at each workgroup count per CU and the merged form, and keeps the
+ * fastest.
  */
 
 struct mg_batch {
@@ -49,6 +53,18 @@ struct mg_batch {
     uint32_t* pitems[PERSIST_PHASES] = {};
     uint32_t pnitems[PERSIST_PHASES] = {};
     PersistCtl* pctl = nullptr;
+    /* the merged form: six launches per step, each over every instance (largest first) in blocks
+     * of 64 particles. -1: by size (kBatchMerged), 0: off (mg_batch_set_persistent, or
+     * mg_batch_autotune found another form faster), 1: on (mg_batch_autotune) */
+    int merged_mode = -1;
+    bool merged = false;              /* in use for the tables built */
+    BatchInst* RI[2] = {};
+    uint16_t *rmap = nullptr, *stmap = nullptr;
+    uint32_t rblocks = 0, stblocks = 0;
+    int merged_ng = 1;
+    size_t merged_n = 0;              /* particles of all instances */
+    bool merged_rows = false;         /* every instance can run split by rows */
+    bool merged_bonds = false, merged_genes = false; /* with bond records; with genes */
     /* per-class timing during autotuning */
     bool timing = false;
     std::vector<hipEvent_t> ev;
@@ -106,6 +122,9 @@ void batch_free_tables(mg_batch* b)
     }
     b->pctl = nullptr;
     b->persist_ok = false;
+    b->RI[0] = b->RI[1] = nullptr;
+    b->rmap = b->stmap = nullptr;
+    b->merged = false;
     for (auto& c : b->cls) {
         c.I[0] = c.I[1] = nullptr;
         c.pmap = c.tmap = nullptr;
@@ -151,6 +170,24 @@ void fill_inst(BatchInst& t, mg_handle* h, const MgGenome* dgen, float dt, unsig
     t.dt = dt;
 }
 
+/* The view of handle h a fused step from now (q = 0) or one step later (q = 1) */
+void fill_inst_at(BatchInst& t, mg_handle* h, const MgGenome* dgen, float dt, unsigned flags, int q)
+{
+    const int ic = h->icur, gc = h->gcur;
+    const bool gs = h->grid_scanned, pb = h->pos_binned, cf = h->cells_fresh;
+    if (q == 1) {
+        h->icur = 1 - ic;
+        h->gcur = 1 - gc;
+        h->grid_scanned = h->pos_binned = h->cells_fresh = true;
+    }
+    fill_inst(t, h, dgen, dt, flags);
+    h->icur = ic;
+    h->gcur = gc;
+    h->grid_scanned = gs;
+    h->pos_binned = pb;
+    h->cells_fresh = cf;
+}
+
 template <int NG> size_t persist_lds() { return band_lds<(NG > 1 ? NG : 1)>(256); }
 
 template <int NG> int persist_occupancy(unsigned* per_cu)
@@ -179,23 +216,11 @@ int persist_build(mg_batch* b, float dt, unsigned flags)
         const uint32_t tnb = (uint32_t)((h->C + SCAN_TILE - 1) / SCAN_TILE);
         if (pnb > 65536 || tnb > 65536) { fits = false; break; }
         for (int q = 0; q < 2; q++) {
-            const int ic = h->icur, gc = h->gcur;
-            const bool gs = h->grid_scanned, pb = h->pos_binned, cf = h->cells_fresh;
-            if (q == 1) {
-                h->icur = 1 - ic;
-                h->gcur = 1 - gc;
-                h->grid_scanned = h->pos_binned = h->cells_fresh = true;
-            }
             BatchInst t;
-            fill_inst(t, h, b->dgen[order[k]], dt, flags);
+            fill_inst_at(t, h, b->dgen[order[k]], dt, flags, q);
             t.pb0 = 0; t.pnb = pnb;
             t.tb0 = 0; t.tnb = tnb;
             tab[q].push_back(t);
-            h->icur = ic;
-            h->gcur = gc;
-            h->grid_scanned = gs;
-            h->pos_binned = pb;
-            h->cells_fresh = cf;
         }
         const int g = tab[0].back().dp.ng;
         ng = std::max(ng, g <= 1 ? 1 : (g == 2 ? 2 : 4));
@@ -261,6 +286,93 @@ int persist_launch(mg_batch* b, int q)
     return MG_OK;
 }
 
+/* Batches of up to this many particles step in the merged form unless a form is chosen. us per
+ * step by particles, merged / persistent / dispatch as tuned (tissues, 32 bond slots, genes):
+ * 16,112 (16 instances): 61 / 318 / 155; 201,509 (32): 211 / 664 / 384; 930,148 (64): 750 / 1,800 /
+ * 939; 1,884,496 (128): 1,424 / 2,921 / 1,621; 3,721,327 (200): 2,651 / 4,997 / 3,006. One launch
+ * per phase for all size classes has one tail instead of one per class, and it takes the sweeps
+ * split by rows; larger batches keep the persistent launch as their default and
+ * mg_batch_autotune decides. */
+const size_t kBatchMerged = 1u << 22;
+
+int merged_build(mg_batch* b, float dt, unsigned flags)
+{
+    const int n = (int)b->hs.size();
+    b->merged_n = 0;
+    for (const mg_handle* h : b->hs) b->merged_n += (size_t)h->N;
+    if (b->merged_mode == 0 || (b->merged_mode < 0 && b->merged_n > kBatchMerged)) return MG_OK;
+    std::vector<int> order(n);
+    for (int i = 0; i < n; i++) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->hs[x]->N > b->hs[y]->N; });
+    std::vector<BatchInst> tab[2];
+    std::vector<uint16_t> pm, tm;
+    b->merged_ng = 1;
+    b->merged_rows = b->merged_bonds = true;
+    b->merged_genes = (flags & MG_STEP_GENES) != 0;
+    for (int k = 0; k < n; k++) {
+        mg_handle* h = b->hs[order[k]];
+        const uint32_t pnb = nblk(h->N, 64), tnb = (uint32_t)((h->C + SCAN_TILE - 1) / SCAN_TILE);
+        for (int q = 0; q < 2; q++) {
+            BatchInst t;
+            fill_inst_at(t, h, b->dgen[order[k]], dt, flags, q);
+            t.pb0 = (uint32_t)pm.size(); t.pnb = pnb;
+            t.tb0 = (uint32_t)tm.size(); t.tnb = tnb;
+            tab[q].push_back(t);
+            if (!rows_of_three(h, t.pressure)) b->merged_rows = false;
+            if (h->B == 0 || !t.force.ETR) b->merged_bonds = false;
+        }
+        const int ng = tab[0].back().dp.ng;
+        b->merged_ng = std::max(b->merged_ng, ng <= 1 ? 1 : (ng == 2 ? 2 : 4));
+        pm.insert(pm.end(), pnb, (uint16_t)k);
+        tm.insert(tm.end(), tnb, (uint16_t)k);
+    }
+    b->rblocks = (uint32_t)pm.size();
+    b->stblocks = (uint32_t)tm.size();
+    for (int q = 0; q < 2; q++) {
+        CHK(balloc(b, &b->RI[q], tab[q].size()));
+        HIPCHK(hipMemcpyAsync(b->RI[q], tab[q].data(), tab[q].size() * sizeof(BatchInst), hipMemcpyHostToDevice, b->st));
+    }
+    CHK(balloc(b, &b->rmap, pm.size()));
+    CHK(balloc(b, &b->stmap, tm.size()));
+    HIPCHK(hipMemcpyAsync(b->rmap, pm.data(), pm.size() * 2, hipMemcpyHostToDevice, b->st));
+    HIPCHK(hipMemcpyAsync(b->stmap, tm.data(), tm.size() * 2, hipMemcpyHostToDevice, b->st));
+    HIPCHK(hipStreamSynchronize(b->st)); /* the host copies go away with this scope */
+    b->merged = true;
+    return MG_OK;
+}
+
+/* One fused step of every instance in the merged form. The split by rows follows the single
+ * model's rules (launch_pressure, launch_force_advance, launch_diffuse_rows) at the particles of
+ * the whole batch: what counts is how far they fill the chip. */
+int merged_launch(mg_batch* b, int q)
+{
+    const BatchInst* I = b->RI[q];
+    const dim3 grid(b->rblocks), one(64);
+    if (b->merged_rows && b->merged_n <= (size_t)kPressureRows9)
+        hipLaunchKernelGGL(kb_pressure_rows<9>, grid, dim3(64 * 9), 0, b->st, I, b->rmap);
+    else if (b->merged_rows)
+        hipLaunchKernelGGL(kb_pressure_rows<3>, grid, dim3(64 * 3), 0, b->st, I, b->rmap);
+    else
+        hipLaunchKernelGGL((kb_pressure<8, 128>), grid, one, (band_lds<0, 128>(64)), b->st, I, b->rmap);
+    if (b->merged_rows && b->merged_bonds && b->merged_n <= (size_t)kForceRows9)
+        hipLaunchKernelGGL(kb_force_advance_rows, grid, dim3(64 * (RS_ROWS + 2)), 0, b->st, I, b->rmap);
+    else
+        hipLaunchKernelGGL(kb_force_advance, grid, one, band_lds<1>(64), b->st, I, b->rmap);
+    if (b->merged_rows && b->merged_genes && b->merged_n <= (size_t)kDiffuseRows)
+        hipLaunchKernelGGL(kb_diffuse_rows, grid, dim3(64 * RS_ROWS), 0, b->st, I, b->rmap);
+    else if (b->merged_ng <= 1)
+        hipLaunchKernelGGL(kb_diffuse_genes_insert<1>, grid, one, band_lds<1>(64), b->st, I, b->rmap);
+    else if (b->merged_ng == 2)
+        hipLaunchKernelGGL(kb_diffuse_genes_insert<2>, grid, one, band_lds<2>(64), b->st, I, b->rmap);
+    else
+        hipLaunchKernelGGL(kb_diffuse_genes_insert<4>, grid, one, band_lds<4>(64), b->st, I, b->rmap);
+    hipLaunchKernelGGL(kb_scan, dim3(b->stblocks), dim3(256), 0, b->st, I, b->stmap);
+    hipLaunchKernelGGL(kb_place, grid, one, 0, b->st, I, b->rmap);
+    hipLaunchKernelGGL(kb_sort_gather, grid, one, 0, b->st, I, b->rmap);
+    HIPCHK(hipGetLastError());
+    return MG_OK;
+}
+
 int batch_build(mg_batch* b, float dt, unsigned flags)
 {
     batch_free_tables(b);
@@ -284,23 +396,10 @@ int batch_build(mg_batch* b, float dt, unsigned flags)
             pm.insert(pm.end(), pnb, (uint16_t)k);
             tm.insert(tm.end(), tnb, (uint16_t)k);
             for (int q = 0; q < 2; q++) {
-                /* q = 1: the state one fused step later */
-                const int ic = h->icur, gc = h->gcur;
-                const bool gs = h->grid_scanned, pb = h->pos_binned, cf = h->cells_fresh;
-                if (q == 1) {
-                    h->icur = 1 - ic;
-                    h->gcur = 1 - gc;
-                    h->grid_scanned = h->pos_binned = h->cells_fresh = true;
-                }
                 BatchInst& t = tab[q][k];
-                fill_inst(t, h, b->dgen[c.members[k]], dt, flags);
+                fill_inst_at(t, h, b->dgen[c.members[k]], dt, flags, q);
                 t.pb0 = pb0; t.pnb = pnb;
                 t.tb0 = tb0; t.tnb = tnb;
-                h->icur = ic;
-                h->gcur = gc;
-                h->grid_scanned = gs;
-                h->pos_binned = pb;
-                h->cells_fresh = cf;
             }
             const int ng = tab[0][k].dp.ng;
             c.ng = std::max(c.ng, ng <= 1 ? 1 : (ng == 2 ? 2 : 4));
@@ -321,6 +420,7 @@ int batch_build(mg_batch* b, float dt, unsigned flags)
     }
     HIPCHK(hipStreamSynchronize(b->st));
     CHK(persist_build(b, dt, flags));
+    CHK(merged_build(b, dt, flags));
     b->sig.resize(b->hs.size());
     for (size_t i = 0; i < b->hs.size(); i++) b->sig[i] = handle_sig(b->hs[i]);
     b->sig_dt = dt;
@@ -368,6 +468,7 @@ void batch_mark(mg_batch* b, int cls, int ph, bool start)
  * form (always when timing per phase) */
 int batch_launch(mg_batch* b, int q)
 {
+    if (b->merged && !b->timing) return merged_launch(b, q);
     if (b->persistent && b->persist_ok && !b->timing) return persist_launch(b, q);
     for (size_t ci = 0; ci < b->cls.size(); ci++) {
         auto& c = b->cls[ci];
@@ -663,6 +764,7 @@ static int batch_time_classes(mg_batch* b, int steps, float dt, unsigned flags, 
 int mg_batch_autotune(mg_batch* b, int steps, float dt, unsigned flags, unsigned* threads_out)
 {
     if (!b || steps < 1) { set_err("mg_batch_autotune: bad arguments"); return MG_ERR_ARG; }
+    b->merged_mode = 0;
     const unsigned cand[] = {256, 128, 64};
     const int nc = (int)b->cls.size();
     std::vector<double> best(nc, 1e300), ms;
@@ -733,10 +835,22 @@ int mg_batch_autotune(mg_batch* b, int steps, float dt, unsigned flags, unsigned
             }
         }
     }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
     b->persistent = best_persistent;
     b->persist_use_per_cu = best_per_cu;
+    if (r == MG_OK) {
+        /* the merged form, its tables built by two steps outside the timed ones */
+        b->merged_mode = 1;
+        b->built = false;
+        double ms = 0.0;
+        r = batch_steps(b, 2, dt, flags, false);
+        if (r == MG_OK) r = time_steps(&ms);
+        if (r != MG_OK || ms >= best_ms) {
+            b->merged_mode = 0;
+            b->built = false;
+        }
+    }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
     return r;
 }
 
@@ -769,7 +883,7 @@ int mg_batch_set_tile_shape(mg_batch* b, int cls, int cand_batch, int band_cap)
 int mg_batch_launch_config(mg_batch* b, int* persistent, unsigned* workgroups)
 {
     if (!b) return MG_ERR_ARG;
-    const bool on = b->persistent && b->persist_ok;
+    const bool on = b->persistent && b->persist_ok && !b->merged;
     if (persistent) *persistent = on ? 1 : 0;
     if (workgroups) *workgroups = on ? persist_workgroups(b) : 0u;
     return MG_OK;
@@ -778,8 +892,16 @@ int mg_batch_launch_config(mg_batch* b, int* persistent, unsigned* workgroups)
 int mg_batch_set_persistent(mg_batch* b, int on, unsigned workgroups_per_cu)
 {
     if (!b) return MG_ERR_ARG;
+    HIPCHK(hipStreamSynchronize(b->st));
+    for (int k = 0; k < 2; k++) /* captured for the form before */
+        if (b->graph[k]) {
+            (void)hipGraphExecDestroy(b->graph[k]);
+            b->graph[k] = nullptr;
+        }
     b->persistent = on != 0;
     b->persist_use_per_cu = workgroups_per_cu;
+    b->merged_mode = 0;
+    b->merged = false;
     return MG_OK;
 }
 

@@ -1343,15 +1343,16 @@ __device__ __forceinline__ void rs_record_bonds(const DS& d, const MgParams& p, 
 
 /* contributePressure / computePressure split by rows; writes what k_pressure writes */
 template <int MODE, int W>
-__global__ __launch_bounds__(64 * W, RS_OCC) void k_pressure_rows(DS d, MgParams p, MgGrid g)
+__device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& p, const MgGrid& g, uint32_t bid,
+                                                   uint32_t nblk)
 {
     constexpr int PER = RS_ROWS / W; /* rows per wavefront */
     __shared__ Band<0> bands[W];
     __shared__ float part[RS_ROWS * RS_CELLS][64];
-    const uint32_t bid = xcd_block(), lane = threadIdx.x & 63u;
+    const uint32_t lane = threadIdx.x & 63u;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (d.ZERO)
-        for (uint32_t z = bid * blockDim.x + threadIdx.x; z < d.zero_n; z += gridDim.x * blockDim.x) d.ZERO[z] = 0u;
+        for (uint32_t z = bid * blockDim.x + threadIdx.x; z < d.zero_n; z += nblk * blockDim.x) d.ZERO[z] = 0u;
     if (d.HMW && bid == 0 && threadIdx.x == 0) d.ctr[MG_C_SKIN] = 0u;
     const uint32_t i = bid * 64u + lane;
     uint32_t gc = (i < d.ctr[MG_C_ACTIVE]) ? d.GCELL[i] : MG_GRID_UNDEF;
@@ -1395,6 +1396,12 @@ __global__ __launch_bounds__(64 * W, RS_OCC) void k_pressure_rows(DS d, MgParams
 #pragma unroll
     for (int k = 0; k < RS_ROWS * RS_CELLS; k++) sum += part[k][lane];
     pressure_store<MODE>(d, p, i, sum);
+}
+
+template <int MODE, int W>
+__global__ __launch_bounds__(64 * W, RS_OCC) void k_pressure_rows(DS d, MgParams p, MgGrid g)
+{
+    pressure_rows_body<MODE, W>(d, p, g, xcd_block(), gridDim.x);
 }
 
 /* A hit's fluid force added to cf (P_i, V_i the particle, Pj, Vj the neighbour) */
@@ -1880,14 +1887,14 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_force_advance(DS d, MgParams p, MgGrid g, 
  * order and advances. Bonds come as the pressure pass's records only (d.ETR). */
 #define RS_INC 12
 template <int MODE, int BONDS, int W>
-__global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? RS_OCC : 3) void k_force_advance_rows(DS d, MgParams p, MgGrid g, float dt,
-                                                                                   int special, float zoff)
+__device__ __forceinline__ void force_advance_rows_body(const DS& d, const MgParams& p, const MgGrid& g, float dt,
+                                                        uint32_t bid, int special = 0, float zoff = 0.0f)
 {
     constexpr int PER = RS_ROWS / W; /* rows per wavefront */
     __shared__ Band<1> bands[W];
     __shared__ float part[RS_ROWS * RS_CELLS][3][64];
     __shared__ float own[3][64];
-    const uint32_t bid = xcd_block(), lane = threadIdx.x & 63u;
+    const uint32_t lane = threadIdx.x & 63u;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t i = bid * 64u + lane, N = (uint32_t)d.N, B = (uint32_t)d.B;
     const uint32_t na = d.ctr[MG_C_ACTIVE];
@@ -1994,6 +2001,14 @@ __global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? RS_OCC : 3) void k_f
         }
     }
     if (i < N) advance_other_half(d, p, dt, i, valid, F, special, zoff);
+}
+
+template <int MODE, int BONDS, int W>
+__global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? RS_OCC : 3) void k_force_advance_rows(DS d, MgParams p,
+                                                                                                  MgGrid g, float dt,
+                                                                                                  int special, float zoff)
+{
+    force_advance_rows_body<MODE, BONDS, W>(d, p, g, dt, xcd_block(), special, zoff);
 }
 
 /* ----------------------------------------------------------- diffusion (a12)
@@ -2271,9 +2286,9 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_diffuse_genes_insert(DS d, MgParams p, MgG
 #define RS_GENES 2
 #define RS_INSERT 4
 #define RS_LIST 48
-template <int PART>
-__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_rows(DS d, MgParams p, MgGrid g, MgGenome gen,
-                                                                       DiffPlan dp)
+template <int PART, class Gen>
+__device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p, const MgGrid& g, const Gen& gen,
+                                                  const DiffPlan& dp, uint32_t bid)
 {
     union Stage {
         struct {
@@ -2288,7 +2303,7 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_rows(DS d, MgP
     __shared__ Stage sh;
     __shared__ uint32_t cnt[RS_ROWS][64];
     __shared__ float conc[MG_NUM_TF][64];
-    const uint32_t bid = xcd_block(), lane = threadIdx.x & 63u;
+    const uint32_t lane = threadIdx.x & 63u;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t i = bid * 64u + lane, N = (uint32_t)d.N;
     const uint32_t na = d.ctr[MG_C_ACTIVE], nump = d.ctr[MG_C_NUM_POINTS];
@@ -2506,6 +2521,13 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_rows(DS d, MgP
         /* binning rewrites GCELL, which every wavefront has read before the barriers above */
         insert_one(d, g, i, i < N, i < N ? d.P[i] : make_float4(0.f, 0.f, 0.f, 0.f), d.CNTN, nullptr);
     }
+}
+
+template <int PART>
+__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_rows(DS d, MgParams p, MgGrid g, MgGenome gen,
+                                                                       DiffPlan dp)
+{
+    diffuse_rows_body<PART>(d, p, g, gen, dp, xcd_block());
 }
 
 /* -------------------------------------------------------- bond formation
@@ -3324,6 +3346,33 @@ __global__ LAUNCH_BOUNDS_SWEEP void kb_diffuse_genes_insert(const BatchInst* __r
                                   (Band<NG>*)mg_lds, b - in.pb0);
 }
 
+/* the sweeps split by rows: 64 particles per block, the view's pb0 / pnb count such blocks */
+template <int W>
+__global__ __launch_bounds__(64 * W, RS_OCC) void kb_pressure_rows(const BatchInst* __restrict__ I,
+                                                                   const uint16_t* __restrict__ map)
+{
+    const uint32_t b = xcd_block();
+    const BatchInst& in = I[map[b]];
+    pressure_rows_body<MG_SPH_REFERENCE, W>(global_view(in.pressure), in.p, in.g, b - in.pb0, in.pnb);
+}
+
+__global__ __launch_bounds__(64 * (RS_ROWS + 2), RS_OCC) void kb_force_advance_rows(const BatchInst* __restrict__ I,
+                                                                                   const uint16_t* __restrict__ map)
+{
+    const uint32_t b = xcd_block();
+    const BatchInst& in = I[map[b]];
+    force_advance_rows_body<MG_SPH_REFERENCE, 1, RS_ROWS>(global_view(in.force), in.p, in.g, in.dt, b - in.pb0);
+}
+
+__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void kb_diffuse_rows(const BatchInst* __restrict__ I,
+                                                                        const uint16_t* __restrict__ map)
+{
+    const uint32_t b = xcd_block();
+    const BatchInst& in = I[map[b]];
+    diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT>(global_view(in.diffuse), in.p, in.g, const_genome(in.gen), in.dp,
+                                                         b - in.pb0);
+}
+
 __global__ __launch_bounds__(256) void kb_scan(const BatchInst* __restrict__ I, const uint16_t* __restrict__ map)
 {
     const BatchInst& in = I[map[blockIdx.x]];
@@ -3402,7 +3451,7 @@ __device__ __forceinline__ void persist_barrier(PersistCtl* ctl, unsigned& sense
 }
 
 template <int NG>
-__global__ __launch_bounds__(256) void kb_step(PersistPlan P)
+__global__ __launch_bounds__(256, NG <= 2 ? 3 : 2) void kb_step(PersistPlan P)
 {
     extern __shared__ float4 mg_lds[];
     __shared__ uint32_t s_item;
