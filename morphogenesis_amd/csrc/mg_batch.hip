@@ -61,6 +61,7 @@ struct mg_batch {
     BatchInst* RI[2] = {};
     uint16_t *rmap = nullptr, *stmap = nullptr;
     uint32_t rblocks = 0, stblocks = 0;
+    uint32_t* errw = nullptr;         /* mg_batch_sync's sum of the error flags */
     int merged_ng = 1;
     size_t merged_n = 0;              /* particles of all instances */
     bool merged_rows = false;         /* every instance can run split by rows */
@@ -124,6 +125,7 @@ void batch_free_tables(mg_batch* b)
     b->persist_ok = false;
     b->RI[0] = b->RI[1] = nullptr;
     b->rmap = b->stmap = nullptr;
+    b->errw = nullptr;
     b->merged = false;
     for (auto& c : b->cls) {
         c.I[0] = c.I[1] = nullptr;
@@ -332,6 +334,7 @@ int merged_build(mg_batch* b, float dt, unsigned flags)
         CHK(balloc(b, &b->RI[q], tab[q].size()));
         HIPCHK(hipMemcpyAsync(b->RI[q], tab[q].data(), tab[q].size() * sizeof(BatchInst), hipMemcpyHostToDevice, b->st));
     }
+    CHK(balloc(b, &b->errw, 1));
     CHK(balloc(b, &b->rmap, pm.size()));
     CHK(balloc(b, &b->stmap, tm.size()));
     HIPCHK(hipMemcpyAsync(b->rmap, pm.data(), pm.size() * 2, hipMemcpyHostToDevice, b->st));
@@ -717,13 +720,24 @@ int mg_batch_sync(mg_batch* b)
             return MG_ERR_HIP;
         }
     }
+    auto gave_up = [](uint32_t err) -> int {
+        if (!err) return MG_OK;
+        set_err("mg_batch_sync: a kernel gave up a bounded wait; results are invalid");
+        return MG_ERR_HIP;
+    };
+    if (b->merged) {
+        /* every instance's flag by one kernel and one copy (a copy each: 14 us an instance) */
+        uint32_t err = 0;
+        hipLaunchKernelGGL(k_batch_errors, dim3(1), dim3(256), 0, b->st, b->RI[0], (int)b->hs.size(), b->errw);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(&err, b->errw, 4, hipMemcpyDeviceToHost, b->st));
+        HIPCHK(hipStreamSynchronize(b->st));
+        return gave_up(err);
+    }
     for (mg_handle* h : b->hs) {
         uint32_t err = 0;
         HIPCHK(hipMemcpy(&err, h->ctr + MG_C_ERR, 4, hipMemcpyDeviceToHost));
-        if (err) {
-            set_err("mg_batch_sync: a kernel gave up a bounded wait; results are invalid");
-            return MG_ERR_HIP;
-        }
+        CHK(gave_up(err));
     }
     return MG_OK;
 }

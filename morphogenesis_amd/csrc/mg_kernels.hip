@@ -3393,6 +3393,15 @@ __global__ LAUNCH_BOUNDS_256 void kb_sort_gather(const BatchInst* __restrict__ I
     sort_gather_body(global_view(in.sort), in.vmax, b - in.pb0);
 }
 
+/* *out = the bounded-wait flags of n instances together (one block) */
+__global__ LAUNCH_BOUNDS_256 void k_batch_errors(const BatchInst* __restrict__ I, int n, uint32_t* __restrict__ out)
+{
+    int err = 0;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) err |= I[k].ctr[MG_C_ERR] != 0u;
+    err = __syncthreads_or(err);
+    if (threadIdx.x == 0) *out = (uint32_t)err;
+}
+
 /* --------------------------------------------------- persistent batched step
  * One launch per step for every instance of a batch: a grid of workgroups that stay resident
  * (sized from the occupancy of this kernel) walks the six phases of the fused step, each
