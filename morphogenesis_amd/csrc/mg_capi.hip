@@ -920,8 +920,35 @@ void launch_pressure(mg_handle* h, unsigned nb, const DS& d)
         hipLaunchKernelGGL(k_pressure<MG_SPH_REFERENCE>, dim3(nb), dim3(256), band_lds<0>(256), h->st, d, h->p, h->g);
 }
 
+/* How a force pass of this view runs: wavefronts for the rows of 64 particles (9 or 3; split by
+ * rows the bonds come as records only), or 1 for a lane per particle */
+int force_rows(const mg_handle* h, const DS& d)
+{
+    if (!rows_of_three(h, d)) return 1;
+    if (h->B > 0) return d.ETR && h->N <= kForceRows9 ? 9 : 1;
+    return h->N <= kForceRows9NoBonds ? 9 : h->N <= kForceRows3NoBonds ? 3 : 1;
+}
+
+/* go(kernel, blocks, threads per block) with K<MODE, BONDS, W> for a view split over W wavefronts */
+#define MG_FORCE_ROWS(K, GO, W)                                                                   \
+    do {                                                                                          \
+        const unsigned nr_ = nblk(h->N, 64);                                                      \
+        const bool p6_ = h->sph == MG_SPH_POLY6_SPIKY;                                            \
+        if (h->B > 0) p6_ ? GO(K<MG_SPH_POLY6_SPIKY, 1, 9>, nr_, 704u) : GO(K<MG_SPH_REFERENCE, 1, 9>, nr_, 704u); \
+        else if ((W) == 9) p6_ ? GO(K<MG_SPH_POLY6_SPIKY, 0, 9>, nr_, 576u) : GO(K<MG_SPH_REFERENCE, 0, 9>, nr_, 576u); \
+        else p6_ ? GO(K<MG_SPH_POLY6_SPIKY, 0, 3>, nr_, 192u) : GO(K<MG_SPH_REFERENCE, 0, 3>, nr_, 192u); \
+    } while (0)
+
 void launch_force(mg_handle* h, unsigned nb, const DS& d, int accumulate)
 {
+    const int W = force_rows(h, d);
+    auto go = [&](auto kernel, unsigned blocks, unsigned threads) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, h->st, d, h->p, h->g, accumulate);
+    };
+    if (W > 1) {
+        MG_FORCE_ROWS(k_force_rows, go, W);
+        return;
+    }
     if (h->sph == MG_SPH_POLY6_SPIKY)
         hipLaunchKernelGGL(k_force<MG_SPH_POLY6_SPIKY>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p, h->g,
                            accumulate);
@@ -932,29 +959,22 @@ void launch_force(mg_handle* h, unsigned nb, const DS& d, int accumulate)
 
 void launch_force_advance(mg_handle* h, unsigned nb, const DS& d, float dt, int special, float zoff)
 {
-    const bool poly6 = h->sph == MG_SPH_POLY6_SPIKY;
-    auto rows = [&](auto kernel, unsigned waves) {
-        hipLaunchKernelGGL(kernel, dim3(nblk(h->N, 64)), dim3(64 * waves), 0, h->st, d, h->p, h->g, dt, special, zoff);
+    const int W = force_rows(h, d);
+    auto go = [&](auto kernel, unsigned blocks, unsigned threads) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, h->st, d, h->p, h->g, dt, special, zoff);
     };
-    if (rows_of_three(h, d)) {
-        /* split by rows the bonds come as records only */
-        if (h->B > 0 && d.ETR && h->N <= kForceRows9)
-            return poly6 ? rows(k_force_advance_rows<MG_SPH_POLY6_SPIKY, 1, 9>, 11)
-                         : rows(k_force_advance_rows<MG_SPH_REFERENCE, 1, 9>, 11);
-        if (h->B == 0 && h->N <= kForceRows9NoBonds)
-            return poly6 ? rows(k_force_advance_rows<MG_SPH_POLY6_SPIKY, 0, 9>, 9)
-                         : rows(k_force_advance_rows<MG_SPH_REFERENCE, 0, 9>, 9);
-        if (h->B == 0 && h->N <= kForceRows3NoBonds)
-            return poly6 ? rows(k_force_advance_rows<MG_SPH_POLY6_SPIKY, 0, 3>, 3)
-                         : rows(k_force_advance_rows<MG_SPH_REFERENCE, 0, 3>, 3);
+    if (W > 1) {
+        MG_FORCE_ROWS(k_force_advance_rows, go, W);
+        return;
     }
-    if (poly6)
+    if (h->sph == MG_SPH_POLY6_SPIKY)
         hipLaunchKernelGGL(k_force_advance<MG_SPH_POLY6_SPIKY>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p,
                            h->g, dt, special, zoff);
     else
         hipLaunchKernelGGL(k_force_advance<MG_SPH_REFERENCE>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p,
                            h->g, dt, special, zoff);
 }
+#undef MG_FORCE_ROWS
 
 /* The FCONC float4 groups the diffusion sweep reads and the per-TF coefficients
  * tf_diffusability * diff_scale (the same float operations as the reference's loop). */

@@ -1163,6 +1163,7 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_pressure(DS d, MgParams p, MgGrid g)
 #define RS_ROWS 9
 #define RS_CELLS 3 /* cells per row */
 #define RS_OCC 5   /* wavefronts per SIMD: at most 96 VGPRs */
+#define RS_FOCC 6  /* the force: at most 80, two of its workgroups of eleven per CU */
 
 /* A row of the neighbourhood seen by a wavefront: the lane's cells [b[k], b[k + 1]) and the
  * wavefront's slot band [blo, blo + n) in LDS (staged = 0: the band is wider than the stage and
@@ -1880,15 +1881,15 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_force_advance(DS d, MgParams p, MgGrid g, 
 }
 
 /* ------------------------------------------------- force + advance split by rows
- * k_force_advance for 64 particles per workgroup: a wavefront per row of the neighbourhood (see
+ * k_force_advance (or k_force) for 64 particles per workgroup: a wavefront per row of the neighbourhood (see
  * RS_ROWS) and, with bonds, two more: wavefront 9 sums the own bonds' records and updates their
  * integrators, wavefront 10 fetches the incoming bonds' records (the first RS_INC of each
  * particle into registers) while the rows are swept, then adds everything up in force_one's
  * order and advances. Bonds come as the pressure pass's records only (d.ETR). */
 #define RS_INC 12
-template <int MODE, int BONDS, int W>
-__device__ __forceinline__ void force_advance_rows_body(const DS& d, const MgParams& p, const MgGrid& g, float dt,
-                                                        uint32_t bid, int special = 0, float zoff = 0.0f)
+template <int MODE, int BONDS, int W, class Finish>
+__device__ __forceinline__ void force_rows_body(const DS& d, const MgParams& p, const MgGrid& g, uint32_t bid,
+                                                bool accumulate, Finish finish)
 {
     constexpr int PER = RS_ROWS / W; /* rows per wavefront */
     __shared__ Band<1> bands[W];
@@ -1973,8 +1974,8 @@ __device__ __forceinline__ void force_advance_rows_body(const DS& d, const MgPar
                 ks[k] = d.SLOT[kh];
                 r[k] = d.ETR[(size_t)b * N + kh];
             }
-            /* a term that force_one leaves out adds +0 here: FFORCE is a sum that starts at +0,
-             * so it is never -0 and keeps its bits */
+            /* a term that force_one leaves out adds +0 here: F0 + force is never -0 (force is a sum
+             * that starts at +0), so it keeps its bits */
 #pragma unroll
             for (int k = 0; k < RS_INC; k++) {
                 const f3 t = mk3(r[k].x, r[k].y, r[k].z);
@@ -1987,24 +1988,43 @@ __device__ __forceinline__ void force_advance_rows_body(const DS& d, const MgPar
     f3 F = mk3(0.0f, 0.0f, 0.0f);
     if (valid) {
         f3 fsum = mk3(0.0f, 0.0f, 0.0f);
-#pragma unroll
+#pragma unroll 9 /* whole, the reads of all 81 sums are hoisted and spill */
         for (int k = 0; k < RS_ROWS * RS_CELLS; k++)
             fsum = fsum + mk3(part[k][0][lane], part[k][1][lane], part[k][2][lane]);
         f3 force = mk3(0.0f, 0.0f, 0.0f);
         if (BONDS) force = mk3(own[0][lane], own[1][lane], own[2][lane]);
         force = force + fsum * p.pmass;
-        F = mk3(0.0f, 0.0f, 0.0f) + force;
+        F = (accumulate ? xyz(d.F[i]) : mk3(0.0f, 0.0f, 0.0f)) + force;
         if (BONDS) {
 #pragma unroll
             for (int k = 0; k < RS_INC; k++) F = F + in[k];
             if (e0 + RS_INC < e1) F = incoming_records(d, na, e0 + RS_INC, e1, F);
         }
     }
-    if (i < N) advance_other_half(d, p, dt, i, valid, F, special, zoff);
+    finish(i, valid, F);
 }
 
 template <int MODE, int BONDS, int W>
-__global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? RS_OCC : 3) void k_force_advance_rows(DS d, MgParams p,
+__device__ __forceinline__ void force_advance_rows_body(const DS& d, const MgParams& p, const MgGrid& g, float dt,
+                                                        uint32_t bid, int special = 0, float zoff = 0.0f)
+{
+    force_rows_body<MODE, BONDS, W>(d, p, g, bid, false, [&](uint32_t i, bool valid, f3 F) {
+        if (i < (uint32_t)d.N) advance_other_half(d, p, dt, i, valid, F, special, zoff);
+    });
+}
+
+/* ComputeForceCL (k_force) split by rows */
+template <int MODE, int BONDS, int W>
+__global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? (BONDS ? RS_FOCC : RS_OCC) : 3) void k_force_rows(DS d, MgParams p, MgGrid g,
+                                                                                          int accumulate)
+{
+    force_rows_body<MODE, BONDS, W>(d, p, g, xcd_block(), accumulate != 0, [&](uint32_t i, bool valid, f3 F) {
+        if (valid) d.F[i] = make_float4(F.x, F.y, F.z, 0.0f);
+    });
+}
+
+template <int MODE, int BONDS, int W>
+__global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? (BONDS ? RS_FOCC : RS_OCC) : 3) void k_force_advance_rows(DS d, MgParams p,
                                                                                                   MgGrid g, float dt,
                                                                                                   int special, float zoff)
 {
@@ -3356,7 +3376,7 @@ __global__ __launch_bounds__(64 * W, RS_OCC) void kb_pressure_rows(const BatchIn
     pressure_rows_body<MG_SPH_REFERENCE, W>(global_view(in.pressure), in.p, in.g, b - in.pb0, in.pnb);
 }
 
-__global__ __launch_bounds__(64 * (RS_ROWS + 2), RS_OCC) void kb_force_advance_rows(const BatchInst* __restrict__ I,
+__global__ __launch_bounds__(64 * (RS_ROWS + 2), RS_FOCC) void kb_force_advance_rows(const BatchInst* __restrict__ I,
                                                                                    const uint16_t* __restrict__ map)
 {
     const uint32_t b = xcd_block();
