@@ -1290,14 +1290,16 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
         d.cull = 0; /* positions moved since the binning */
         d.HMR = hm; /* within the skin, unless the force-advance raised MG_C_SKIN */
         const DiffPlan dp = diff_plan(h);
-        if (genes && rows_of_three(h, d) && h->N <= kDiffuseRows)
+        if (!genes)
+            hipLaunchKernelGGL(k_insert_next, dim3(nb), dim3(256), 0, h->st, d, h->g);
+        else if (rows_of_three(h, d) && h->N <= kDiffuseRows)
             launch_diffuse_rows<RS_DIFFUSE | RS_GENES | RS_INSERT>(h, d, dp);
         else if (dp.ng <= 1)
-            hipLaunchKernelGGL(k_diffuse_genes_insert<1>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p, h->g, h->gen, dp, genes);
+            hipLaunchKernelGGL(k_diffuse_genes_insert<1>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p, h->g, h->gen, dp);
         else if (dp.ng == 2)
-            hipLaunchKernelGGL(k_diffuse_genes_insert<2>, dim3(nb), dim3(256), band_lds<2>(256), h->st, d, h->p, h->g, h->gen, dp, genes);
+            hipLaunchKernelGGL(k_diffuse_genes_insert<2>, dim3(nb), dim3(256), band_lds<2>(256), h->st, d, h->p, h->g, h->gen, dp);
         else
-            hipLaunchKernelGGL(k_diffuse_genes_insert<4>, dim3(nb), dim3(256), band_lds<4>(256), h->st, d, h->p, h->g, h->gen, dp, genes);
+            hipLaunchKernelGGL(k_diffuse_genes_insert<4>, dim3(nb), dim3(256), band_lds<4>(256), h->st, d, h->p, h->g, h->gen, dp);
     }
     {
         PhaseScope ps(h, MG_PH_SCAN);
@@ -1315,7 +1317,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
     }
     {
         PhaseScope ps(h, MG_PH_SORT);
-        DS d = make_ds(h, 1, 1);
+        DS d = make_ds(h, 1, genes); /* without gene action the concentrations are where they were */
         d.GMN = h->GMN;
         d.CNT = d.CNTN; /* the grid k_place binned into */
         d.OFF = d.OFFN;
@@ -1325,6 +1327,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
     HIPCHK(hipGetLastError());
     h->icur = 1 - h->icur;
     h->gcur = 1 - h->gcur;
+    if (!genes) h->ccur = 1 - h->ccur;
     h->force_zero = true;
     h->normalized = false;
     h->gene_grid_stale = true;
@@ -1335,8 +1338,8 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
 }
 
 /* Two fused steps captured once into a hipGraph and replayed; the step has a two-step
- * period in its buffer roles (icur, gcur flip every step), so a two-step graph leaves the
- * handle's indices where they started. Recaptured when dt, flags, the parities or the
+ * period in its buffer roles (icur, gcur flip every step, without genes ccur too), so a two-step
+ * graph leaves the handle's indices where they started. Recaptured when dt, flags, the parities or the
  * handle's epoch change. */
 int graph_steps(mg_handle* h, int pairs, float dt, unsigned flags, const mg_net* net = nullptr)
 {

@@ -2277,10 +2277,37 @@ __device__ __forceinline__ void diffuse_genes_insert_body(const DS& d, const MgP
 
 template <int NG>
 __global__ LAUNCH_BOUNDS_SWEEP void k_diffuse_genes_insert(DS d, MgParams p, MgGrid g, MgGenome gen,
-                                                           DiffPlan dp, int genes)
+                                                           DiffPlan dp)
 {
     extern __shared__ float4 mg_lds[];
-    diffuse_genes_insert_body<NG>(d, p, g, gen, dp, genes, (Band<NG>*)mg_lds, xcd_block());
+    diffuse_genes_insert_body<NG>(d, p, g, gen, dp, 1, (Band<NG>*)mg_lds, xcd_block());
+}
+
+/* The fused step's insert without gene action: binning into the next grid and the membership for
+ * the coming sort; bound by its reads (84 bytes per particle) and the binning's atomics. The
+ * concentrations stay where they are and the sort moves them on: through k_diffuse_genes_insert
+ * they were copied once more, and 1,000,000 particles took 49 us instead of 23, 262,144 15.6
+ * instead of 7.6; a step of 32,768 42.7 instead of 41.6. */
+__global__ LAUNCH_BOUNDS_256 void k_insert_next(DS d, MgGrid g)
+{
+    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
+    const bool valid = i < (uint32_t)d.N;
+    float4 P_i = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (valid) {
+        P_i = d.P[i];
+        uint32_t mnext = 0;
+        if (i < d.ctr[MG_C_NUM_POINTS]) {
+            const uint32_t h = d.HOME[i];
+            uint32_t epi[MG_NUM_GENES];
+#pragma unroll
+            for (int k = 0; k < MG_NUM_GENES; k++) epi[k] = d.EPIGEN[(size_t)k * d.N + h];
+#pragma unroll
+            for (int k = 0; k < MG_NUM_GENES; k++)
+                if (epi[k] > 0u) mnext |= 1u << k;
+        }
+        d.GMN[i] = mnext;
+    }
+    insert_one(d, g, i, valid, P_i, d.CNTN, nullptr);
 }
 
 /* ---------------------------------- diffusion, genes and insert split by rows
