@@ -101,6 +101,20 @@ __global__ void k_rehome_flags(const uint32_t* __restrict__ SLOT, uint32_t* __re
     unplaced[h] = s >= (uint32_t)n;
     if (s < (uint32_t)n && atomicExch(&unused[s], 0u) == 0u) stat[0] = 1u; /* set to 1 before the launch */
 }
+/* stat[2]: nonzero when a particle's row of the neighbourhood holds more than 64 candidates */
+__global__ void k_rehome_dense(DS d, MgGrid g, uint32_t* __restrict__ stat)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t gc = i < d.ctr[MG_C_ACTIVE] ? d.GCELL[i] : MG_GRID_UNDEF;
+    if (gc == MG_GRID_UNDEF) return;
+    const uint32_t gc0 = gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
+    bool wide = false;
+    for (int s = 0; s < RS_ROWS; s++) {
+        const uint32_t c = gc0 + (uint32_t)g.adj[s * RS_CELLS];
+        wide |= d.OFF[c + RS_CELLS] - d.OFF[c] > 64u;
+    }
+    if (wide) stat[2] = 1u;
+}
 __global__ void k_rehome_numbers(const uint32_t* __restrict__ unused, const uint32_t* __restrict__ rank,
                                  uint32_t* __restrict__ number, int n)
 {
@@ -329,6 +343,8 @@ struct mg_handle {
     uint64_t* LIVE = nullptr; /* per home: bit a set when bond slot a holds a partner */
     uint64_t* HM = nullptr;   /* hit masks, pressure -> force of a fused step: [row][slot] */
     int hm_rows = 0;          /* rows HM holds per slot */
+    uint32_t* DL = nullptr;   /* dense groups of a fused step */
+    bool dense = false;       /* the last re-homing saw such groups: fused steps list them */
     float4* ET = nullptr;     /* bond records, pressure -> force beside the masks: [bond slot][home] */
     /* grid */
     uint32_t *CNT[2] = {}, *OFF[2] = {};  /* gcur is current; the fused step bins into 1-gcur */
@@ -656,6 +672,7 @@ DS make_ds(mg_handle* h, int kin = 0, int conc = 0)
     d.HMR = nullptr;
     d.ETW = nullptr;
     d.ETR = nullptr;
+    d.DL = nullptr;
     d.dry = 0;
     d.ctr = h->ctr;
     d.N = h->N; d.B = h->B; d.C = h->C;
@@ -832,8 +849,10 @@ int normalize(mg_handle* h)
  * incoming-bond row keeping its entries in their order, so the force gathers the same terms
  * in the same order: no result changes. */
 const int kRehomeSteps = 2048;
+const int kDiffuseRows = 57344; /* largest model whose diffusion is split by rows, see launch_diffuse_rows */
+bool rows_of_three(const mg_handle* h, const DS& d) { return d.rows && h->g.srch == RS_CELLS; }
 
-/* Device only but for one 8-byte read: each array is scattered into the staging buffer and copied
+/* Device only but for one 12-byte read: each array is scattered into the staging buffer and copied
  * back, so no address changes and captured graphs stay valid. 64,000 particles with 32 bond slots:
  * 0.65 ms (with the permutation and the rows made on the host and every array allocated anew
  * 3.7 ms; 262,144: 9 ms), on each new state and every kRehomeSteps. */
@@ -842,7 +861,7 @@ int rehome(mg_handle* h)
     const int N = h->N, B = h->B;
     const unsigned nb = nblk(N), tiles = (unsigned)((N + SCAN_TILE - 1) / SCAN_TILE);
     const size_t row = ((size_t)N * 4 + 255) / 256 * 256;
-    const size_t words = 5 * row + (2 * (size_t)tiles + 2) * 4;
+    const size_t words = 5 * row + (2 * (size_t)tiles + 3) * 4;
     size_t most = (size_t)MG_NUM_GENES * N * 4; /* the largest array moved */
     if (B > 0) most = std::max(most, (size_t)B * N * sizeof(float4));
     most = std::max(most, std::max<size_t>(h->inc_cap, 1) * 4);
@@ -858,16 +877,25 @@ int rehome(mg_handle* h)
         hipLaunchKernelGGL(k_tile_scan, dim3(tiles), dim3(256), 0, h->st, in, out, N, excl);
     };
     CHK(fill_u32(h, unused, 1, N));
-    CHK(fill_u32(h, stat, 0, 2));
+    CHK(fill_u32(h, stat, 0, 3));
     hipLaunchKernelGGL(k_rehome_flags, dim3(nb), dim3(256), 0, h->st, h->SLOT, unused, unplaced, stat, N);
     sum(unused, rank);
     hipLaunchKernelGGL(k_rehome_numbers, dim3(nb), dim3(256), 0, h->st, unused, rank, number, N);
     sum(unplaced, rank);
     hipLaunchKernelGGL(k_rehome_sigma, dim3(nb), dim3(256), 0, h->st, h->SLOT, rank, number, sigma, stat, N);
+    const DS now = make_ds(h);
+    if (N > kDiffuseRows && rows_of_three(h, now))
+        hipLaunchKernelGGL(k_rehome_dense, dim3(nb), dim3(256), 0, h->st, now, h->g, stat);
     HIPCHK(hipGetLastError());
-    uint32_t seen[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(seen, stat, 8, hipMemcpyDeviceToHost, h->st));
+    uint32_t seen[3] = {0, 0, 0};
+    HIPCHK(hipMemcpyAsync(seen, stat, 12, hipMemcpyDeviceToHost, h->st));
     HIPCHK(hipStreamSynchronize(h->st));
+    if (seen[2] && !h->DL) {
+        const size_t n = 1 + MG_DENSE_MAX + (size_t)nb * 4;
+        CHK(dalloc(h, &h->DL, n));
+        CHK(fill_u32(h, h->DL, 0, n));
+    }
+    h->dense = seen[2] != 0;
     if (seen[0]) return MG_OK; /* not a permutation: leave the homes as they are */
     h->rehome_due = false;
     h->steps_since_rehome = 0;
@@ -944,8 +972,6 @@ template <int NX, int CAP = BAND_CAP> constexpr size_t band_lds(unsigned threads
 const int kPressureRows9 = 49152;
 const int kForceRows9 = 147456, kForceRows9NoBonds = 40960, kForceRows3NoBonds = 131072;
 
-bool rows_of_three(const mg_handle* h, const DS& d) { return d.rows && h->g.srch == RS_CELLS; }
-
 /* the pressure and force launches for the handle's SPH kernels */
 void launch_pressure(mg_handle* h, unsigned nb, const DS& d)
 {
@@ -973,13 +999,14 @@ int force_rows(const mg_handle* h, const DS& d)
     return h->N <= kForceRows9NoBonds ? 9 : h->N <= kForceRows3NoBonds ? 3 : 1;
 }
 
-/* go(kernel, blocks, threads per block) with K<MODE, BONDS, W> for a view split over W wavefronts */
-#define MG_FORCE_ROWS(K, GO, W)                                                                   \
+/* go(kernel, blocks, threads per block) with K<MODE, BONDS, W> for a view split over W wavefronts,
+ * or over nine for its dense groups */
+#define MG_FORCE_ROWS(K, GO, D, W)                                                                   \
     do {                                                                                          \
-        const unsigned nr_ = nblk(h->N, 64);                                                      \
+        const unsigned nr_ = (D).DL ? MG_DENSE_MAX : nblk(h->N, 64);                              \
         const bool p6_ = h->sph == MG_SPH_POLY6_SPIKY;                                            \
         if (h->B > 0) p6_ ? GO(K<MG_SPH_POLY6_SPIKY, 1, 9>, nr_, 704u) : GO(K<MG_SPH_REFERENCE, 1, 9>, nr_, 704u); \
-        else if ((W) == 9) p6_ ? GO(K<MG_SPH_POLY6_SPIKY, 0, 9>, nr_, 576u) : GO(K<MG_SPH_REFERENCE, 0, 9>, nr_, 576u); \
+        else if ((W) == 9 || (D).DL) p6_ ? GO(K<MG_SPH_POLY6_SPIKY, 0, 9>, nr_, 576u) : GO(K<MG_SPH_REFERENCE, 0, 9>, nr_, 576u); \
         else p6_ ? GO(K<MG_SPH_POLY6_SPIKY, 0, 3>, nr_, 192u) : GO(K<MG_SPH_REFERENCE, 0, 3>, nr_, 192u); \
     } while (0)
 
@@ -989,9 +1016,9 @@ void launch_force(mg_handle* h, unsigned nb, const DS& d, int accumulate)
     auto go = [&](auto kernel, unsigned blocks, unsigned threads) {
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, h->st, d, h->p, h->g, accumulate);
     };
-    if (W > 1) {
-        MG_FORCE_ROWS(k_force_rows, go, W);
-        return;
+    if (W > 1 || d.DL) {
+        MG_FORCE_ROWS(k_force_rows, go, d, W);
+        if (W > 1) return;
     }
     if (h->sph == MG_SPH_POLY6_SPIKY)
         hipLaunchKernelGGL(k_force<MG_SPH_POLY6_SPIKY>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p, h->g,
@@ -1007,9 +1034,9 @@ void launch_force_advance(mg_handle* h, unsigned nb, const DS& d, float dt, int 
     auto go = [&](auto kernel, unsigned blocks, unsigned threads) {
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, h->st, d, h->p, h->g, dt, special, zoff);
     };
-    if (W > 1) {
-        MG_FORCE_ROWS(k_force_advance_rows, go, W);
-        return;
+    if (W > 1 || d.DL) {
+        MG_FORCE_ROWS(k_force_advance_rows, go, d, W);
+        if (W > 1) return;
     }
     if (h->sph == MG_SPH_POLY6_SPIKY)
         hipLaunchKernelGGL(k_force_advance<MG_SPH_POLY6_SPIKY>, dim3(nb), dim3(256), band_lds<1>(256), h->st, d, h->p,
@@ -1052,8 +1079,6 @@ DiffPlan diff_plan(const mg_handle* h)
  * three cells per axis on the row-structured grid): fused with the insert 32,768 particles
  * 24.8 us against 48.8 with a lane per particle, 46,656: 39.9 / 49.3, 54,872: 46.3 / 50.3,
  * 64,000: 53.9 / 50.5. */
-const int kDiffuseRows = 57344;
-
 template <int PART> void launch_diffuse_rows(mg_handle* h, const DS& d, const DiffPlan& dp)
 {
     hipLaunchKernelGGL(k_diffuse_rows<PART>, dim3(nblk(h->N, 64)), dim3(64 * RS_ROWS), 0, h->st, d, h->p, h->g, h->gen, dp);
@@ -1239,14 +1264,24 @@ uint64_t* hit_masks(const mg_handle* h)
  * read by the force pass that visits them (the same positions) */
 float4* bond_records(const mg_handle* h, const uint64_t* hm) { return hm ? h->ET : nullptr; }
 
+/* the list of dense groups for a fused step (see dense_listed): larger models than the diffusion
+ * split by rows throughout, whose pressure pass is split over three wavefronts and hands masks on */
+uint32_t* dense_groups(const mg_handle* h, const uint64_t* hm)
+{
+    const bool rows = h->grid_scanned && h->adj_rows && h->g.srch == RS_CELLS;
+    return h->dense && rows && hm && h->N > kDiffuseRows && (h->B == 0 || h->ET) ? h->DL : nullptr;
+}
+
 int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nullptr)
 {
     const int genes = (flags & MG_STEP_GENES) ? 1 : 0;
     const unsigned nb = nblk(h->N);
     uint64_t* hm = hit_masks(h);
+    uint32_t* dl = dense_groups(h, hm);
     {
         PhaseScope ps(h, MG_PH_PRESSURE);
         DS d = make_ds(h);
+        d.DL = dl;
         d.ZERO = h->CNT[1 - h->gcur];
         d.zero_n = (uint32_t)h->C;
         d.HMW = hm;
@@ -1263,6 +1298,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
             DS d = make_ds(h);
             d.HMR = hm;
             d.ETR = bond_records(h, hm);
+            if (force_rows(h, d) == 1) d.DL = dl;
             launch_force(h, nb, d, 0);
         }
         {
@@ -1281,6 +1317,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
         DS d = make_ds(h);
         d.HMR = hm;
         d.ETR = bond_records(h, hm);
+        if (force_rows(h, d) == 1) d.DL = dl;
         launch_force_advance(h, nb, d, dt, special, zoff);
     }
     {
@@ -1290,6 +1327,10 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
         d.cull = 0; /* positions moved since the binning */
         d.HMR = hm; /* within the skin, unless the force-advance raised MG_C_SKIN */
         const DiffPlan dp = diff_plan(h);
+        if (genes && dl) {
+            d.DL = dl;
+            hipLaunchKernelGGL(k_diffuse_dense, dim3(MG_DENSE_MAX), dim3(64 * RS_ROWS), 0, h->st, d, h->p, h->g, h->gen, dp);
+        }
         if (!genes)
             hipLaunchKernelGGL(k_insert_next, dim3(nb), dim3(256), 0, h->st, d, h->g);
         else if (rows_of_three(h, d) && h->N <= kDiffuseRows)
@@ -1313,6 +1354,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
         DS d = make_ds(h);
         d.CNT = d.CNTN;
         d.OFF = d.OFFN;
+        d.DL = dl;
         hipLaunchKernelGGL(k_place, dim3(nb), dim3(256), 0, h->st, d);
     }
     {
@@ -1344,7 +1386,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
 int graph_steps(mg_handle* h, int pairs, float dt, unsigned flags, const mg_net* net = nullptr)
 {
     ensure_hit_masks(h); /* allocates (and bumps the epoch) before any capture, not inside it */
-    const int parity = ((h->cells_fresh && h->grid_scanned) << 4) | (h->kcur << 3) | (h->icur << 2) |
+    const int parity = (h->dense << 5) | ((h->cells_fresh && h->grid_scanned) << 4) | (h->kcur << 3) | (h->icur << 2) |
                        (h->ccur << 1) | h->gcur;
     const uint64_t nv = net ? net_version(net) : 0;
     if (!h->graph || h->graph_epoch != h->epoch || h->graph_dt != dt || h->graph_flags != flags ||

@@ -50,6 +50,8 @@ enum {
 #define MG_SKIN_LIM 1.0201f
 #define MG_SKIN_DISP2 1.6e-5f
 
+#define MG_DENSE_MAX 1024u
+
 struct DS {
     /* sorted, current */
     float4 *P, *V, *VEL, *F;
@@ -98,6 +100,10 @@ struct DS {
      * incoming bonds instead of evaluating each bond twice. Null when not in use. */
     float4* ETW;
     const float4* ETR;
+    /* Dense groups of a fused step: [0] how many, [1 ..] up to MG_DENSE_MAX groups of 64 slots,
+     * then per group whether it is listed. The pressure pass lists them, the force and diffusion
+     * passes split them by rows, and the placement empties the list. Null when not in use. */
+    uint32_t* DL;
     /* 1: a force pass that changes no bond record (no integrators, no breaking), for the
      * learned step's training inputs */
     int dry;

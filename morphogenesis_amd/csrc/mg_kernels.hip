@@ -453,7 +453,11 @@ __device__ __forceinline__ void place_body(const DS& d, uint32_t bid)
     d.PERM[d.OFF[c] + d.GNDX[s]] = s;
 }
 
-__global__ LAUNCH_BOUNDS_256 void k_place(DS d) { place_body(d, blockIdx.x); }
+__global__ LAUNCH_BOUNDS_256 void k_place(DS d)
+{
+    if (d.DL && blockIdx.x == 0 && threadIdx.x == 0) d.DL[0] = 0u; /* its readers of this step are done */
+    place_body(d, blockIdx.x);
+}
 
 /* ------------------------------------------------------- counting sort (a7)
  * countingSortFull (src/fluid_system_cuda.cu:196-296) with the host resets of
@@ -1350,6 +1354,7 @@ __device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& 
     constexpr int PER = RS_ROWS / W; /* rows per wavefront */
     __shared__ Band<0> bands[W];
     __shared__ float part[RS_ROWS * RS_CELLS][64];
+    __shared__ uint32_t list_me[W];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (d.ZERO)
@@ -1362,6 +1367,7 @@ __device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& 
     const f3 pi = valid ? xyz(d.P[i]) : mk3(0.f, 0.f, 0.f);
     const float inv_sr = pressure_inv_sr<MODE>(p), tlim = d.HMW ? fmaxf(MG_SKIN_LIM, p.r2) : p.r2;
     auto none = [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); };
+    bool wide = false; /* a row's window exceeds the 64 slots of a mask */
     for (int q = 0; q < PER; q++) {
         const int s = (int)w * PER + q;
 #pragma unroll
@@ -1369,6 +1375,7 @@ __device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& 
         RsRow r;
         if (q > 0) wave_lds_sync(); /* the previous row's reads are done */
         if (!rs_stage<0>(d, g, bands[w], valid, gc, s, none, r) || !valid) continue;
+        wide |= r.b[RS_CELLS] - r.b[0] > 64u;
         uint32_t flo, fhi, nflush = 0u;
         rs_live_range(d, g, r, s, pi, tlim, flo, fhi);
         float csum = 0.0f;
@@ -1391,8 +1398,24 @@ __device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& 
         if (d.HMW) d.HMW[(size_t)s * d.N + i] = r.b[RS_CELLS] - r.b[0] > 64u ? ~0ull : rec;
     }
     if (valid && d.ETW) rs_record_bonds<W>(d, p, i, w);
+    if (W == 3 && d.DL) {
+        const uint64_t wides = __ballot(wide);
+        if (lane == 0) list_me[w] = wides != 0ull;
+    }
     __syncthreads();
-    if (w != 0u || !valid) return;
+    if (w != 0u) return;
+    if (W == 3 && d.DL && lane == 0) {
+        uint32_t listed = 0u;
+        if (list_me[0] | list_me[1] | list_me[2]) {
+            const uint32_t at = atomicAdd(&d.DL[0], 1u);
+            if (at < MG_DENSE_MAX) {
+                d.DL[1 + at] = bid;
+                listed = 1u;
+            }
+        }
+        d.DL[1 + MG_DENSE_MAX + bid] = listed;
+    }
+    if (!valid) return;
     float sum = 0.0f;
 #pragma unroll
     for (int k = 0; k < RS_ROWS * RS_CELLS; k++) sum += part[k][lane];
@@ -1403,6 +1426,27 @@ template <int MODE, int W>
 __global__ __launch_bounds__(64 * W, RS_OCC) void k_pressure_rows(DS d, MgParams p, MgGrid g)
 {
     pressure_rows_body<MODE, W>(d, p, g, xcd_block(), gridDim.x);
+}
+
+/* Dense groups. A wavefront with one lane per particle walks its rows alone, so a few groups of 64
+ * in crowded cells (drops, compressed tissue) outlast the rest of a large model's pass by the
+ * length of their walk, with the chip idle. In a fused step of a model that had such groups when its
+ * homes were last numbered, the pressure pass lists the groups with a row of more than 64
+ * candidates (the hit masks end there too); the force and the diffusion take them nine wavefronts
+ * each, in a launch of their own, and the one-lane kernels pass them by. A falling column and four
+ * drops, 1,014,784 particles: force 444 -> 276 + 85 us, diffusion and genes 554 -> 236 + 142. */
+__device__ __forceinline__ bool dense_listed(const DS& d, uint32_t bid)
+{
+    return d.DL && d.DL[1 + MG_DENSE_MAX + bid * (blockDim.x >> 6) + (threadIdx.x >> 6)] != 0u;
+}
+/* the group a workgroup of a kernel split by rows works on; false: none */
+__device__ __forceinline__ bool rows_group(const DS& d, uint32_t& bid)
+{
+    bid = xcd_block();
+    if (!d.DL) return true;
+    if (blockIdx.x >= min(d.DL[0], MG_DENSE_MAX)) return false;
+    bid = d.DL[1 + blockIdx.x];
+    return true;
 }
 
 /* A hit's fluid force added to cf (P_i, V_i the particle, Pj, Vj the neighbour) */
@@ -1680,7 +1724,9 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_force(DS d, MgParams p, MgGrid g, int accu
 {
     extern __shared__ float4 mg_lds[];
     Band<1>* bands = (Band<1>*)mg_lds;
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t bid = xcd_block();
+    if (dense_listed(d, bid)) return;
+    const uint32_t i = bid * blockDim.x + threadIdx.x;
     const uint32_t na = d.ctr[MG_C_ACTIVE];
     const uint32_t gc = (i < na) ? d.GCELL[i] : MG_GRID_UNDEF;
     const bool valid = gc != MG_GRID_UNDEF;
@@ -1877,7 +1923,9 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_force_advance(DS d, MgParams p, MgGrid g, 
                                                     float zoff)
 {
     extern __shared__ float4 mg_lds[];
-    force_advance_body<MODE>(d, p, g, (Band<1>*)mg_lds, dt, xcd_block(), special, zoff);
+    const uint32_t bid = xcd_block();
+    if (dense_listed(d, bid)) return;
+    force_advance_body<MODE>(d, p, g, (Band<1>*)mg_lds, dt, bid, special, zoff);
 }
 
 /* ------------------------------------------------- force + advance split by rows
@@ -2018,7 +2066,9 @@ template <int MODE, int BONDS, int W>
 __global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? (BONDS ? RS_FOCC : RS_OCC) : 3) void k_force_rows(DS d, MgParams p, MgGrid g,
                                                                                           int accumulate)
 {
-    force_rows_body<MODE, BONDS, W>(d, p, g, xcd_block(), accumulate != 0, [&](uint32_t i, bool valid, f3 F) {
+    uint32_t bid;
+    if (!rows_group(d, bid)) return;
+    force_rows_body<MODE, BONDS, W>(d, p, g, bid, accumulate != 0, [&](uint32_t i, bool valid, f3 F) {
         if (valid) d.F[i] = make_float4(F.x, F.y, F.z, 0.0f);
     });
 }
@@ -2028,7 +2078,9 @@ __global__ __launch_bounds__(64 * (W + 2 * BONDS), W == 9 ? (BONDS ? RS_FOCC : R
                                                                                                   MgGrid g, float dt,
                                                                                                   int special, float zoff)
 {
-    force_advance_rows_body<MODE, BONDS, W>(d, p, g, dt, xcd_block(), special, zoff);
+    uint32_t bid;
+    if (!rows_group(d, bid)) return;
+    force_advance_rows_body<MODE, BONDS, W>(d, p, g, dt, bid, special, zoff);
 }
 
 /* ----------------------------------------------------------- diffusion (a12)
@@ -2280,7 +2332,9 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_diffuse_genes_insert(DS d, MgParams p, MgG
                                                            DiffPlan dp)
 {
     extern __shared__ float4 mg_lds[];
-    diffuse_genes_insert_body<NG>(d, p, g, gen, dp, 1, (Band<NG>*)mg_lds, xcd_block());
+    const uint32_t bid = xcd_block();
+    if (dense_listed(d, bid)) return;
+    diffuse_genes_insert_body<NG>(d, p, g, gen, dp, 1, (Band<NG>*)mg_lds, bid);
 }
 
 /* The fused step's insert without gene action: binning into the next grid and the membership for
@@ -2333,15 +2387,105 @@ __global__ LAUNCH_BOUNDS_256 void k_insert_next(DS d, MgGrid g)
 #define RS_GENES 2
 #define RS_INSERT 4
 #define RS_LIST 48
-template <int PART, class Gen>
+#define RS_AHEAD 4 /* hits a reader has in flight: with 8 most of a window's last eight are idle loads */
+#define RS_WINDOWS 4 /* of 64 slots, per row of a dense group: later ones are tested by their readers */
+struct RsLists {
+    Band<0> bands[RS_ROWS];
+    uint2 list[RS_LIST][64]; /* (weight, slot); NaN: recorded, not a hit */
+};
+struct RsMasks {
+    uint64_t mask[RS_ROWS][RS_WINDOWS][64];
+    uint32_t from[RS_ROWS][64], to[RS_ROWS][64]; /* the row's slots */
+};
+
+/* Diffusion of a dense group (dense_listed): hundreds of hits per particle would pass through the
+ * list a row at a time, the other wavefronts waiting. The wavefronts leave their rows' hit masks in
+ * LDS instead, one test per candidate, and the wavefront of each float4 group of FCONC walks the
+ * bits. Returns the sums of terms in nw, for wavefronts w < dp.ng. Bound by the scattered 16-byte
+ * reads of FCONC (64 cache lines per load). Some 400 groups of ~270 hits, with the genes: 142 us
+ * (through the list 344, and 278 without testing a row again each round; walking each window in
+ * step 241; eight hits in flight 212). */
+__device__ __forceinline__ void diffuse_dense(const DS& d, const MgGrid& g, const DiffPlan& dp, RsMasks& sh, bool valid,
+                                              uint32_t i, uint32_t gc0, uint32_t grp, float r2, float d2, bool hm_ok,
+                                              float4 cur, float nw[4])
+{
+    const uint32_t lane = threadIdx.x & 63u, N = (uint32_t)d.N;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto getp = [&](uint32_t j) { return d.P[j]; };
+    f3 pi = mk3(0.f, 0.f, 0.f);
+    uint32_t from = 0u, to = 0u;
+    if (valid && dp.ng > 0) {
+        pi = xyz(d.P[i]);
+        const uint32_t c0 = gc0 + (uint32_t)g.adj[w * RS_CELLS];
+        from = min(d.OFF[c0], N);
+        to = max(min(d.OFF[c0 + RS_CELLS], N), from);
+        const uint64_t given = hm_ok ? d.HMR[(size_t)w * N + i] : ~0ull;
+        if (given != ~0ull) {
+            sh.mask[w][0][lane] = given; /* of a row within one window */
+        } else {
+            for (uint32_t t = 0u; t < RS_WINDOWS && from + 64u * t < to; t++)
+                sh.mask[w][t][lane] = rs_test(from + 64u * t, min(from + 64u * t + 64u, to), pi, r2, getp);
+        }
+    }
+    sh.from[w][lane] = from;
+    sh.to[w][lane] = to;
+    __syncthreads();
+    if ((int)w < dp.ng && valid) {
+        const float4* C4 = (const float4*)d.CONC;
+        const float u4[4] = {cur.x, cur.y, cur.z, cur.w};
+        /* every lane goes through its own windows: in step, the busiest lane of each window would
+         * set the pace of all */
+        int s = -1;
+        uint32_t b = 0u, end = 0u, t = 0u;
+        uint64_t m = 0ull;
+        auto refill = [&]() { /* the next window with hits; m = 0: none is left */
+            while (m == 0ull) {
+                b += 64u;
+                t++;
+                while (b >= end) {
+                    if (++s == RS_ROWS) return;
+                    b = sh.from[s][lane];
+                    end = sh.to[s][lane];
+                    t = 0u;
+                }
+                m = t < RS_WINDOWS ? sh.mask[s][t][lane] : rs_test(b, min(b + 64u, end), pi, r2, getp);
+            }
+        };
+        refill();
+        while (m != 0ull) {
+            float4 pj[RS_AHEAD], cn[RS_AHEAD];
+            bool has[RS_AHEAD];
+#pragma unroll
+            for (int q = 0; q < RS_AHEAD; q++) {
+                has[q] = m != 0ull;
+                const uint32_t j = b + (has[q] ? (uint32_t)__builtin_ctzll(m) : 0u);
+                m &= m - 1ull;
+                pj[q] = d.P[j];
+                cn[q] = C4[(size_t)j * 4u + grp];
+            }
+            refill();
+#pragma unroll
+            for (int q = 0; q < RS_AHEAD; q++) {
+                const f3 dist = pi - xyz(pj[q]);
+                const float dsq = dot3(dist, dist);
+                if (!(has[q] && dsq < r2 && dsq > 0.0f)) continue;
+                const float cc = (r2 - dsq) * d2;
+                const float c4[4] = {cn[q].x, cn[q].y, cn[q].z, cn[q].w};
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (dp.dm & (1u << (4u * w + (uint32_t)k))) nw[k] += dp.D[4u * w + (uint32_t)k] * cc * (c4[k] - u4[k]);
+            }
+        }
+    }
+    __syncthreads(); /* the masks' LDS is used again */
+}
+
+template <int PART, bool DENSE, class Gen>
 __device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p, const MgGrid& g, const Gen& gen,
                                                   const DiffPlan& dp, uint32_t bid)
 {
     union Stage {
-        struct {
-            Band<0> bands[RS_ROWS];
-            uint2 list[RS_LIST][64]; /* (weight, slot); NaN: recorded, not a hit */
-        } a;
+        std::conditional_t<DENSE, RsMasks, RsLists> a;
         struct {
             float act[MG_NUM_GENES][64];
             uint32_t depi[MG_NUM_GENES][64];
@@ -2376,92 +2520,101 @@ __device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p
     if (PART & RS_DIFFUSE) {
         const float d2 = p.psimscale * p.psimscale, r2 = p.r2 / d2;
         const bool hm_ok = d.HMR != nullptr && d.ctr[MG_C_SKIN] == 0u && r2 == 1.0f;
-        f3 pi = mk3(0.f, 0.f, 0.f);
-        uint64_t m = 0ull;
-        if (valid) {
-            pi = xyz(d.P[i]);
-            m = hm_ok ? d.HMR[(size_t)w * N + i] : ~0ull;
-        }
-        RsRow r;
-        const bool any = dp.ng > 0 && rs_stage<0>(d, g, sh.a.bands[w], valid,
-                                                  gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1), (int)w,
-                                                  [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); }, r);
-        const bool test = m == ~0ull; /* the row's candidates have to be tested, 64 slots at a time */
-        auto getp_band = [&](uint32_t j) { return sh.a.bands[w].p[j - r.blo]; };
-        auto getp_global = [&](uint32_t j) { return d.P[j]; };
-        uint32_t n = 0u;
-        if (any && valid) {
-            if (test) {
-                for (uint32_t b = r.b[0]; b < r.b[RS_CELLS]; b += 64u) {
-                    const uint32_t hi = min(b + 64u, r.b[RS_CELLS]);
-                    m = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
-                    n += (uint32_t)__builtin_popcountll(m);
-                }
-            } else {
-                n = (uint32_t)__builtin_popcountll(m);
-            }
-        }
-        cnt[w][lane] = n;
-        __syncthreads();
-        uint32_t at = 0u, tot = 0u;
-#pragma unroll
-        for (uint32_t q = 0; q < RS_ROWS; q++) {
-            const uint32_t c = cnt[q][lane];
-            if (q < w) at += c;
-            tot += c;
-        }
-        const uint32_t most = wave_max(tot);
         float nw[4] = {0.f, 0.f, 0.f, 0.f};
-        const bool adds = (int)w < dp.ng;
-        for (uint32_t base = 0u; base < most; base += RS_LIST) {
-            if (any && valid && n != 0u) {
-                uint32_t k = at;
-                uint32_t b = r.b[0];
-                do {
-                    uint64_t mm = m;
-                    /* a row of one window keeps the mask of the count */
-                    if (test && r.b[RS_CELLS] - r.b[0] > 64u) {
+        if constexpr (DENSE) {
+            diffuse_dense(d, g, dp, sh.a, valid, i, gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1), grp, r2, d2, hm_ok,
+                          cur, nw);
+        } else {
+            f3 pi = mk3(0.f, 0.f, 0.f);
+            uint64_t m = 0ull;
+            if (valid) {
+                pi = xyz(d.P[i]);
+                m = hm_ok ? d.HMR[(size_t)w * N + i] : ~0ull;
+            }
+            RsRow r;
+            const bool any = dp.ng > 0 && rs_stage<0>(d, g, sh.a.bands[w], valid,
+                                                      gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1), (int)w,
+                                                      [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); }, r);
+            const bool test = m == ~0ull; /* the row's candidates have to be tested, 64 slots at a time */
+            auto getp_band = [&](uint32_t j) { return sh.a.bands[w].p[j - r.blo]; };
+            auto getp_global = [&](uint32_t j) { return d.P[j]; };
+            uint32_t n = 0u;
+            if (any && valid) {
+                if (test) {
+                    for (uint32_t b = r.b[0]; b < r.b[RS_CELLS]; b += 64u) {
                         const uint32_t hi = min(b + 64u, r.b[RS_CELLS]);
-                        mm = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
+                        m = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
+                        n += (uint32_t)__builtin_popcountll(m);
                     }
-                    while (mm != 0ull) {
-                        const uint32_t j = b + (uint32_t)__builtin_ctzll(mm);
-                        mm &= mm - 1ull;
-                        const uint32_t e = k - base; /* wraps below the round's entries */
-                        k++;
-                        if (e >= RS_LIST) continue;
+                } else {
+                    n = (uint32_t)__builtin_popcountll(m);
+                }
+            }
+            cnt[w][lane] = n;
+            __syncthreads();
+            uint32_t at = 0u, tot = 0u;
+#pragma unroll
+            for (uint32_t q = 0; q < RS_ROWS; q++) {
+                const uint32_t c = cnt[q][lane];
+                if (q < w) at += c;
+                tot += c;
+            }
+            const uint32_t most = wave_max(tot);
+            const bool adds = (int)w < dp.ng;
+            /* the row's hits in turn, k the place of the next: `left` of the window from b, then the
+             * windows from `next` on. A row of one window keeps the mask of the count; wider ones are
+             * tested once more as the list takes them */
+            uint32_t k = at, b = 0u, next = 0u, stop = 0u;
+            uint64_t left = 0ull;
+            if (any && valid && n != 0u) {
+                b = next = r.b[0];
+                if (test && r.b[RS_CELLS] - r.b[0] > 64u) stop = r.b[RS_CELLS];
+                else left = m;
+            }
+            for (uint32_t base = 0u; base < most; base += RS_LIST) {
+                const uint32_t end = base + RS_LIST;
+                while (k < end && (left != 0ull || next < stop)) {
+                    if (left == 0ull) {
+                        b = next;
+                        next += 64u;
+                        const uint32_t hi = min(next, stop);
+                        left = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
+                    }
+                    while (left != 0ull && k < end) {
+                        const uint32_t j = b + (uint32_t)__builtin_ctzll(left);
+                        left &= left - 1ull;
                         const float4 pj = r.staged ? getp_band(j) : getp_global(j);
                         const f3 dist = pi - xyz(pj);
                         const float dsq = dot3(dist, dist);
                         const float cc = dsq < r2 && dsq > 0.0f ? (r2 - dsq) * d2 : __builtin_nanf("");
-                        sh.a.list[e][lane] = make_uint2(__float_as_uint(cc), j);
-                    }
-                    b += 64u;
-                } while (test && b < r.b[RS_CELLS]);
-            }
-            __syncthreads();
-            if (adds) {
-                const uint32_t ne = tot > base ? min(tot - base, (uint32_t)RS_LIST) : 0u;
-                for (uint32_t e0 = 0; e0 < ne; e0 += 4) {
-                    uint2 en[4];
-                    float4 cn[4];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) en[q] = sh.a.list[min(e0 + (uint32_t)q, ne - 1u)][lane];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) cn[q] = C4[(size_t)en[q].y * 4u + grp];
-#pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        const float cc = __uint_as_float(en[q].x);
-                        if (!(e0 + (uint32_t)q < ne && cc == cc)) continue;
-                        const float c4[4] = {cn[q].x, cn[q].y, cn[q].z, cn[q].w};
-                        const float u4[4] = {cur.x, cur.y, cur.z, cur.w};
-#pragma unroll
-                        for (int t = 0; t < 4; t++)
-                            if (dp.dm & (1u << (4u * w + (uint32_t)t))) nw[t] += dp.D[4u * w + (uint32_t)t] * cc * (c4[t] - u4[t]);
+                        sh.a.list[k - base][lane] = make_uint2(__float_as_uint(cc), j);
+                        k++;
                     }
                 }
+                __syncthreads();
+                if (adds) {
+                    const uint32_t ne = tot > base ? min(tot - base, (uint32_t)RS_LIST) : 0u;
+                    for (uint32_t e0 = 0; e0 < ne; e0 += 4) {
+                        uint2 en[4];
+                        float4 cn[4];
+#pragma unroll
+                        for (int q = 0; q < 4; q++) en[q] = sh.a.list[min(e0 + (uint32_t)q, ne - 1u)][lane];
+#pragma unroll
+                        for (int q = 0; q < 4; q++) cn[q] = C4[(size_t)en[q].y * 4u + grp];
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            const float cc = __uint_as_float(en[q].x);
+                            if (!(e0 + (uint32_t)q < ne && cc == cc)) continue;
+                            const float c4[4] = {cn[q].x, cn[q].y, cn[q].z, cn[q].w};
+                            const float u4[4] = {cur.x, cur.y, cur.z, cur.w};
+#pragma unroll
+                            for (int t = 0; t < 4; t++)
+                                if (dp.dm & (1u << (4u * w + (uint32_t)t))) nw[t] += dp.D[4u * w + (uint32_t)t] * cc * (c4[t] - u4[t]);
+                        }
+                    }
+                }
+                __syncthreads();
             }
-            __syncthreads();
         }
         if (valid && w < 4u) {
             cur.x = (float)gen.tf_breakdown_rate[4u * grp + 0u] * (cur.x + nw[0]);
@@ -2574,7 +2727,15 @@ template <int PART>
 __global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_rows(DS d, MgParams p, MgGrid g, MgGenome gen,
                                                                        DiffPlan dp)
 {
-    diffuse_rows_body<PART>(d, p, g, gen, dp, xcd_block());
+    diffuse_rows_body<PART, false>(d, p, g, gen, dp, xcd_block());
+}
+
+/* the listed dense groups of a fused step */
+__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_dense(DS d, MgParams p, MgGrid g, MgGenome gen,
+                                                                        DiffPlan dp)
+{
+    uint32_t bid;
+    if (rows_group(d, bid)) diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT, true>(d, p, g, gen, dp, bid);
 }
 
 /* -------------------------------------------------------- bond formation
@@ -3416,7 +3577,7 @@ __global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void kb_diffuse_rows(const Ba
 {
     const uint32_t b = xcd_block();
     const BatchInst& in = I[map[b]];
-    diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT>(global_view(in.diffuse), in.p, in.g, const_genome(in.gen), in.dp,
+    diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT, false>(global_view(in.diffuse), in.p, in.g, const_genome(in.gen), in.dp,
                                                          b - in.pb0);
 }
 
