@@ -892,10 +892,10 @@ int rehome(mg_handle* h)
     HIPCHK(hipStreamSynchronize(h->st));
     if (seen[2] && !h->DL) {
         const size_t n = 1 + MG_DENSE_MAX + (size_t)nb * 4;
-        CHK(dalloc(h, &h->DL, n));
-        CHK(fill_u32(h, h->DL, 0, n));
+        if (dalloc(h, &h->DL, n) == MG_OK) CHK(fill_u32(h, h->DL, 0, n));
+        else h->DL = nullptr; /* no list: such groups wait for their lanes */
     }
-    h->dense = seen[2] != 0;
+    h->dense = seen[2] != 0 && h->DL;
     if (seen[0]) return MG_OK; /* not a permutation: leave the homes as they are */
     h->rehome_due = false;
     h->steps_since_rehome = 0;

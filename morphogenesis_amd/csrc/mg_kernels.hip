@@ -1209,10 +1209,17 @@ __device__ __forceinline__ bool rs_stage(const DS& d, const MgGrid& g, Band<NX>&
     return true;
 }
 
-/* The candidates [lo, hi) (at most 64) of point pi with 0 < dsq < lim, bit k = slot lo + k */
+/* The candidates [lo, hi) (at most 64) of point pi with dsq < lim, and perhaps some just beyond:
+ * bit k = slot lo + k. Every reader of the mask tests the exact dsq again, so the test here may be
+ * cheap: the squares are summed onto -lim with fused operations, the limit widened by 1e-6 of itself
+ * (both forms of dsq lie within 4e-7 of the exact sum), and the sign is the bit. Seven VALU
+ * operations per candidate; with compares of the exact dsq it was fourteen, and the pressure of
+ * 262,144 particles took 67.5 us instead of 61.5, of the 1,014,784 of dense_listed 340 instead of
+ * 299. */
 template <class GetP>
 __device__ __forceinline__ uint64_t rs_test(uint32_t lo, uint32_t hi, f3 pi, float lim, GetP getp)
 {
+    const float far = -__builtin_fmaf(lim, 1.000001f, 1e-37f);
     uint64_t m = 0ull;
     for (uint32_t j0 = lo; j0 < hi; j0 += 4) {
         float4 pj[4];
@@ -1220,14 +1227,14 @@ __device__ __forceinline__ uint64_t rs_test(uint32_t lo, uint32_t hi, f3 pi, flo
         for (int q = 0; q < 4; q++) pj[q] = getp(j0 + (uint32_t)q);
         uint32_t nib = 0u;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 3; q >= 0; q--) {
             const f3 dist = pi - xyz(pj[q]);
-            const float dsq = dot3(dist, dist);
-            if (j0 + (uint32_t)q < hi && dsq < lim && dsq > 0.0f) nib |= 1u << q;
+            const float t = __builtin_fmaf(dist.z, dist.z, __builtin_fmaf(dist.y, dist.y, __builtin_fmaf(dist.x, dist.x, far)));
+            nib = __builtin_amdgcn_alignbit(nib, __float_as_uint(t), 31); /* nib << 1 | t < 0 */
         }
         m |= (uint64_t)nib << (j0 - lo);
     }
-    return m;
+    return hi - lo < 64u ? m & ((1ull << (hi - lo)) - 1ull) : m;
 }
 
 /* Visits the hits (0 < dsq < lim) of a staged row in ascending slots: `given` (bit k = slot
@@ -1395,6 +1402,8 @@ __device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& 
         else
             rec = rs_walk<0>(r, ~0ull, flo, fhi, pi, p.r2, tlim, [&](uint32_t j) { return d.P[j]; }, none, visit,
                              end_cell);
+        /* the point itself is no hit: left in, its bit costs every reader a visit */
+        if (s == RS_ROWS / 2 && i - r.b[0] < 64u) rec &= ~(1ull << (i - r.b[0]));
         if (d.HMW) d.HMW[(size_t)s * d.N + i] = r.b[RS_CELLS] - r.b[0] > 64u ? ~0ull : rec;
     }
     if (valid && d.ETW) rs_record_bonds<W>(d, p, i, w);
