@@ -101,19 +101,34 @@ __global__ void k_rehome_flags(const uint32_t* __restrict__ SLOT, uint32_t* __re
     unplaced[h] = s >= (uint32_t)n;
     if (s < (uint32_t)n && atomicExch(&unused[s], 0u) == 0u) stat[0] = 1u; /* set to 1 before the launch */
 }
-/* stat[2]: nonzero when a particle's row of the neighbourhood holds more than 64 candidates */
-__global__ void k_rehome_dense(DS d, MgGrid g, uint32_t* __restrict__ stat)
+/* How crowded the neighbourhoods are: stat[2], the sum over wavefronts of their particles' candidates
+ * / 64; then stat[4], the width from which a row counts as crowded (more than 64 slots, a mask's, and
+ * kDenseTimes the mean), and stat[3], the particles with such a row. */
+const uint32_t kDenseTimes = 4;
+template <bool COUNT> __global__ void k_rehome_dense(DS d, MgGrid g, uint32_t* __restrict__ stat)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t gc = i < d.ctr[MG_C_ACTIVE] ? d.GCELL[i] : MG_GRID_UNDEF;
-    if (gc == MG_GRID_UNDEF) return;
-    const uint32_t gc0 = gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, na = d.ctr[MG_C_ACTIVE];
+    const uint32_t gc = i < na ? d.GCELL[i] : MG_GRID_UNDEF;
+    const uint32_t mean = COUNT ? (uint32_t)((uint64_t)stat[2] * 64u / (RS_ROWS * max(na, 1u))) : 0u;
+    const uint32_t row = max(64u, kDenseTimes * mean);
+    uint32_t total = 0u;
     bool wide = false;
-    for (int s = 0; s < RS_ROWS; s++) {
-        const uint32_t c = gc0 + (uint32_t)g.adj[s * RS_CELLS];
-        wide |= d.OFF[c + RS_CELLS] - d.OFF[c] > 64u;
+    if (gc != MG_GRID_UNDEF) {
+        const uint32_t gc0 = gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
+        for (int s = 0; s < RS_ROWS; s++) {
+            const uint32_t c = gc0 + (uint32_t)g.adj[s * RS_CELLS], n = d.OFF[c + RS_CELLS] - d.OFF[c];
+            total += n;
+            wide |= n > row;
+        }
     }
-    if (wide) stat[2] = 1u;
+    if (COUNT) {
+        const uint64_t wides = __ballot(wide);
+        if ((threadIdx.x & 63u) == 0 && wides != 0ull) atomicAdd(&stat[3], (uint32_t)__builtin_popcountll(wides));
+        if (i == 0) stat[4] = row;
+    } else {
+        for (int o = 32; o > 0; o >>= 1) total += (uint32_t)__shfl_xor((int)total, o);
+        if ((threadIdx.x & 63u) == 0) atomicAdd(&stat[2], total / 64u);
+    }
 }
 __global__ void k_rehome_numbers(const uint32_t* __restrict__ unused, const uint32_t* __restrict__ rank,
                                  uint32_t* __restrict__ number, int n)
@@ -344,7 +359,8 @@ struct mg_handle {
     uint64_t* HM = nullptr;   /* hit masks, pressure -> force of a fused step: [row][slot] */
     int hm_rows = 0;          /* rows HM holds per slot */
     uint32_t* DL = nullptr;   /* dense groups of a fused step */
-    bool dense = false;       /* the last re-homing saw such groups: fused steps list them */
+    bool crowded = false;     /* the last re-homing saw crowded rows throughout */
+    uint32_t dense_row = 0;   /* the last re-homing saw few: fused steps list groups with wider rows */
     float4* ET = nullptr;     /* bond records, pressure -> force beside the masks: [bond slot][home] */
     /* grid */
     uint32_t *CNT[2] = {}, *OFF[2] = {};  /* gcur is current; the fused step bins into 1-gcur */
@@ -673,6 +689,7 @@ DS make_ds(mg_handle* h, int kin = 0, int conc = 0)
     d.ETW = nullptr;
     d.ETR = nullptr;
     d.DL = nullptr;
+    d.dense_row = 0;
     d.dry = 0;
     d.ctr = h->ctr;
     d.N = h->N; d.B = h->B; d.C = h->C;
@@ -849,10 +866,22 @@ int normalize(mg_handle* h)
  * incoming-bond row keeping its entries in their order, so the force gathers the same terms
  * in the same order: no result changes. */
 const int kRehomeSteps = 2048;
+/* Dense groups are listed when their particles are few: where crowding is common no group outlasts
+ * the rest, and splitting 1,024 of 4,096 groups costs more than it gives. 262,144 particles, force
+ * and diffusion with lists against a lane per particle, us: spacing 0.42 (rows of 40 on average, some
+ * beyond 64) 162 + 223 / 117 + 121; spacing 0.3 (111 on average) a step of 1,460 / 1,098. With few, see
+ * dense_listed: 1,014,784 particles 352 + 368 / 444 + 554; 4,194,304 with cells of up to 147: 1,280 +
+ * 1,728 / 1,531 + 1,839. */
+const int kDenseShare = 8;
+/* Models of more than kDiffuseRows particles whose rows hold this many candidates on average keep the
+ * one-lane pressure: 262,144 particles at rows of 111 277 us split over three wavefronts, 228 with a
+ * lane per particle (bands beyond the LDS stage: the one-lane sweep has more loads in flight); at rows
+ * of 64 137 / 156. */
+const uint32_t kCrowdedRow = 84;
 const int kDiffuseRows = 57344; /* largest model whose diffusion is split by rows, see launch_diffuse_rows */
 bool rows_of_three(const mg_handle* h, const DS& d) { return d.rows && h->g.srch == RS_CELLS; }
 
-/* Device only but for one 12-byte read: each array is scattered into the staging buffer and copied
+/* Device only but for one 20-byte read: each array is scattered into the staging buffer and copied
  * back, so no address changes and captured graphs stay valid. 64,000 particles with 32 bond slots:
  * 0.65 ms (with the permutation and the rows made on the host and every array allocated anew
  * 3.7 ms; 262,144: 9 ms), on each new state and every kRehomeSteps. */
@@ -861,7 +890,7 @@ int rehome(mg_handle* h)
     const int N = h->N, B = h->B;
     const unsigned nb = nblk(N), tiles = (unsigned)((N + SCAN_TILE - 1) / SCAN_TILE);
     const size_t row = ((size_t)N * 4 + 255) / 256 * 256;
-    const size_t words = 5 * row + (2 * (size_t)tiles + 3) * 4;
+    const size_t words = 5 * row + (2 * (size_t)tiles + 5) * 4;
     size_t most = (size_t)MG_NUM_GENES * N * 4; /* the largest array moved */
     if (B > 0) most = std::max(most, (size_t)B * N * sizeof(float4));
     most = std::max(most, std::max<size_t>(h->inc_cap, 1) * 4);
@@ -877,25 +906,33 @@ int rehome(mg_handle* h)
         hipLaunchKernelGGL(k_tile_scan, dim3(tiles), dim3(256), 0, h->st, in, out, N, excl);
     };
     CHK(fill_u32(h, unused, 1, N));
-    CHK(fill_u32(h, stat, 0, 3));
+    CHK(fill_u32(h, stat, 0, 5));
     hipLaunchKernelGGL(k_rehome_flags, dim3(nb), dim3(256), 0, h->st, h->SLOT, unused, unplaced, stat, N);
     sum(unused, rank);
     hipLaunchKernelGGL(k_rehome_numbers, dim3(nb), dim3(256), 0, h->st, unused, rank, number, N);
     sum(unplaced, rank);
     hipLaunchKernelGGL(k_rehome_sigma, dim3(nb), dim3(256), 0, h->st, h->SLOT, rank, number, sigma, stat, N);
     const DS now = make_ds(h);
-    if (N > kDiffuseRows && rows_of_three(h, now))
-        hipLaunchKernelGGL(k_rehome_dense, dim3(nb), dim3(256), 0, h->st, now, h->g, stat);
+    if (N > kDiffuseRows && rows_of_three(h, now)) {
+        hipLaunchKernelGGL(k_rehome_dense<false>, dim3(nb), dim3(256), 0, h->st, now, h->g, stat);
+        hipLaunchKernelGGL(k_rehome_dense<true>, dim3(nb), dim3(256), 0, h->st, now, h->g, stat);
+    }
     HIPCHK(hipGetLastError());
-    uint32_t seen[3] = {0, 0, 0};
-    HIPCHK(hipMemcpyAsync(seen, stat, 12, hipMemcpyDeviceToHost, h->st));
+    uint32_t seen[5] = {0, 0, 0, 0, 0};
+    HIPCHK(hipMemcpyAsync(seen, stat, sizeof(seen), hipMemcpyDeviceToHost, h->st));
     HIPCHK(hipStreamSynchronize(h->st));
-    if (seen[2] && !h->DL) {
+    const bool few = seen[3] != 0 && seen[3] <= (uint32_t)N / kDenseShare;
+    if (few && !h->DL) {
         const size_t n = 1 + MG_DENSE_MAX + (size_t)nb * 4;
         if (dalloc(h, &h->DL, n) == MG_OK) CHK(fill_u32(h, h->DL, 0, n));
         else h->DL = nullptr; /* no list: such groups wait for their lanes */
     }
-    h->dense = seen[2] != 0 && h->DL;
+    const uint32_t dense_row = few && h->DL ? seen[4] : 0u;
+    const bool crowded = seen[4] >= kDenseTimes * kCrowdedRow;
+    /* captured steps list by the old width, or not at all */
+    if (dense_row != h->dense_row || crowded != h->crowded) h->epoch++;
+    h->dense_row = dense_row;
+    h->crowded = crowded;
     if (seen[0]) return MG_OK; /* not a permutation: leave the homes as they are */
     h->rehome_due = false;
     h->steps_since_rehome = 0;
@@ -979,7 +1016,7 @@ void launch_pressure(mg_handle* h, unsigned nb, const DS& d)
     auto rows = [&](auto kernel, unsigned waves) {
         hipLaunchKernelGGL(kernel, dim3(nblk(h->N, 64)), dim3(64 * waves), 0, h->st, d, h->p, h->g);
     };
-    if (rows_of_three(h, d)) {
+    if (rows_of_three(h, d) && !(h->crowded && h->N > kPressureRows9)) {
         if (h->N <= kPressureRows9)
             return poly6 ? rows(k_pressure_rows<MG_SPH_POLY6_SPIKY, 9>, 9) : rows(k_pressure_rows<MG_SPH_REFERENCE, 9>, 9);
         return poly6 ? rows(k_pressure_rows<MG_SPH_POLY6_SPIKY, 3>, 3) : rows(k_pressure_rows<MG_SPH_REFERENCE, 3>, 3);
@@ -1269,7 +1306,7 @@ float4* bond_records(const mg_handle* h, const uint64_t* hm) { return hm ? h->ET
 uint32_t* dense_groups(const mg_handle* h, const uint64_t* hm)
 {
     const bool rows = h->grid_scanned && h->adj_rows && h->g.srch == RS_CELLS;
-    return h->dense && rows && hm && h->N > kDiffuseRows && (h->B == 0 || h->ET) ? h->DL : nullptr;
+    return h->dense_row && !h->crowded && rows && hm && h->N > kDiffuseRows && (h->B == 0 || h->ET) ? h->DL : nullptr;
 }
 
 int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nullptr)
@@ -1282,6 +1319,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
         PhaseScope ps(h, MG_PH_PRESSURE);
         DS d = make_ds(h);
         d.DL = dl;
+        d.dense_row = h->dense_row;
         d.ZERO = h->CNT[1 - h->gcur];
         d.zero_n = (uint32_t)h->C;
         d.HMW = hm;
@@ -1386,7 +1424,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
 int graph_steps(mg_handle* h, int pairs, float dt, unsigned flags, const mg_net* net = nullptr)
 {
     ensure_hit_masks(h); /* allocates (and bumps the epoch) before any capture, not inside it */
-    const int parity = (h->dense << 5) | ((h->cells_fresh && h->grid_scanned) << 4) | (h->kcur << 3) | (h->icur << 2) |
+    const int parity = ((h->cells_fresh && h->grid_scanned) << 4) | (h->kcur << 3) | (h->icur << 2) |
                        (h->ccur << 1) | h->gcur;
     const uint64_t nv = net ? net_version(net) : 0;
     if (!h->graph || h->graph_epoch != h->epoch || h->graph_dt != dt || h->graph_flags != flags ||

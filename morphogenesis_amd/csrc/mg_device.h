@@ -104,6 +104,7 @@ struct DS {
      * then per group whether it is listed. The pressure pass lists them, the force and diffusion
      * passes split them by rows, and the placement empties the list. Null when not in use. */
     uint32_t* DL;
+    uint32_t dense_row; /* a group is listed when a row holds more candidates */
     /* 1: a force pass that changes no bond record (no integrators, no breaking), for the
      * learned step's training inputs */
     int dry;

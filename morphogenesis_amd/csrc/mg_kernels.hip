@@ -1374,7 +1374,7 @@ __device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& 
     const f3 pi = valid ? xyz(d.P[i]) : mk3(0.f, 0.f, 0.f);
     const float inv_sr = pressure_inv_sr<MODE>(p), tlim = d.HMW ? fmaxf(MG_SKIN_LIM, p.r2) : p.r2;
     auto none = [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); };
-    bool wide = false; /* a row's window exceeds the 64 slots of a mask */
+    bool wide = false; /* a crowded row (dense_listed) */
     for (int q = 0; q < PER; q++) {
         const int s = (int)w * PER + q;
 #pragma unroll
@@ -1382,7 +1382,7 @@ __device__ __forceinline__ void pressure_rows_body(const DS& d, const MgParams& 
         RsRow r;
         if (q > 0) wave_lds_sync(); /* the previous row's reads are done */
         if (!rs_stage<0>(d, g, bands[w], valid, gc, s, none, r) || !valid) continue;
-        wide |= r.b[RS_CELLS] - r.b[0] > 64u;
+        wide |= r.b[RS_CELLS] - r.b[0] > d.dense_row;
         uint32_t flo, fhi, nflush = 0u;
         rs_live_range(d, g, r, s, pi, tlim, flo, fhi);
         float csum = 0.0f;
@@ -1439,10 +1439,11 @@ __global__ __launch_bounds__(64 * W, RS_OCC) void k_pressure_rows(DS d, MgParams
 
 /* Dense groups. A wavefront with one lane per particle walks its rows alone, so a few groups of 64
  * in crowded cells (drops, compressed tissue) outlast the rest of a large model's pass by the
- * length of their walk, with the chip idle. In a fused step of a model that had such groups when its
- * homes were last numbered, the pressure pass lists the groups with a row of more than 64
- * candidates (the hit masks end there too); the force and the diffusion take them nine wavefronts
- * each, in a launch of their own, and the one-lane kernels pass them by. A falling column and four
+ * length of their walk, with the chip idle. In a fused step of a model that had a few such groups when
+ * its homes were last numbered, the pressure pass lists the groups with a row of more than
+ * d.dense_row candidates (64, where the hit masks end, and four times the mean); the force and the
+ * diffusion take them nine wavefronts each, in a launch of their own, and the one-lane kernels pass
+ * them by. A falling column and four
  * drops, 1,014,784 particles: force 444 -> 276 + 85 us, diffusion and genes 554 -> 236 + 142. */
 __device__ __forceinline__ bool dense_listed(const DS& d, uint32_t bid)
 {
@@ -2397,7 +2398,7 @@ __global__ LAUNCH_BOUNDS_256 void k_insert_next(DS d, MgGrid g)
 #define RS_INSERT 4
 #define RS_LIST 48
 #define RS_AHEAD 4 /* hits a reader has in flight: with 8 most of a window's last eight are idle loads */
-#define RS_WINDOWS 4 /* of 64 slots, per row of a dense group: later ones are tested by their readers */
+#define RS_WINDOWS 8 /* of 64 slots, per row of a dense group: later ones are tested by their readers */
 struct RsLists {
     Band<0> bands[RS_ROWS];
     uint2 list[RS_LIST][64]; /* (weight, slot); NaN: recorded, not a hit */

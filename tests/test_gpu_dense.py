@@ -1,7 +1,9 @@
 """Dense groups split by rows in the fused steps of larger models (`dense_groups`) against the FP32
 oracle, bit for bit: a drop of crowded cells beside a body of ordinary spacing, above the sizes at
 which the diffusion, the force without bonds and the force with bonds go back to a lane per particle;
-more dense groups than the list holds; and a drop that is there only after the homes were numbered."""
+crowding throughout, which lists nothing and keeps the one-lane pressure; and a drop that is there
+only after the homes were numbered. (The 4,194,304-particle configuration has more dense groups than
+the list holds.)"""
 import sys
 
 import numpy as np
@@ -38,7 +40,7 @@ def with_drop(dims, b, genes, spacing, drop, seed=7):
     ((32, 32, 57), 6, True, 0, 0.5, 1000),   # 58,368: diffusion
     ((51, 51, 51), 0, False, 1, 0.5, 1000),  # 132,651: force without bonds
     ((48, 48, 65), 6, True, 0, 0.5, 3000),   # 149,760: force with bonds, diffusion
-    ((41, 42, 41), 4, True, 0, 0.26, 0),     # 70,602: every group is dense, 1,104 of them
+    ((41, 42, 41), 4, True, 0, 0.26, 0),     # 70,602: crowded throughout
 ])
 def test_dense_groups_match_oracle(built, dims, b, genes, sph, spacing, drop):
     sc = with_drop(dims, b, genes, spacing, drop)
