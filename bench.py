@@ -26,7 +26,7 @@ HBM_PEAK_GBS = 8000.0
 PHASES = ["pressure", "force", "advance", "diffusion", "genes", "insert", "scan", "place",
           "sort", "lists", "fill", "learn"]
 # kernels of the fused step (mg_step) behind each timed phase
-KERNEL_OF_PHASE = {"pressure": "k_pressure", "force": "k_force_advance",
+KERNEL_OF_PHASE = {"pressure": "k_pressure_rows", "force": "k_force_advance",
                    "diffusion": "k_diffuse_genes_insert", "scan": "k_scan_lookback",
                    "place": "k_place", "sort": "k_sort_gather",
                    "lists": "k_dense_lists", "fill": "k_fill_u32"}
