@@ -999,6 +999,7 @@ template <int NX, int CAP = BAND_CAP> constexpr size_t band_lds(unsigned threads
  * bonded tissue drifting off the cell faces; in brackets the fluid without bonds):
  *   pressure   32,768: 17.5 /  29.0 /  66.6;  46,656: 27.4 / 30.5 / 66.4;  54,872: 35.5 / 30.8 / 66.4;
  *              110,592: 55 / 40 / 68;  262,144: 112 / 68 / 92;  512,000: 237 / 142 / 183
+ *              (with the exact test of candidates; three at 262,144 take 61.5 with rs_test's)
  *   force      32,768: 15.7 / 21.6 / 45.6;  110,592: 43 / 53 / 53;  140,608: 53 / 66 / 59;
  *              175,616: 67 / 80 / 63;  262,144: 101 / 110 / 73
  *             [46,656: 25 / 21 / 41;  64,000: 32 / 22 / 42;  110,592: 50 / 37 / 41;  140,608: 63 / 48 / 47]

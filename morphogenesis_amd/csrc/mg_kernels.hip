@@ -1162,7 +1162,7 @@ __global__ LAUNCH_BOUNDS_SWEEP void k_pressure(DS d, MgParams p, MgGrid g)
  * wavefront takes three rows in turn. A row's candidates are tested into a mask first and the
  * mask's bits visited then: half the registers of the one-lane sweep (51 against 102 in the
  * pressure), so twice the wavefronts per SIMD hide each other's latency. The 512-particle tissue's
- * pressure 40 -> 12 us and force 32 -> 10 us, at 29,667 particles 63 -> 16 and 44 -> 14; the
+ * pressure 40 -> 10.5 us and force 32 -> 9 us, at 29,667 particles 63 -> 15 and 46 -> 15; the
  * host chooses W by size (launch_pressure, launch_force_advance). */
 #define RS_ROWS 9
 #define RS_CELLS 3 /* cells per row */
@@ -2390,7 +2390,7 @@ __global__ LAUNCH_BOUNDS_256 void k_insert_next(DS d, MgGrid g)
  * four wavefronts add the secretions of four TFs each, genes in order, while wavefront 8 counts
  * the epigenetic states down and stores them. Wavefront 7 bins the particle.
  *
- * 512 particles 34 -> 19 us, 29,667 46 -> 20 (a lane per particle was one serial chain: sweep,
+ * 512 particles 34 -> 17 us, 29,667 44 -> 20 (a lane per particle was one serial chain: sweep,
  * then every gene in turn); with the chip full it loses, as most wavefronts wait while few
  * work (64,000 particles 50 -> 54 us), so larger models keep a lane per particle. */
 #define RS_DIFFUSE 1
