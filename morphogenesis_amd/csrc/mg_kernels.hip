@@ -3630,8 +3630,9 @@ __global__ LAUNCH_BOUNDS_256 void k_batch_errors(const BatchInst* __restrict__ I
  *
  * Barrier: sense reversal. The last workgroup to arrive resets the arrival count and the
  * queue of the phase that just ended (every workgroup has left it), then flips `sense`; the
- * others wait for the flip with an agent-scope acquire, so the phase's writes, released by
- * every arriving workgroup, are visible to all XCDs after it. Queue 5 (the last phase) is
+ * others poll for the flip. Every workgroup releases its phase's writes at agent scope before it
+ * arrives; the last one acquires the others' before the flip releases them all, and each waiter
+ * acquires after the flip, so they are visible to all XCDs after it. Queue 5 (the last phase) is
  * reset at the first barrier of the next launch. Nothing needs clearing between launches,
  * so the launch replays from a graph as it is. A wait that exceeds its bound raises `err`
  * and gives up (the step's results are then invalid) instead of spinning forever, e.g.
@@ -3658,6 +3659,8 @@ __device__ __forceinline__ void persist_barrier(PersistCtl* ctl, unsigned& sense
         const unsigned arrived =
             __hip_atomic_fetch_add(&ctl->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
         if (arrived == gridDim.x) {
+            /* the others' arrivals, which `sense` hands on with its own */
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             __hip_atomic_store(&ctl->q[ended], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (ended == 0) __hip_atomic_store(&ctl->q[PERSIST_PHASES - 1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&ctl->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
