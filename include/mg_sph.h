@@ -179,6 +179,9 @@ int mg_step_timed(mg_handle* h, int nsteps, float dt, unsigned flags, double* ms
  * can run scans across the point where a 32-bit ticket would wrap. The value must be a
  * multiple of the scan's tile count, ceil(C / 4096), as it always is between launches. */
 int mg_debug_set_scan_ticket(mg_handle* h, uint64_t ticket);
+/* Test hook: the after-th device allocation that the library makes on the calling thread from now
+ * on fails, once, as where memory has run out (0: none). */
+int mg_debug_fail_allocation(int after);
 
 /* ---- batched instances (no counterpart in the reference, which steps one FluidSystem) ----
  * A batch steps many independent handles (each with its own buffers, grid, parameters and

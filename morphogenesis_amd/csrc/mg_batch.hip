@@ -101,7 +101,7 @@ uint64_t handle_sig(const mg_handle* h)
 template <typename T> int balloc(mg_batch* b, T** p, size_t count)
 {
     void* q = nullptr;
-    HIPCHK(hipMalloc(&q, std::max<size_t>(count * sizeof(T), 256)));
+    HIPCHK(dev_malloc(&q, std::max<size_t>(count * sizeof(T), 256)));
     b->allocs.push_back(q);
     *p = (T*)q;
     return MG_OK;

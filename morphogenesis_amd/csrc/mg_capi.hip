@@ -36,11 +36,14 @@ void set_err(const char* fmt, ...)
     g_err = buf;
 }
 
+/* A failure is reported once: hipGetLastError() keeps it until it is read, and would hand it to the
+ * launches of a route that goes on without what failed, or of the next call. */
 #define HIPCHK(x)                                                                             \
     do {                                                                                      \
         hipError_t e_ = (x);                                                                  \
         if (e_ != hipSuccess) {                                                               \
             set_err("%s failed: %s (%s:%d)", #x, hipGetErrorString(e_), __FILE__, __LINE__);  \
+            (void)hipGetLastError();                                                          \
             return MG_ERR_HIP;                                                                \
         }                                                                                     \
     } while (0)
@@ -414,11 +417,21 @@ struct mg_handle {
 
 namespace {
 
+/* mg_debug_fail_allocation: the device allocations left until one fails (0: none does) */
+thread_local int g_fail_allocation = 0;
+
+/* hipMalloc, or its failure where a test asked for one */
+hipError_t dev_malloc(void** q, size_t bytes)
+{
+    if (g_fail_allocation > 0 && --g_fail_allocation == 0) bytes = (size_t)1 << 60;
+    return hipMalloc(q, bytes);
+}
+
 template <typename T> int dalloc(mg_handle* h, T** p, size_t count)
 {
     void* q = nullptr;
     size_t bytes = std::max<size_t>(count * sizeof(T), 256);
-    HIPCHK(hipMalloc(&q, bytes));
+    HIPCHK(dev_malloc(&q, bytes));
     h->allocs.push_back(q);
     *p = (T*)q;
     return MG_OK;
@@ -1824,6 +1837,12 @@ int mg_get_grid(mg_handle* h, MgGrid* out)
     if (!h || !out) { set_err("mg_get_grid: null argument"); return MG_ERR_ARG; }
     if (!h->have_grid) { set_err("mg_get_grid: no grid set"); return MG_ERR_STATE; }
     *out = h->g;
+    return MG_OK;
+}
+
+int mg_debug_fail_allocation(int after)
+{
+    g_fail_allocation = std::max(after, 0);
     return MG_OK;
 }
 

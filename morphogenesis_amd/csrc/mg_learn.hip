@@ -47,7 +47,7 @@ namespace {
 template <typename T> int nalloc(mg_net* n, T** p, size_t count)
 {
     void* q = nullptr;
-    HIPCHK(hipMalloc(&q, std::max<size_t>(count * sizeof(T), 256)));
+    HIPCHK(dev_malloc(&q, std::max<size_t>(count * sizeof(T), 256)));
     n->allocs.push_back(q);
     *p = (T*)q;
     return MG_OK;
