@@ -105,10 +105,9 @@ int net_reserve(mg_net* n, size_t rows)
     CHK(nalloc(n, &n->ops.fz2, S * MLP_H));
     CHK(nalloc(n, &n->ops.fy, S * MLP_OUT));
     CHK(nalloc(n, &n->lpart, S / NET_ROWS));
-    if (!n->part) {
-        CHK(nalloc(n, &n->part, kNetSplits * kNParams));
-        CHK(nalloc(n, &n->bpart, 256 * NET_BIASES));
-    }
+    /* each by itself: after a failure between the two the next call allocates what is missing */
+    if (!n->part) CHK(nalloc(n, &n->part, kNetSplits * kNParams));
+    if (!n->bpart) CHK(nalloc(n, &n->bpart, 256 * NET_BIASES));
     n->cap = S;
     return MG_OK;
 }

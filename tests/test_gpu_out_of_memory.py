@@ -44,3 +44,30 @@ def test_step_without_its_optional_buffers(built, drop):
         got = run(k)
         for buf in want:
             assert_bits_equal(got[buf], want[buf], f"allocation {k} failed: {F.BUFFER_NAMES[buf]}")
+
+
+def test_training_workspace(built):
+    """Each of the training workspace's twelve allocations failing in turn, then the same gradients."""
+    from morphogenesis_amd.learned import Net
+    from tests.test_gpu_learned import identity_norm, random_data
+
+    X, T, M = random_data(300, 4)
+
+    def net():
+        n = Net(seed=3)
+        n.set_norm(*identity_norm(), 1.0)
+        n.load_data(X, T, M)
+        return n
+
+    want = net()
+    loss, g = want.grad(7, 290)
+    want.close()
+    for k in range(1, 13):
+        say("case: training workspace, allocation", k, "fails")
+        n = net()
+        n.lib.mg_debug_fail_allocation(k)
+        with pytest.raises(F.MgError):
+            n.grad(7, 290)
+        loss2, g2 = n.grad(7, 290)
+        assert loss2 == loss and np.array_equal(g, g2), k
+        n.close()
