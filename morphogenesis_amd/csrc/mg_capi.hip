@@ -362,6 +362,7 @@ struct mg_handle {
     uint64_t* HM = nullptr;   /* hit masks, pressure -> force of a fused step: [row][slot] */
     int hm_rows = 0;          /* rows HM holds per slot */
     uint32_t* DL = nullptr;   /* dense groups of a fused step */
+    bool listing = false;     /* a step lists into DL; its placement, which empties DL, is not launched yet */
     bool crowded = false;     /* the last re-homing saw crowded rows throughout */
     uint32_t dense_row = 0;   /* the last re-homing saw few: fused steps list groups with wider rows */
     float4* ET = nullptr;     /* bond records, pressure -> force beside the masks: [bond slot][home] */
@@ -1329,6 +1330,12 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
     const unsigned nb = nblk(h->N);
     uint64_t* hm = hit_masks(h);
     uint32_t* dl = dense_groups(h, hm);
+    if (dl) {
+        /* a step given up between its pressure and its placement (an error of the network's launch)
+         * leaves its list: taken on, every group of it would be advanced and binned twice */
+        if (h->listing) CHK(fill_u32(h, dl, 0, 1));
+        h->listing = true;
+    }
     {
         PhaseScope ps(h, MG_PH_PRESSURE);
         DS d = make_ds(h);
@@ -1408,6 +1415,7 @@ int do_fused_step(mg_handle* h, float dt, unsigned flags, const mg_net* net = nu
         d.OFF = d.OFFN;
         d.DL = dl;
         hipLaunchKernelGGL(k_place, dim3(nb), dim3(256), 0, h->st, d);
+        h->listing = false;
     }
     {
         PhaseScope ps(h, MG_PH_SORT);
