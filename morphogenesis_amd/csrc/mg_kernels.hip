@@ -689,9 +689,11 @@ __device__ __forceinline__ uint32_t wave_min(uint32_t v)
 __device__ __forceinline__ uint32_t wave_max(uint32_t v) { return ~wave_min(~v); }
 
 /* The candidates of one cell, slots [lo, hi), K at a time. getp(j) / getx(j, q) fetch the
- * position / extra field q of slot j; extras are fetched for the hits of a batch only. */
-template <int K, int NX, class GetP, class GetX, class Visit>
-__device__ __forceinline__ void cell_candidates(uint32_t lo, uint32_t hi, f3 pi, float lim, GetP getp,
+ * position / extra field q of slot j; extras are fetched for the hits of a batch only. REC (the
+ * sweep that records hit masks): particles at the same position are hits too, all but the slot `self`
+ * itself, since a mask's later readers may find them apart; visit tests dsq > 0. */
+template <int K, int NX, bool REC, class GetP, class GetX, class Visit>
+__device__ __forceinline__ void cell_candidates(uint32_t lo, uint32_t hi, uint32_t self, f3 pi, float lim, GetP getp,
                                                 GetX getx, Visit visit)
 {
     constexpr int NXX = NX > 0 ? NX : 1;
@@ -704,7 +706,7 @@ __device__ __forceinline__ void cell_candidates(uint32_t lo, uint32_t hi, f3 pi,
         for (int q = 0; q < K; q++) {
             const f3 dist = pi - xyz(pj[q]);
             const float dsq = dist.x * dist.x + dist.y * dist.y + dist.z * dist.z;
-            hit[q] = (j0 + (uint32_t)q < hi) && dsq < lim && dsq > 0.0f;
+            hit[q] = (j0 + (uint32_t)q < hi) && dsq < lim && (REC ? j0 + (uint32_t)q != self : dsq > 0.0f);
         }
         float4 ex[K][NXX];
 #pragma unroll
@@ -787,8 +789,8 @@ __device__ __forceinline__ void sweep(const DS& d, const MgGrid& g, Band<NX, CAP
     bool fits = band_of(0, blo, bhi);
     fetch(fits, blo, bhi);
     RowBounds nxt = row_bounds(d, g, valid ? gc0 : cmin, 0);
-    /* HM == 1: record the candidates of each row within rec_lim (>= lim) and visit those
-     * within lim (pressure); HM == 2: test only the recorded candidates (force, diffusion) */
+    /* HM == 1: record the candidates of each row within rec_lim (>= lim), all but the slot `self` of
+     * the point, and visit those within lim at a distance (pressure); HM == 2: test only the recorded candidates (force, diffusion) */
     const bool hm_w = HM == 1 && rows && d.HMW != nullptr;
     const bool hm_r = HM == 2 && rows && d.HMR != nullptr && hm_ok;
     const float tlim = hm_w ? fmaxf(rec_lim, lim) : lim; /* candidate test and culling */
@@ -928,7 +930,7 @@ __device__ __forceinline__ void sweep(const DS& d, const MgGrid& g, Band<NX, CAP
         uint64_t rec = 0ull;
         auto visit_rec = [&](uint32_t j, float4 pj, f3 dist, float dsq, const float4* x) {
             if (!wide) rec |= 1ull << ((j - wlo) & 63u);
-            if (dsq < lim) visit(j, pj, dist, dsq, x);
+            if (dsq < lim && (HM != 1 || dsq > 0.0f)) visit(j, pj, dist, dsq, x);
         };
         float gyz = 0.0f;
         if (cull) {
@@ -979,12 +981,12 @@ __device__ __forceinline__ void sweep(const DS& d, const MgGrid& g, Band<NX, CAP
                     visit_rec(j, pj, dist, dsq, x);
                 };
                 if (cfits) {
-                    cell_candidates<K, NX>(
-                        lo, hi, pi, tlim, [&](uint32_t j) { return wb.p[j - cblo]; },
+                    cell_candidates<K, NX, HM == 1>(
+                        lo, hi, self, pi, tlim, [&](uint32_t j) { return wb.p[j - cblo]; },
                         [&](uint32_t j, int x) { return wb.x[x][j - cblo]; }, visit_flat);
                 } else {
-                    cell_candidates<K, NX>(
-                        lo, hi, pi, tlim, [&](uint32_t j) { return d.P[j]; },
+                    cell_candidates<K, NX, HM == 1>(
+                        lo, hi, self, pi, tlim, [&](uint32_t j) { return d.P[j]; },
                         [&](uint32_t j, int x) { return xload(j, x); }, visit_flat);
                 }
                 end_cell();
@@ -997,12 +999,12 @@ __device__ __forceinline__ void sweep(const DS& d, const MgGrid& g, Band<NX, CAP
             if (!live_of(k)) continue;
             const uint32_t lo = rb.b[k], hi = max(rb.b[k + 1], lo);
             if (cfits) {
-                cell_candidates<K, NX>(
-                    lo, hi, pi, tlim, [&](uint32_t j) { return wb.p[j - cblo]; },
+                cell_candidates<K, NX, HM == 1>(
+                    lo, hi, self, pi, tlim, [&](uint32_t j) { return wb.p[j - cblo]; },
                     [&](uint32_t j, int x) { return wb.x[x][j - cblo]; }, visit_rec);
             } else {
-                cell_candidates<K, NX>(
-                    lo, hi, pi, tlim, [&](uint32_t j) { return d.P[j]; },
+                cell_candidates<K, NX, HM == 1>(
+                    lo, hi, self, pi, tlim, [&](uint32_t j) { return d.P[j]; },
                     [&](uint32_t j, int x) { return xload(j, x); }, visit_rec);
             }
             end_cell();
