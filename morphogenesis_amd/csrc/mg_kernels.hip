@@ -2401,11 +2401,12 @@ __global__ LAUNCH_BOUNDS_256 void k_insert_next(DS d, MgGrid g)
 #define RS_GENES 2
 #define RS_INSERT 4
 #define RS_LIST 48
+#define RS_NO_HIT 0xFFFFFFFFu /* no weight: arithmetic's own NaN is 0x7FC00000 or 0xFFC00000 */
 #define RS_AHEAD 4 /* hits a reader has in flight: with 8 most of a window's last eight are idle loads */
 #define RS_WINDOWS 8 /* of 64 slots, per row of a dense group: later ones are tested by their readers */
 struct RsLists {
     Band<0> bands[RS_ROWS];
-    uint2 list[RS_LIST][64]; /* (weight, slot); NaN: recorded, not a hit */
+    uint2 list[RS_LIST][64]; /* (weight, slot); RS_NO_HIT: recorded, not a hit */
 };
 struct RsMasks {
     uint64_t mask[RS_ROWS][RS_WINDOWS][64];
@@ -2600,8 +2601,8 @@ __device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p
                         const float4 pj = r.staged ? getp_band(j) : getp_global(j);
                         const f3 dist = pi - xyz(pj);
                         const float dsq = dot3(dist, dist);
-                        const float cc = dsq < r2 && dsq > 0.0f ? (r2 - dsq) * d2 : __builtin_nanf("");
-                        sh.a.list[k - base][lane] = make_uint2(__float_as_uint(cc), j);
+                        const float cc = (r2 - dsq) * d2;
+                        sh.a.list[k - base][lane] = make_uint2(dsq < r2 && dsq > 0.0f ? __float_as_uint(cc) : RS_NO_HIT, j);
                         k++;
                     }
                 }
@@ -2618,7 +2619,7 @@ __device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p
 #pragma unroll
                         for (int q = 0; q < 4; q++) {
                             const float cc = __uint_as_float(en[q].x);
-                            if (!(e0 + (uint32_t)q < ne && cc == cc)) continue;
+                            if (!(e0 + (uint32_t)q < ne && en[q].x != RS_NO_HIT)) continue;
                             const float c4[4] = {cn[q].x, cn[q].y, cn[q].z, cn[q].w};
                             const float u4[4] = {cur.x, cur.y, cur.z, cur.w};
 #pragma unroll
