@@ -2402,27 +2402,37 @@ __global__ LAUNCH_BOUNDS_256 void k_insert_next(DS d, MgGrid g)
 #define RS_INSERT 4
 #define RS_LIST 48
 #define RS_NO_HIT 0xFFFFFFFFu /* no weight: arithmetic's own NaN is 0x7FC00000 or 0xFFC00000 */
-#define RS_AHEAD 4 /* hits a reader has in flight: with 8 most of a window's last eight are idle loads */
-#define RS_WINDOWS 8 /* of 64 slots, per row of a dense group: later ones are tested by their readers */
+#define RS_AHEAD 3 /* hits a reader has in flight: with four and more, registers cost a third workgroup per CU */
+#define RS_CROWDED 96u /* candidates of a row from which its group is crowded, see diffuse_crowded */
+#define RS_MASKS 48 /* windows of 64 slots whose masks are in LDS at a time (crowded groups) */
+/* 96 SGPRs leave room for eight wavefronts per SIMD, so three workgroups of nine per CU find their
+ * places: with the 106 that the crowded path asks for 50,653 particles take 48.5 us instead of 39.1 */
+#define RS_DIFFUSE_BOUNDS __launch_bounds__(64 * RS_ROWS, RS_OCC) __attribute__((amdgpu_num_sgpr(96)))
 struct RsLists {
     Band<0> bands[RS_ROWS];
     uint2 list[RS_LIST][64]; /* (weight, slot); RS_NO_HIT: recorded, not a hit */
 };
 struct RsMasks {
-    uint64_t mask[RS_ROWS][RS_WINDOWS][64];
+    uint64_t mask[RS_MASKS][64];
+    uint32_t first[RS_MASKS][64];                /* the slot of a mask's bit 0 */
     uint32_t from[RS_ROWS][64], to[RS_ROWS][64]; /* the row's slots */
+    uint32_t wins[RS_ROWS];                      /* windows of the row, of the lane that has most */
 };
 
-/* Diffusion of a dense group (dense_listed): hundreds of hits per particle would pass through the
- * list a row at a time, the other wavefronts waiting. The wavefronts leave their rows' hit masks in
- * LDS instead, one test per candidate, and the wavefront of each float4 group of FCONC walks the
- * bits. Returns the sums of terms in nw, for wavefronts w < dp.ng. Bound by the scattered 16-byte
- * reads of FCONC (64 cache lines per load). Some 400 groups of ~270 hits, with the genes: 142 us
- * (through the list 344, and 278 without testing a row again each round; walking each window in
- * step 241; eight hits in flight 212). */
-__device__ __forceinline__ void diffuse_dense(const DS& d, const MgGrid& g, const DiffPlan& dp, RsMasks& sh, bool valid,
-                                              uint32_t i, uint32_t gc0, uint32_t grp, float r2, float d2, bool hm_ok,
-                                              float4 cur, float nw[4])
+/* Diffusion of a group with a crowded row (more than RS_CROWDED candidates): hundreds of hits per
+ * particle would pass through the list a few at a time, the other wavefronts waiting, and each row be
+ * tested for the count and again for the list. The wavefronts leave hit masks in LDS instead, one test
+ * per candidate, RS_MASKS windows of 64 slots at a time in row order, dealt to them in turn; then the
+ * wavefront of each float4 group of FCONC walks the bits. Returns the sums of terms in nw, for
+ * wavefronts w < dp.ng. Bound by the scattered 16-byte reads of FCONC (64 cache lines per load).
+ * Diffusion and genes, us, a lane per particle / through the list / so: 8,000 particles at rows of 64
+ * 217 / 54 / 57, of 111 312 / 124 / 101, of 282 598 / 416 / 182, of 1,093 1,499 / 2,300 / 820; 54,872 at
+ * 111 318 / 342 / 215, at 282 656 / 1,040 / 493. Listed groups (dense_listed) in a drop at rows of
+ * up to 1,093 in 262,144 particles: 1,000 with a lane per particle; with masks for the first 512 slots
+ * of a row only and the rest tested by the readers it was 2,600. */
+__device__ __forceinline__ void diffuse_crowded(const DS& d, const MgGrid& g, const DiffPlan& dp, RsMasks& sh, bool valid,
+                                                uint32_t i, uint32_t gc0, uint32_t grp, float r2, float d2, bool hm_ok,
+                                                float4 cur, float nw[4])
 {
     const uint32_t lane = threadIdx.x & 63u, N = (uint32_t)d.N;
     const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2434,73 +2444,81 @@ __device__ __forceinline__ void diffuse_dense(const DS& d, const MgGrid& g, cons
         const uint32_t c0 = gc0 + (uint32_t)g.adj[w * RS_CELLS];
         from = min(d.OFF[c0], N);
         to = max(min(d.OFF[c0 + RS_CELLS], N), from);
-        const uint64_t given = hm_ok ? d.HMR[(size_t)w * N + i] : ~0ull;
-        if (given != ~0ull) {
-            sh.mask[w][0][lane] = given; /* of a row within one window */
-        } else {
-            for (uint32_t t = 0u; t < RS_WINDOWS && from + 64u * t < to; t++)
-                sh.mask[w][t][lane] = rs_test(from + 64u * t, min(from + 64u * t + 64u, to), pi, r2, getp);
-        }
     }
     sh.from[w][lane] = from;
     sh.to[w][lane] = to;
+    const uint32_t most = wave_max((to - from + 63u) / 64u);
+    if (lane == 0) sh.wins[w] = most;
     __syncthreads();
-    if ((int)w < dp.ng && valid) {
-        const float4* C4 = (const float4*)d.CONC;
-        const float u4[4] = {cur.x, cur.y, cur.z, cur.w};
-        /* every lane goes through its own windows: in step, the busiest lane of each window would
-         * set the pace of all */
-        int s = -1;
-        uint32_t b = 0u, end = 0u, t = 0u;
-        uint64_t m = 0ull;
-        auto refill = [&]() { /* the next window with hits; m = 0: none is left */
-            while (m == 0ull) {
-                b += 64u;
-                t++;
-                while (b >= end) {
-                    if (++s == RS_ROWS) return;
-                    b = sh.from[s][lane];
-                    end = sh.to[s][lane];
-                    t = 0u;
+    uint32_t total = 0u;
+    for (int s = 0; s < RS_ROWS; s++) total += sh.wins[s];
+    /* the reader's place: window k, bits m left of the one from slot b; every lane goes through its own:
+     * in step, the busiest lane of each window would set the pace of all */
+    uint32_t k = 0u, b = 0u;
+    uint64_t m = 0ull;
+    for (uint32_t r0 = 0u; r0 < total; r0 += RS_MASKS) {
+        const uint32_t r1 = min(total, r0 + RS_MASKS);
+        for (uint32_t q = r0 + w; q < r1; q += RS_ROWS) {
+            uint32_t row = 0u, first = 0u; /* of window q */
+            while (q >= first + sh.wins[row]) first += sh.wins[row++];
+            const uint32_t lo = sh.from[row][lane] + 64u * (q - first), end = sh.to[row][lane];
+            uint64_t hits = 0ull;
+            if (lo < end) {
+                /* a recorded mask is of a row within one window */
+                const uint64_t given = hm_ok && q == first ? d.HMR[(size_t)row * N + i] : ~0ull;
+                hits = given != ~0ull ? given : rs_test(lo, min(lo + 64u, end), pi, r2, getp);
+            }
+            sh.mask[q - r0][lane] = hits;
+            sh.first[q - r0][lane] = lo;
+        }
+        __syncthreads();
+        if ((int)w < dp.ng && valid) {
+            const float4* C4 = (const float4*)d.CONC;
+            const float u4[4] = {cur.x, cur.y, cur.z, cur.w};
+            auto refill = [&]() { /* the next window with hits; m = 0: none is left in LDS */
+                while (m == 0ull && k < r1) {
+                    m = sh.mask[k - r0][lane];
+                    b = sh.first[k - r0][lane];
+                    k++;
                 }
-                m = t < RS_WINDOWS ? sh.mask[s][t][lane] : rs_test(b, min(b + 64u, end), pi, r2, getp);
-            }
-        };
-        refill();
-        while (m != 0ull) {
-            float4 pj[RS_AHEAD], cn[RS_AHEAD];
-            bool has[RS_AHEAD];
-#pragma unroll
-            for (int q = 0; q < RS_AHEAD; q++) {
-                has[q] = m != 0ull;
-                const uint32_t j = b + (has[q] ? (uint32_t)__builtin_ctzll(m) : 0u);
-                m &= m - 1ull;
-                pj[q] = d.P[j];
-                cn[q] = C4[(size_t)j * 4u + grp];
-            }
+            };
             refill();
+            while (m != 0ull) {
+                float4 pj[RS_AHEAD], cn[RS_AHEAD];
+                bool has[RS_AHEAD];
 #pragma unroll
-            for (int q = 0; q < RS_AHEAD; q++) {
-                const f3 dist = pi - xyz(pj[q]);
-                const float dsq = dot3(dist, dist);
-                if (!(has[q] && dsq < r2 && dsq > 0.0f)) continue;
-                const float cc = (r2 - dsq) * d2;
-                const float c4[4] = {cn[q].x, cn[q].y, cn[q].z, cn[q].w};
+                for (int q = 0; q < RS_AHEAD; q++) {
+                    has[q] = m != 0ull;
+                    const uint32_t j = b + (has[q] ? (uint32_t)__builtin_ctzll(m) : 0u);
+                    m &= m - 1ull;
+                    pj[q] = d.P[j];
+                    cn[q] = C4[(size_t)j * 4u + grp];
+                }
+                refill();
 #pragma unroll
-                for (int k = 0; k < 4; k++)
-                    if (dp.dm & (1u << (4u * w + (uint32_t)k))) nw[k] += dp.D[4u * w + (uint32_t)k] * cc * (c4[k] - u4[k]);
+                for (int q = 0; q < RS_AHEAD; q++) {
+                    const f3 dist = pi - xyz(pj[q]);
+                    const float dsq = dot3(dist, dist);
+                    if (!(has[q] && dsq < r2 && dsq > 0.0f)) continue;
+                    const float cc = (r2 - dsq) * d2;
+                    const float c4[4] = {cn[q].x, cn[q].y, cn[q].z, cn[q].w};
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (dp.dm & (1u << (4u * w + (uint32_t)e))) nw[e] += dp.D[4u * w + (uint32_t)e] * cc * (c4[e] - u4[e]);
+                }
             }
         }
+        __syncthreads(); /* the masks' LDS is used again */
     }
-    __syncthreads(); /* the masks' LDS is used again */
 }
 
-template <int PART, bool DENSE, class Gen>
+template <int PART, class Gen>
 __device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p, const MgGrid& g, const Gen& gen,
                                                   const DiffPlan& dp, uint32_t bid)
 {
     union Stage {
-        std::conditional_t<DENSE, RsMasks, RsLists> a;
+        RsLists a;
+        RsMasks crowd;
         struct {
             float act[MG_NUM_GENES][64];
             uint32_t depi[MG_NUM_GENES][64];
@@ -2536,45 +2554,47 @@ __device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p
         const float d2 = p.psimscale * p.psimscale, r2 = p.r2 / d2;
         const bool hm_ok = d.HMR != nullptr && d.ctr[MG_C_SKIN] == 0u && r2 == 1.0f;
         float nw[4] = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (DENSE) {
-            diffuse_dense(d, g, dp, sh.a, valid, i, gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1), grp, r2, d2, hm_ok,
-                          cur, nw);
-        } else {
-            f3 pi = mk3(0.f, 0.f, 0.f);
-            uint64_t m = 0ull;
-            if (valid) {
-                pi = xyz(d.P[i]);
-                m = hm_ok ? d.HMR[(size_t)w * N + i] : ~0ull;
-            }
-            RsRow r;
-            const bool any = dp.ng > 0 && rs_stage<0>(d, g, sh.a.bands[w], valid,
-                                                      gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1), (int)w,
-                                                      [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); }, r);
-            const bool test = m == ~0ull; /* the row's candidates have to be tested, 64 slots at a time */
-            auto getp_band = [&](uint32_t j) { return sh.a.bands[w].p[j - r.blo]; };
-            auto getp_global = [&](uint32_t j) { return d.P[j]; };
-            uint32_t n = 0u;
-            if (any && valid) {
-                if (test) {
-                    for (uint32_t b = r.b[0]; b < r.b[RS_CELLS]; b += 64u) {
-                        const uint32_t hi = min(b + 64u, r.b[RS_CELLS]);
-                        m = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
-                        n += (uint32_t)__builtin_popcountll(m);
-                    }
-                } else {
-                    n = (uint32_t)__builtin_popcountll(m);
+        const uint32_t gc0 = gc - (uint32_t)((1 * g.res[2] + 1) * g.res[0] + 1);
+        f3 pi = mk3(0.f, 0.f, 0.f);
+        uint64_t m = 0ull;
+        if (valid) {
+            pi = xyz(d.P[i]);
+            m = hm_ok ? d.HMR[(size_t)w * N + i] : ~0ull;
+        }
+        RsRow r;
+        const bool any = dp.ng > 0 && rs_stage<0>(d, g, sh.a.bands[w], valid, gc0, (int)w,
+                                                  [](uint32_t, int) { return make_float4(0.f, 0.f, 0.f, 0.f); }, r);
+        auto getp_band = [&](uint32_t j) { return sh.a.bands[w].p[j - r.blo]; };
+        auto getp_global = [&](uint32_t j) { return d.P[j]; };
+        const bool test = m == ~0ull; /* the row's candidates have to be tested, 64 slots at a time */
+        uint32_t n = 0u;
+        bool crowded = false;
+        if (any && valid) {
+            crowded = test && r.b[RS_CELLS] > r.b[0] + RS_CROWDED;
+            if (test && !crowded) {
+                for (uint32_t b = r.b[0]; b < r.b[RS_CELLS]; b += 64u) {
+                    const uint32_t hi = min(b + 64u, r.b[RS_CELLS]);
+                    m = r.staged ? rs_test(b, hi, pi, r2, getp_band) : rs_test(b, hi, pi, r2, getp_global);
+                    n += (uint32_t)__builtin_popcountll(m);
                 }
+            } else if (!crowded) {
+                n = (uint32_t)__builtin_popcountll(m);
             }
-            cnt[w][lane] = n;
-            __syncthreads();
-            uint32_t at = 0u, tot = 0u;
+        }
+        const uint32_t kCrowd = 1u << 16; /* beyond the counts of nine rows */
+        cnt[w][lane] = crowded ? kCrowd : n;
+        __syncthreads();
+        uint32_t at = 0u, tot = 0u;
 #pragma unroll
-            for (uint32_t q = 0; q < RS_ROWS; q++) {
-                const uint32_t c = cnt[q][lane];
-                if (q < w) at += c;
-                tot += c;
-            }
-            const uint32_t most = wave_max(tot);
+        for (uint32_t q = 0; q < RS_ROWS; q++) {
+            const uint32_t c = cnt[q][lane];
+            if (q < w) at += c;
+            tot += c;
+        }
+        const uint32_t most = wave_max(tot);
+        if (most >= kCrowd) {
+            diffuse_crowded(d, g, dp, sh.crowd, valid, i, gc0, grp, r2, d2, hm_ok, cur, nw);
+        } else {
             const bool adds = (int)w < dp.ng;
             /* the row's hits in turn, k the place of the next: `left` of the window from b, then the
              * windows from `next` on. A row of one window keeps the mask of the count; wider ones are
@@ -2739,18 +2759,18 @@ __device__ __forceinline__ void diffuse_rows_body(const DS& d, const MgParams& p
 }
 
 template <int PART>
-__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_rows(DS d, MgParams p, MgGrid g, MgGenome gen,
+__global__ RS_DIFFUSE_BOUNDS void k_diffuse_rows(DS d, MgParams p, MgGrid g, MgGenome gen,
                                                                        DiffPlan dp)
 {
-    diffuse_rows_body<PART, false>(d, p, g, gen, dp, xcd_block());
+    diffuse_rows_body<PART>(d, p, g, gen, dp, xcd_block());
 }
 
 /* the listed dense groups of a fused step */
-__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void k_diffuse_dense(DS d, MgParams p, MgGrid g, MgGenome gen,
+__global__ RS_DIFFUSE_BOUNDS void k_diffuse_dense(DS d, MgParams p, MgGrid g, MgGenome gen,
                                                                         DiffPlan dp)
 {
     uint32_t bid;
-    if (rows_group(d, bid)) diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT, true>(d, p, g, gen, dp, bid);
+    if (rows_group(d, bid)) diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT>(d, p, g, gen, dp, bid);
 }
 
 /* -------------------------------------------------------- bond formation
@@ -3587,12 +3607,12 @@ __global__ __launch_bounds__(64 * (RS_ROWS + 2), RS_FOCC) void kb_force_advance_
     force_advance_rows_body<MG_SPH_REFERENCE, 1, RS_ROWS>(global_view(in.force), in.p, in.g, in.dt, b - in.pb0);
 }
 
-__global__ __launch_bounds__(64 * RS_ROWS, RS_OCC) void kb_diffuse_rows(const BatchInst* __restrict__ I,
+__global__ RS_DIFFUSE_BOUNDS void kb_diffuse_rows(const BatchInst* __restrict__ I,
                                                                         const uint16_t* __restrict__ map)
 {
     const uint32_t b = xcd_block();
     const BatchInst& in = I[map[b]];
-    diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT, false>(global_view(in.diffuse), in.p, in.g, const_genome(in.gen), in.dp,
+    diffuse_rows_body<RS_DIFFUSE | RS_GENES | RS_INSERT>(global_view(in.diffuse), in.p, in.g, const_genome(in.gen), in.dp,
                                                          b - in.pb0);
 }
 
