@@ -179,6 +179,11 @@ int mg_step_timed(mg_handle* h, int nsteps, float dt, unsigned flags, double* ms
  * can run scans across the point where a 32-bit ticket would wrap. The value must be a
  * multiple of the scan's tile count, ceil(C / 4096), as it always is between launches. */
 int mg_debug_set_scan_ticket(mg_handle* h, uint64_t ticket);
+/* Test hook: how the handle's fused steps treat crowded cells since its cells were last looked at
+ * (when its homes were numbered, and every 256 steps): the candidates of a row from which a group of 64
+ * particles is dense (0: none is listed), 1 in *crowded where rows are wide throughout, and the groups
+ * that the last step listed. Any pointer may be null. */
+int mg_debug_crowding(mg_handle* h, uint32_t* dense_row, int* crowded, uint32_t* listed);
 /* Test hook: the after-th device allocation that the library makes on the calling thread from now
  * on fails, once, as where memory has run out (0: none). */
 int mg_debug_fail_allocation(int after);

@@ -363,8 +363,8 @@ struct mg_handle {
     int hm_rows = 0;          /* rows HM holds per slot */
     uint32_t* DL = nullptr;   /* dense groups of a fused step */
     bool listing = false;     /* a step lists into DL; its placement, which empties DL, is not launched yet */
-    bool crowded = false;     /* the last re-homing saw crowded rows throughout */
-    uint32_t dense_row = 0;   /* the last re-homing saw few: fused steps list groups with wider rows */
+    bool crowded = false;     /* the last look saw crowded rows throughout */
+    uint32_t dense_row = 0;   /* the last look saw few: fused steps list groups with wider rows */
     float4* ET = nullptr;     /* bond records, pressure -> force beside the masks: [bond slot][home] */
     /* grid */
     uint32_t *CNT[2] = {}, *OFF[2] = {};  /* gcur is current; the fused step bins into 1-gcur */
@@ -394,6 +394,7 @@ struct mg_handle {
      * slots) and every kRehomeSteps fused steps */
     bool rehome_due = false;
     int steps_since_rehome = 0;
+    int looked_at = 0; /* steps_since_rehome when the crowding was last looked at */
     double time = 0.0;
     std::vector<void*> allocs;
     /* phase timing (mg_step_timed) */
@@ -895,6 +896,54 @@ const uint32_t kCrowdedRow = 84;
 const int kDiffuseRows = 57344; /* largest model whose diffusion is split by rows, see launch_diffuse_rows */
 bool rows_of_three(const mg_handle* h, const DS& d) { return d.rows && h->g.srch == RS_CELLS; }
 
+/* stat[2 .. 4] of the current grid (see k_rehome_dense; cleared before), for models that choose by it */
+void count_crowding(mg_handle* h, uint32_t* stat)
+{
+    const DS now = make_ds(h);
+    if (h->N <= kDiffuseRows || !rows_of_three(h, now)) return;
+    hipLaunchKernelGGL(k_rehome_dense<false>, dim3(nblk(h->N)), dim3(256), 0, h->st, now, h->g, stat);
+    hipLaunchKernelGGL(k_rehome_dense<true>, dim3(nblk(h->N)), dim3(256), 0, h->st, now, h->g, stat);
+}
+
+/* What the counts say of the steps to come: whether they list dense groups, from which width on, and
+ * whether the pressure keeps one lane per particle. Captured steps have the choice in them: a width
+ * within a quarter of the old one is no new choice. */
+int choose_forms(mg_handle* h, const uint32_t seen[5])
+{
+    const bool few = seen[3] != 0 && seen[3] <= (uint32_t)h->N / kDenseShare;
+    if (few && !h->DL) {
+        const size_t n = 1 + MG_DENSE_MAX + (size_t)nblk(h->N) * 4;
+        if (dalloc(h, &h->DL, n) == MG_OK) CHK(fill_u32(h, h->DL, 0, n));
+        else h->DL = nullptr; /* no list: such groups wait for their lanes */
+    }
+    const uint32_t row = few && h->DL ? seen[4] : 0u, old = h->dense_row;
+    const bool crowded = seen[4] >= kDenseTimes * kCrowdedRow;
+    const bool same = row == old || (row != 0 && old != 0 && row <= old + old / 4 && old <= row + row / 4);
+    if (same && crowded == h->crowded) return MG_OK;
+    h->epoch++;
+    h->dense_row = row;
+    h->crowded = crowded;
+    return MG_OK;
+}
+
+/* The crowding alone, every kLookSteps: particles that crowd between two re-homings would step in the
+ * wrong forms for up to kRehomeSteps (262,144 particles with a drop, all crowded later: 3,980 us a step
+ * with the drop's list, 3,645 without; without a drop 1,443 and 1,371). Two kernels and a 20-byte read. */
+const int kLookSteps = 256;
+int look(mg_handle* h)
+{
+    CHK(staging(h, 256));
+    uint32_t* stat = (uint32_t*)h->staging;
+    CHK(fill_u32(h, stat, 0, 5));
+    count_crowding(h, stat);
+    HIPCHK(hipGetLastError());
+    uint32_t seen[5];
+    HIPCHK(hipMemcpyAsync(seen, stat, sizeof(seen), hipMemcpyDeviceToHost, h->st));
+    HIPCHK(hipStreamSynchronize(h->st));
+    h->looked_at = h->steps_since_rehome;
+    return choose_forms(h, seen);
+}
+
 /* Device only but for one 20-byte read: each array is scattered into the staging buffer and copied
  * back, so no address changes and captured graphs stay valid. 64,000 particles with 32 bond slots:
  * 0.65 ms (with the permutation and the rows made on the host and every array allocated anew
@@ -926,30 +975,16 @@ int rehome(mg_handle* h)
     hipLaunchKernelGGL(k_rehome_numbers, dim3(nb), dim3(256), 0, h->st, unused, rank, number, N);
     sum(unplaced, rank);
     hipLaunchKernelGGL(k_rehome_sigma, dim3(nb), dim3(256), 0, h->st, h->SLOT, rank, number, sigma, stat, N);
-    const DS now = make_ds(h);
-    if (N > kDiffuseRows && rows_of_three(h, now)) {
-        hipLaunchKernelGGL(k_rehome_dense<false>, dim3(nb), dim3(256), 0, h->st, now, h->g, stat);
-        hipLaunchKernelGGL(k_rehome_dense<true>, dim3(nb), dim3(256), 0, h->st, now, h->g, stat);
-    }
+    count_crowding(h, stat);
     HIPCHK(hipGetLastError());
     uint32_t seen[5] = {0, 0, 0, 0, 0};
     HIPCHK(hipMemcpyAsync(seen, stat, sizeof(seen), hipMemcpyDeviceToHost, h->st));
     HIPCHK(hipStreamSynchronize(h->st));
-    const bool few = seen[3] != 0 && seen[3] <= (uint32_t)N / kDenseShare;
-    if (few && !h->DL) {
-        const size_t n = 1 + MG_DENSE_MAX + (size_t)nb * 4;
-        if (dalloc(h, &h->DL, n) == MG_OK) CHK(fill_u32(h, h->DL, 0, n));
-        else h->DL = nullptr; /* no list: such groups wait for their lanes */
-    }
-    const uint32_t dense_row = few && h->DL ? seen[4] : 0u;
-    const bool crowded = seen[4] >= kDenseTimes * kCrowdedRow;
-    /* captured steps list by the old width, or not at all */
-    if (dense_row != h->dense_row || crowded != h->crowded) h->epoch++;
-    h->dense_row = dense_row;
-    h->crowded = crowded;
+    CHK(choose_forms(h, seen));
     if (seen[0]) return MG_OK; /* not a permutation: leave the homes as they are */
     h->rehome_due = false;
     h->steps_since_rehome = 0;
+    h->looked_at = 0;
     if (!seen[1]) return MG_OK;
     void* tmp = h->staging;
     auto back = [&](void* field, size_t bytes) -> int {
@@ -998,7 +1033,10 @@ int rehome(mg_handle* h)
 
 int maybe_rehome(mg_handle* h)
 {
-    if (h->force_zero && (h->rehome_due || h->steps_since_rehome >= kRehomeSteps)) return rehome(h);
+    if (!h->force_zero) return MG_OK;
+    if (h->rehome_due || h->steps_since_rehome >= kRehomeSteps) return rehome(h);
+    /* (a batch steps its own forms) */
+    if (h->N > kDiffuseRows && !h->batch && h->steps_since_rehome - h->looked_at >= kLookSteps) return look(h);
     return MG_OK;
 }
 
@@ -1851,6 +1889,21 @@ int mg_get_grid(mg_handle* h, MgGrid* out)
 int mg_debug_fail_allocation(int after)
 {
     g_fail_allocation = std::max(after, 0);
+    return MG_OK;
+}
+
+int mg_debug_crowding(mg_handle* h, uint32_t* dense_row, int* crowded, uint32_t* listed)
+{
+    CHK(ready(h));
+    if (dense_row) *dense_row = h->dense_row;
+    if (crowded) *crowded = h->crowded;
+    if (!listed) return MG_OK;
+    *listed = 0;
+    if (!dense_groups(h, hit_masks(h))) return MG_OK;
+    std::vector<uint32_t> flag((size_t)nblk(h->N, 64));
+    HIPCHK(hipMemcpyAsync(flag.data(), h->DL + 1 + MG_DENSE_MAX, flag.size() * 4, hipMemcpyDeviceToHost, h->st));
+    HIPCHK(hipStreamSynchronize(h->st));
+    for (uint32_t f : flag) *listed += f != 0;
     return MG_OK;
 }
 
