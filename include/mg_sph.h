@@ -184,6 +184,9 @@ int mg_debug_set_scan_ticket(mg_handle* h, uint64_t ticket);
  * particles is dense (0: none is listed), 1 in *crowded where rows are wide throughout, and the groups
  * that the last step listed. Any pointer may be null. */
 int mg_debug_crowding(mg_handle* h, uint32_t* dense_row, int* crowded, uint32_t* listed);
+/* Test hook: how many uploads and downloads of the process went through the library's pinned memory
+ * (large ones from or to ordinary, pageable memory). */
+int mg_debug_bounced_copies(uint64_t* count);
 /* Test hook: the after-th device allocation that the library makes on the calling thread from now
  * on fails, once, as where memory has run out (0: none). */
 int mg_debug_fail_allocation(int after);

@@ -234,6 +234,7 @@ def declare(lib, prefix: str):
         sig["debug_set_scan_ticket"] = [h, C.c_uint64]
         sig["debug_fail_allocation"] = [C.c_int]
         sig["debug_crowding"] = [h, P(C.c_uint32), P(C.c_int), P(C.c_uint32)]
+        sig["debug_bounced_copies"] = [P(C.c_uint64)]
         fl3 = P(C.c_float)
         sig["derive_params"] = [P(MgParams)] + [C.c_float] * 5 + [fl3, fl3] + [C.c_float] * 16
         sig["derive_grid"] = [P(MgGrid), fl3, fl3, C.c_float, C.c_float, C.c_float]
