@@ -232,6 +232,13 @@ int mg_batch_set_tile_shape(mg_batch* b, int cls, int cand_batch, int band_cap);
 /* The launch form in use: *persistent = 1 for one persistent launch per step (with
  * *workgroups workgroups of 256 threads), 0 for a form of launches per phase. Either may be null. */
 int mg_batch_launch_config(mg_batch* b, int* persistent, unsigned* workgroups);
+/* The form of the next step: one launch per phase and size class, one persistent launch, or one
+ * launch per phase over every instance. */
+enum { MG_BATCH_BY_SIZE = -1, MG_BATCH_DISPATCH = 0, MG_BATCH_PERSISTENT = 1, MG_BATCH_MERGED = 2 };
+int mg_batch_form(mg_batch* b, int* form);
+/* Chooses it (at the block sizes, tile shapes and workgroups per CU in use); MG_BATCH_BY_SIZE: the
+ * default, by the batch's particles. Every form gives the same bits. */
+int mg_batch_set_form(mg_batch* b, int form);
 /* Chooses the form: on = 1 persistent (workgroups_per_cu workgroups on each CU, 0 = all that
  * stay resident; batches whose instances exceed 65,535 blocks of 256 use the dispatch form),
  * on = 0 the dispatch form. */

@@ -249,6 +249,8 @@ def declare(lib, prefix: str):
         sig["batch_class_config"] = [h, C.c_int, P(C.c_int), P(C.c_uint), P(C.c_int), P(C.c_int)]
         sig["batch_set_tile_shape"] = [h, C.c_int, C.c_int, C.c_int]
         sig["batch_set_persistent"] = [h, C.c_int, C.c_uint]
+        sig["batch_form"] = [h, P(C.c_int)]
+        sig["batch_set_form"] = [h, C.c_int]
     else:
         sig["create"] = [P(h), C.c_int, C.c_int, C.c_int]
         sig["insert_particles"] = [h]

@@ -6,6 +6,8 @@ import ctypes as C
 
 from morphogenesis_amd import _ffi as F
 
+FORMS = ("dispatch", "persistent", "merged")  # MG_BATCH_*
+
 
 class Batch:
     """Steps the given FluidSystem objects together. While the batch exists their work runs on
@@ -63,13 +65,24 @@ class Batch:
 
     def launch_config(self):
         """(persistent, workgroups): 1 and the workgroup count for one persistent launch per
-        step, 0 for the dispatch form."""
+        step, 0 for a form of launches per phase (form() says which)."""
         on, wg = C.c_int(), C.c_uint()
         self._call("batch_launch_config", self.h, C.byref(on), C.byref(wg))
         return int(on.value), int(wg.value)
 
     def set_persistent(self, on: bool, workgroups_per_cu: int = 0):
         self._call("batch_set_persistent", self.h, int(bool(on)), int(workgroups_per_cu))
+
+    def form(self):
+        """The form of the next step: "merged" (one launch per phase over every instance),
+        "persistent" (one launch per step) or "dispatch" (one launch per phase and size class)."""
+        f = C.c_int()
+        self._call("batch_form", self.h, C.byref(f))
+        return FORMS[f.value]
+
+    def set_form(self, form: str):
+        """Chooses the form; "by size": the default, by the batch's particles."""
+        self._call("batch_set_form", self.h, -1 if form == "by size" else FORMS.index(form))
 
     def close(self):
         if self.h:

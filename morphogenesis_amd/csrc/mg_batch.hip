@@ -297,12 +297,15 @@ int persist_launch(mg_batch* b, int q)
  * mg_batch_autotune decides. */
 const size_t kBatchMerged = 1u << 22;
 
+bool merged_wanted(const mg_batch* b)
+{
+    return b->merged_mode > 0 || (b->merged_mode < 0 && b->merged_n <= kBatchMerged);
+}
+
 int merged_build(mg_batch* b, float dt, unsigned flags)
 {
     const int n = (int)b->hs.size();
-    b->merged_n = 0;
-    for (const mg_handle* h : b->hs) b->merged_n += (size_t)h->N;
-    if (b->merged_mode == 0 || (b->merged_mode < 0 && b->merged_n > kBatchMerged)) return MG_OK;
+    if (!merged_wanted(b)) return MG_OK;
     std::vector<int> order(n);
     for (int i = 0; i < n; i++) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return b->hs[x]->N > b->hs[y]->N; });
@@ -655,6 +658,7 @@ int mg_batch_create(mg_batch** out, mg_handle* const* handles, int n)
         return MG_ERR_HIP;
     }
     b->hs.assign(handles, handles + n);
+    for (const mg_handle* h : b->hs) b->merged_n += (size_t)h->N;
     b->cls.resize(kBatchClasses);
     std::vector<int> order(n);
     for (int i = 0; i < n; i++) order[i] = i;
@@ -753,6 +757,14 @@ int mg_batch_classes(mg_batch* b, int* nclass, int* members, unsigned* threads)
     return MG_OK;
 }
 
+/* merged_mode from now on: the next step builds its tables, and until then none are in use */
+static void batch_merge(mg_batch* b, int merged_mode)
+{
+    b->merged_mode = merged_mode;
+    b->merged = false;
+    b->built = false;
+}
+
 /* `steps` dispatch-form steps with HIP events per launch group; ms[class] accumulates the
  * milliseconds of the launches of phase `ph` (every phase when ph < 0) */
 static int batch_time_classes(mg_batch* b, int steps, float dt, unsigned flags, int ph,
@@ -775,10 +787,9 @@ static int batch_time_classes(mg_batch* b, int steps, float dt, unsigned flags, 
     return MG_OK;
 }
 
-int mg_batch_autotune(mg_batch* b, int steps, float dt, unsigned flags, unsigned* threads_out)
+static int batch_autotune(mg_batch* b, int steps, float dt, unsigned flags, unsigned* threads_out)
 {
-    if (!b || steps < 1) { set_err("mg_batch_autotune: bad arguments"); return MG_ERR_ARG; }
-    b->merged_mode = 0;
+    batch_merge(b, 0);
     const unsigned cand[] = {256, 128, 64};
     const int nc = (int)b->cls.size();
     std::vector<double> best(nc, 1e300), ms;
@@ -853,18 +864,29 @@ int mg_batch_autotune(mg_batch* b, int steps, float dt, unsigned flags, unsigned
     b->persist_use_per_cu = best_per_cu;
     if (r == MG_OK) {
         /* the merged form, its tables built by two steps outside the timed ones */
-        b->merged_mode = 1;
-        b->built = false;
+        batch_merge(b, 1);
         double ms = 0.0;
         r = batch_steps(b, 2, dt, flags, false);
         if (r == MG_OK) r = time_steps(&ms);
-        if (r != MG_OK || ms >= best_ms) {
-            b->merged_mode = 0;
-            b->built = false;
-        }
+        if (r != MG_OK || ms >= best_ms) batch_merge(b, 0);
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
+    return r;
+}
+
+int mg_batch_autotune(mg_batch* b, int steps, float dt, unsigned flags, unsigned* threads_out)
+{
+    if (!b || steps < 1) { set_err("mg_batch_autotune: bad arguments"); return MG_ERR_ARG; }
+    const int merged_mode = b->merged_mode;
+    const bool persistent = b->persistent;
+    const unsigned per_cu = b->persist_use_per_cu;
+    const int r = batch_autotune(b, steps, dt, flags, threads_out);
+    if (r != MG_OK) { /* the form stays what it was */
+        b->persistent = persistent;
+        b->persist_use_per_cu = per_cu;
+        batch_merge(b, merged_mode);
+    }
     return r;
 }
 
@@ -900,6 +922,27 @@ int mg_batch_launch_config(mg_batch* b, int* persistent, unsigned* workgroups)
     const bool on = b->persistent && b->persist_ok && !b->merged;
     if (persistent) *persistent = on ? 1 : 0;
     if (workgroups) *workgroups = on ? persist_workgroups(b) : 0u;
+    return MG_OK;
+}
+
+int mg_batch_form(mg_batch* b, int* form)
+{
+    if (!b || !form) return MG_ERR_ARG;
+    const bool merged = b->built ? b->merged : merged_wanted(b);
+    *form = merged ? MG_BATCH_MERGED
+            : b->persistent && (b->persist_ok || !b->built) ? MG_BATCH_PERSISTENT : MG_BATCH_DISPATCH;
+    return MG_OK;
+}
+
+int mg_batch_set_form(mg_batch* b, int form)
+{
+    if (!b || form < MG_BATCH_BY_SIZE || form > MG_BATCH_MERGED) {
+        set_err("mg_batch_set_form: no such form");
+        return MG_ERR_ARG;
+    }
+    CHK(mg_batch_set_persistent(b, form != MG_BATCH_DISPATCH, b->persist_use_per_cu));
+    if (form == MG_BATCH_MERGED) batch_merge(b, 1);
+    if (form == MG_BATCH_BY_SIZE) batch_merge(b, -1);
     return MG_OK;
 }
 
