@@ -206,6 +206,33 @@ def cpu_baseline(scene, budget_s: float = 15.0) -> dict:
                       f"{el:.1f} s, FP32 oracle (CPU restatement), {threads} threads on {model}"}
 
 
+BATCH_STEP = {"merged": "one launch per phase over every instance",
+              "persistent": "one persistent launch per step for all instances",
+              "dispatch": "one launch per phase and size class"}
+
+
+def time_other_forms(bat, steps: int, dt: float, flags: int, form: str, ms: float) -> dict:
+    """ms per step of every launch form of the batch: `ms` for `form`, in use; the others over
+    `steps` graph-replayed steps each, after which `form` is in use again."""
+    from morphogenesis_amd import _ffi as F
+
+    out = {form: ms}
+    for other in BATCH_STEP:
+        if other == form:
+            continue
+        bat.set_form(other)
+        bat.step(2, dt, flags | F.STEP_GRAPH)
+        bat.sync()
+        if bat.form() != other:  # instances too large for the persistent launch
+            continue
+        t = time.perf_counter()
+        bat.step(steps, dt, flags | F.STEP_GRAPH)
+        bat.sync()
+        out[other] = (time.perf_counter() - t) / steps * 1e3
+    bat.set_form(form)
+    return out
+
+
 def run_batch(args, count: int = 256):
     """The batched workload: `count` bonded tissue blocks of log-uniform size in
     [2048, 65536] particles, each with its own domain, grid and genome, stepped together."""
@@ -231,28 +258,18 @@ def run_batch(args, count: int = 256):
     bat = Batch(systems)
     chosen = bat.autotune(2, dt, flags)
     if args.batch_form != "auto":
-        bat.set_persistent(args.batch_form == "persistent")
+        bat.set_form(args.batch_form)
+    form = bat.form()
     persistent, workgroups = bat.launch_config()
-    progress(f"autotuned: block sizes {chosen}, persistent launch {persistent} ({workgroups} workgroups)")
+    progress(f"autotuned: block sizes {chosen}, form {form} ({workgroups} workgroups)")
     bat.step(args.warmup, dt, flags | F.STEP_GRAPH)
     bat.sync()
     t0 = time.perf_counter()
     bat.step(args.steps, dt, flags | F.STEP_GRAPH)
     bat.sync()
     elapsed = time.perf_counter() - t0
-    # the other launch form over the same number of steps, for comparison (not the value)
-    forms = {("persistent" if persistent else "dispatch"): elapsed / args.steps * 1e3}
-    if persistent or bat.launch_config()[0] == 0:
-        bat.set_persistent(not persistent)
-        other = bat.launch_config()[0]
-        if other != persistent:
-            bat.step(2, dt, flags | F.STEP_GRAPH)
-            bat.sync()
-            t1 = time.perf_counter()
-            bat.step(args.steps, dt, flags | F.STEP_GRAPH)
-            bat.sync()
-            forms["persistent" if other else "dispatch"] = (time.perf_counter() - t1) / args.steps * 1e3
-        bat.set_persistent(bool(persistent))
+    # the other forms over the same number of steps, for comparison (not the value)
+    forms = time_other_forms(bat, args.steps, dt, flags, form, elapsed / args.steps * 1e3)
     ms = (C.c_double * len(PHASES))()
     calls = (C.c_int * len(PHASES))()
     bat._call("batch_step_timed", bat.h, args.timed_steps, dt, flags, ms, calls)
@@ -286,13 +303,12 @@ def run_batch(args, count: int = 256):
         "config": {"workload": args.workload, "instances": count, "particles": total,
                    "bonds_per_particle": 32, "dt": dt, "genes": bool(flags & F.STEP_GENES),
                    "hipgraph": True,
-                   "launch": {"persistent": bool(persistent), "workgroups": workgroups,
+                   "launch": {"form": form, "persistent": bool(persistent), "workgroups": workgroups,
                               "ms_per_step_by_form": {k: round(v, 4) for k, v in forms.items()}},
                    "size_classes": bat.class_config(),
                    "autotuned_threads": chosen,
                    "step": ("pressure+force+advance+diffusion+genes+insert+scan+sort, "
-                            + ("one persistent launch per step for all instances" if persistent
-                               else "one launch per phase and size class"))},
+                            + BATCH_STEP[form])},
         "roofline": {"bound": "hbm", "kernel": kern[dom], "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": load_traffic(kern[dom], args.workload),
@@ -300,7 +316,8 @@ def run_batch(args, count: int = 256):
                      "algorithmic_basis": "reference layout, per particle: " +
                                           ", ".join(f"{k} {v:.1f} B" for k, v in terms.items()),
                      "avg_launch_ms": per_step[dom],
-                     "timing": "per-phase times of the dispatch form (HIP events around each launch group)",
+                     "timing": "per-phase times of the dispatch form (HIP events around each launch group)"
+                               + ("" if form == "dispatch" else f"; the value is the {form} form's"),
                      "layout": {"bytes_per_launch": lay, "achieved": lay_ach, "frac": lay_ach / HBM_PEAK_GBS,
                                 "basis": "this build's HBM layout, every element once"}},
         "step_breakdown_ms": {p: round(v, 5) for p, v in per_step.items()},
@@ -581,7 +598,7 @@ def main():
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--timed-steps", type=int, default=20)
     ap.add_argument("--no-graph", action="store_true", help="launch the step kernels eagerly")
-    ap.add_argument("--batch-form", choices=("auto", "persistent", "dispatch"), default="auto",
+    ap.add_argument("--batch-form", choices=("auto", "merged", "persistent", "dispatch"), default="auto",
                     help="tissue_batch_256: the launch form (auto: the autotuner's choice)")
     ap.add_argument("--no-config-run", action="store_true",
                     help="leave out the timing of the configuration's whole run")
