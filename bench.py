@@ -25,11 +25,22 @@ METRIC = ("particle-steps/sec + % HBM peak, 262k bonded tissue; learned 4×dt vs
 HBM_PEAK_GBS = 8000.0
 PHASES = ["pressure", "force", "advance", "diffusion", "genes", "insert", "scan", "place",
           "sort", "lists", "fill", "learn"]
-# kernels of the fused step (mg_step) behind each timed phase
-KERNEL_OF_PHASE = {"pressure": "k_pressure_rows", "force": "k_force_advance",
-                   "diffusion": "k_diffuse_genes_insert", "scan": "k_scan_lookback",
-                   "place": "k_place", "sort": "k_sort_gather",
-                   "lists": "k_dense_lists", "fill": "k_fill_u32"}
+
+
+def kernels_of_phase(scene, crowded: bool = False) -> dict:
+    """The kernel of the fused step (mg_step) behind each timed phase of this scene: which sweeps are
+    split by rows follows the library's sizes (launch_pressure, launch_force_advance, do_fused_step);
+    `crowded` as mg_debug_crowding tells it. A model with
+    bonds splits its force only with bond records (cut-off 1)."""
+    rows = int(scene.grid.srch) == 3
+    force_rows = rows and (scene.n <= 147456 and float(scene.params.r2) == 1.0 if scene.b else scene.n <= 131072)
+    genes = bool(scene.flags & 1)
+    return {"pressure": "k_pressure_rows" if rows and not (crowded and scene.n > 49152) else "k_pressure",
+            "force": "k_force_advance_rows" if force_rows else "k_force_advance",
+            "diffusion": "k_insert_next" if not genes else "k_diffuse_rows" if rows and scene.n <= 57344
+            else "k_diffuse_genes_insert",
+            "scan": "k_scan_lookback", "place": "k_place", "sort": "k_sort_gather", "lists": "k_dense_lists",
+            "fill": "k_fill_u32"}
 
 
 def bond_records_in_use(scene) -> bool:
@@ -421,7 +432,7 @@ def run_learned(args):
     print(json.dumps(out))
 
 
-def roofline(dom: str, scene, stats: dict, dom_ms: float, workload: str) -> dict:
+def roofline(dom: str, scene, stats: dict, dom_ms: float, workload: str, crowded: bool = False) -> dict:
     """The dominant kernel against HBM bandwidth. `achieved` counts the compulsory bytes of
     the reference's layout for the work the kernel does (reference_layout_bytes, terms
     listed); `layout` counts the compulsory bytes of this build's own layout
@@ -431,9 +442,10 @@ def roofline(dom: str, scene, stats: dict, dom_ms: float, workload: str) -> dict
     lay = algorithmic_bytes(dom, scene, stats)
     ach = ref_bytes / (dom_ms * 1e-3) / 1e9
     lay_ach = lay / (dom_ms * 1e-3) / 1e9
-    return {"bound": "hbm", "kernel": KERNEL_OF_PHASE[dom], "achieved": ach, "peak": HBM_PEAK_GBS,
+    kernel = kernels_of_phase(scene, crowded)[dom]
+    return {"bound": "hbm", "kernel": kernel, "achieved": ach, "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
-            "traffic": load_traffic(KERNEL_OF_PHASE[dom], workload),
+            "traffic": load_traffic(kernel, workload),
             "algorithmic_bytes_per_launch": ref_bytes,
             "algorithmic_basis": "reference layout, per particle: " +
                                  ", ".join(f"{k} {v:.1f} B" for k, v in terms.items()),
@@ -678,19 +690,22 @@ def main():
     if r != 0:
         raise F.MgError(sim.last_error())
     per_step = {ph: ms[i] / args.timed_steps for i, ph in enumerate(PHASES) if calls[i]}
-    dom = max((p for p in per_step if p in KERNEL_OF_PHASE and p not in ("fill", "place")),
+    crowded = C.c_int()
+    lib.mg_debug_crowding(sim.h, None, C.byref(crowded), None)
+    names = kernels_of_phase(scene, bool(crowded.value))
+    dom = max((p for p in per_step if p in names and p not in ("fill", "place")),
               key=lambda p: per_step[p])
     dom_ms = per_step[dom]  # one launch per step
     breakdown = {p: round(v, 5) for p, v in per_step.items()}
     kernels = {}
     for p, v in per_step.items():
-        if p in KERNEL_OF_PHASE and algorithmic_bytes(p, scene, stats) > 0:
+        if p in names and algorithmic_bytes(p, scene, stats) > 0:
             bts = algorithmic_bytes(p, scene, stats)
             rb, _ = reference_layout_bytes(p, scene, stats)
-            kernels[KERNEL_OF_PHASE[p]] = {"ms": round(v, 5), "alg_bytes": int(bts),
-                                           "GB/s": round(bts / (v * 1e-3) / 1e9, 1)}
+            kernels[names[p]] = {"ms": round(v, 5), "alg_bytes": int(bts),
+                                 "GB/s": round(bts / (v * 1e-3) / 1e9, 1)}
             if rb:
-                kernels[KERNEL_OF_PHASE[p]]["ref_layout_GB/s"] = round(rb / (v * 1e-3) / 1e9, 1)
+                kernels[names[p]]["ref_layout_GB/s"] = round(rb / (v * 1e-3) / 1e9, 1)
     ms_per_step = elapsed / args.steps * 1e3
     value = scene.n * args.steps / elapsed
     out = {
@@ -711,7 +726,7 @@ def main():
                    "cells": scene.c, "dt": scene.dt, "genes": bool(scene.flags & F.STEP_GENES),
                    "hipgraph": not args.no_graph,
                    "step": "pressure+force+advance+diffusion+genes+insert+scan+sort"},
-        "roofline": roofline(dom, scene, stats, dom_ms, args.workload),
+        "roofline": roofline(dom, scene, stats, dom_ms, args.workload, bool(crowded.value)),
         "step_breakdown_ms": breakdown,
         "kernels": kernels,
         "mean_neighbours": round(stats["neighbours"], 2),
