@@ -50,3 +50,22 @@ def test_pinned_buffers_are_not_copied_twice(built, n, offset):
     finally:
         sim.close()
         hip.hipHostFree(p)
+
+
+def test_threads_each_with_a_handle(built):
+    """Large copies of several handles from several threads at once; a thread's failure is the test's."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    def work(k):
+        rng = np.random.default_rng(k)
+        sim = system(263000 + 777 * k)
+        for _ in range(4):
+            conc = words(rng, (sim.n, F.NUM_TF), np.float32)
+            sim.upload(F.FCONC, conc)
+            assert np.array_equal(sim.download(F.FCONC).view(np.uint32), conc.view(np.uint32)), k
+        sim.close()
+        return k
+
+    print("case: five threads, a handle each", flush=True)
+    with ThreadPoolExecutor(5) as pool:
+        assert [f.result() for f in [pool.submit(work, k) for k in range(5)]] == list(range(5))
