@@ -30,12 +30,12 @@ PHASES = ["pressure", "force", "advance", "diffusion", "genes", "insert", "scan"
 def kernels_of_phase(scene, crowded: bool = False) -> dict:
     """The kernel of the fused step (mg_step) behind each timed phase of this scene: which sweeps are
     split by rows follows the library's sizes (launch_pressure, launch_force_advance, do_fused_step);
-    `crowded` as mg_debug_crowding tells it. A model with
-    bonds splits its force only with bond records (cut-off 1)."""
+    `crowded` as mg_debug_crowding tells it. A model with bonds splits its force only with bond
+    records (cut-off 1)."""
     rows = int(scene.grid.srch) == 3
     force_rows = rows and (scene.n <= 147456 and float(scene.params.r2) == 1.0 if scene.b else scene.n <= 131072)
     genes = bool(scene.flags & 1)
-    return {"pressure": "k_pressure_rows" if rows and not (crowded and scene.n > 49152) else "k_pressure",
+    return {"pressure": "k_pressure_rows" if rows and not crowded else "k_pressure",
             "force": "k_force_advance_rows" if force_rows else "k_force_advance",
             "diffusion": "k_insert_next" if not genes else "k_diffuse_rows" if rows and scene.n <= 57344
             else "k_diffuse_genes_insert",

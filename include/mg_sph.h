@@ -181,8 +181,8 @@ int mg_step_timed(mg_handle* h, int nsteps, float dt, unsigned flags, double* ms
 int mg_debug_set_scan_ticket(mg_handle* h, uint64_t ticket);
 /* Test hook: how the handle's fused steps treat crowded cells since its cells were last looked at
  * (when its homes were numbered, and every 256 steps): the candidates of a row from which a group of 64
- * particles is dense (0: none is listed), 1 in *crowded where rows are wide throughout, and the groups
- * that the last step listed. Any pointer may be null. */
+ * particles is dense (0: none is listed), 1 in *crowded where rows are wide throughout and the pressure
+ * keeps a lane per particle, and the groups that the last step listed. Any pointer may be null. */
 int mg_debug_crowding(mg_handle* h, uint32_t* dense_row, int* crowded, uint32_t* listed);
 /* Test hook: how many uploads and downloads of the process went through the library's pinned memory
  * (large ones from or to ordinary, pageable memory). */

@@ -363,7 +363,7 @@ struct mg_handle {
     int hm_rows = 0;          /* rows HM holds per slot */
     uint32_t* DL = nullptr;   /* dense groups of a fused step */
     bool listing = false;     /* a step lists into DL; its placement, which empties DL, is not launched yet */
-    bool crowded = false;     /* the last look saw crowded rows throughout */
+    bool crowded = false;     /* the last look saw crowded rows throughout: the pressure keeps its lanes */
     uint32_t dense_row = 0;   /* the last look saw few: fused steps list groups with wider rows */
     float4* ET = nullptr;     /* bond records, pressure -> force beside the masks: [bond slot][home] */
     /* grid */
@@ -905,10 +905,13 @@ const int kRehomeSteps = 2048;
  * dense_listed: 1,014,784 particles 352 + 368 / 444 + 554; 4,194,304 with cells of up to 147: 1,280 +
  * 1,728 / 1,531 + 1,839. */
 const int kDenseShare = 8;
-/* Models of more than kDiffuseRows particles whose rows hold this many candidates on average keep the
- * one-lane pressure: 262,144 particles at rows of 111 277 us split over three wavefronts, 228 with a
- * lane per particle (bands beyond the LDS stage: the one-lane sweep has more loads in flight); at rows
- * of 64 137 / 156. */
+/* Models of more than kPressureCrowded particles whose rows hold this many candidates on average keep the
+ * one-lane pressure (bands beyond the LDS stage: the one-lane sweep has more loads in flight). us, split
+ * over three wavefronts / with a lane per particle: 262,144 particles at rows of 64 137 / 156, of 111
+ * 262 / 224, of 282 637 / 529; 198,476 at 111 237 / 234, at 282 535 / 515; 175,560 216 / 210 and
+ * 482 / 450; 146,016, which leave the lanes less to overlap, 165 / 194 and 382 / 442; 60,840 122 / 179 and
+ * 269 / 399. */
+const int kPressureCrowded = 163840;
 const uint32_t kCrowdedRow = 84;
 const int kDiffuseRows = 57344; /* largest model whose diffusion is split by rows, see launch_diffuse_rows */
 bool rows_of_three(const mg_handle* h, const DS& d) { return d.rows && h->g.srch == RS_CELLS; }
@@ -934,7 +937,7 @@ int choose_forms(mg_handle* h, const uint32_t seen[5])
         else h->DL = nullptr; /* no list: such groups wait for their lanes */
     }
     const uint32_t row = few && h->DL ? seen[4] : 0u, old = h->dense_row;
-    const bool crowded = seen[4] >= kDenseTimes * kCrowdedRow;
+    const bool crowded = h->N > kPressureCrowded && seen[4] >= kDenseTimes * kCrowdedRow;
     const bool same = row == old || (row != 0 && old != 0 && row <= old + old / 4 && old <= row + row / 4);
     if (same && crowded == h->crowded) return MG_OK;
     h->epoch++;
@@ -1086,7 +1089,7 @@ void launch_pressure(mg_handle* h, unsigned nb, const DS& d)
     auto rows = [&](auto kernel, unsigned waves) {
         hipLaunchKernelGGL(kernel, dim3(nblk(h->N, 64)), dim3(64 * waves), 0, h->st, d, h->p, h->g);
     };
-    if (rows_of_three(h, d) && !(h->crowded && h->N > kPressureRows9)) {
+    if (rows_of_three(h, d) && !h->crowded) {
         if (h->N <= kPressureRows9)
             return poly6 ? rows(k_pressure_rows<MG_SPH_POLY6_SPIKY, 9>, 9) : rows(k_pressure_rows<MG_SPH_REFERENCE, 9>, 9);
         return poly6 ? rows(k_pressure_rows<MG_SPH_POLY6_SPIKY, 3>, 3) : rows(k_pressure_rows<MG_SPH_REFERENCE, 3>, 3);

@@ -3,6 +3,7 @@ zero distance is no hit), but the advance separates them, so in the same step th
 masks of the pressure pass, which the diffusion visits, have to hold such pairs. Bit-equal to the
 oracle in every form of the step: split by rows, a lane per particle (the crowded models' pressure,
 and wide cells), and the batch's merged, dispatch and persistent forms."""
+import ctypes as C
 import sys
 
 import numpy as np
@@ -40,8 +41,8 @@ def paired(dims, b, spacing, seed=11, pairs=200):
 
 @pytest.mark.parametrize("dims,b,spacing,sph", [
     ((8, 8, 8), 4, 0.5, 0),        # nine wavefronts per 64 particles
-    ((41, 42, 41), 4, 0.26, 0),    # 70,602 crowded throughout: the pressure a lane per particle
-    ((41, 42, 41), 0, 0.26, 1),
+    ((55, 56, 57), 4, 0.28, 0),    # 175,560 crowded throughout: the pressure a lane per particle
+    ((55, 56, 57), 0, 0.28, 1),
     ((40, 40, 40), 4, 0.5, 0),     # three wavefronts
 ])
 def test_single_model(built, dims, b, spacing, sph):
@@ -52,6 +53,9 @@ def test_single_model(built, dims, b, spacing, sph):
         sim.set_sph_kernels(sph)
         sim.Run2PhysicalSort()
         sim.step(1, sc.dt, sc.flags)
+    crowded = C.c_int()
+    assert g.lib.mg_debug_crowding(g.h, None, C.byref(crowded), None) == F.MG_OK
+    assert crowded.value == int(sc.n > 163840)
     compare_all(g, o, "one step")
     for sim in (g, o):
         sim.step(2, sc.dt, sc.flags | (F.STEP_GRAPH if sim is g else 0))

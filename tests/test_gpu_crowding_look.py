@@ -41,7 +41,7 @@ def scale(sim, f, only=slice(None)):
 
 @pytest.mark.parametrize("drop", [0, 1000])
 def test_choice_follows_the_particles(built, drop):
-    sc = with_drop((32, 32, 64), 4, True, 0.5, drop)
+    sc = with_drop((56, 56, 56), 4, True, 0.5, drop)
     sc.buffers[F.FVEL][:] = 0
     sc.buffers[F.FVEVAL][:] = 0
     sc.params.diff_scale = 1e-5  # hundreds of neighbours: concentrations stay finite
