@@ -395,6 +395,7 @@ struct mg_handle {
     bool rehome_due = false;
     int steps_since_rehome = 0;
     int looked_at = 0; /* steps_since_rehome when the crowding was last looked at */
+    int look_in = 0;   /* pressure passes of phase calls until it is looked at */
     double time = 0.0;
     std::vector<void*> allocs;
     /* phase timing (mg_step_timed) */
@@ -925,6 +926,14 @@ void count_crowding(mg_handle* h, uint32_t* stat)
     hipLaunchKernelGGL(k_rehome_dense<true>, dim3(nblk(h->N)), dim3(256), 0, h->st, now, h->g, stat);
 }
 
+/* How often the crowding alone is looked at: particles that crowd between two re-homings would step in
+ * the wrong forms for up to kRehomeSteps (262,144 particles with a drop, all crowded later: 3,980 us a
+ * step with the drop's list, 3,645 without; without a drop 1,443 and 1,371), and phase calls number no
+ * homes at all (262,144 particles at rows of 282, pressure, force, advance and sort: 1,458 us split over
+ * three wavefronts, 1,332 with the pressure's lanes). Two kernels and a 20-byte read: 80 us at 262,144
+ * particles. */
+const int kLookSteps = 256;
+
 /* What the counts say of the steps to come: whether they list dense groups, from which width on, and
  * whether the pressure keeps one lane per particle. Captured steps have the choice in them: a width
  * within a quarter of the old one is no new choice. */
@@ -939,6 +948,7 @@ int choose_forms(mg_handle* h, const uint32_t seen[5])
     const uint32_t row = few && h->DL ? seen[4] : 0u, old = h->dense_row;
     const bool crowded = h->N > kPressureCrowded && seen[4] >= kDenseTimes * kCrowdedRow;
     const bool same = row == old || (row != 0 && old != 0 && row <= old + old / 4 && old <= row + row / 4);
+    h->look_in = kLookSteps;
     if (same && crowded == h->crowded) return MG_OK;
     h->epoch++;
     h->dense_row = row;
@@ -946,10 +956,6 @@ int choose_forms(mg_handle* h, const uint32_t seen[5])
     return MG_OK;
 }
 
-/* The crowding alone, every kLookSteps: particles that crowd between two re-homings would step in the
- * wrong forms for up to kRehomeSteps (262,144 particles with a drop, all crowded later: 3,980 us a step
- * with the drop's list, 3,645 without; without a drop 1,443 and 1,371). Two kernels and a 20-byte read. */
-const int kLookSteps = 256;
 int look(mg_handle* h)
 {
     CHK(staging(h, 256));
@@ -1561,6 +1567,7 @@ int ensure_force(mg_handle* h)
  * same positions and grid may share them, as inside one inner loop */
 int do_pressure(mg_handle* h, uint64_t* hm = nullptr)
 {
+    if (h->N > kPressureCrowded && h->grid_scanned && --h->look_in < 0) CHK(look(h));
     PhaseScope ps(h, MG_PH_PRESSURE);
     DS d = make_ds(h);
     d.HMW = hm;

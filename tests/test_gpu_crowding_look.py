@@ -70,3 +70,26 @@ def test_choice_follows_the_particles(built, drop):
             assert_bits_equal(sim.download(buf), ref.download(buf), f"scaled by {f}: {F.BUFFER_NAMES[buf]}")
     for s in (sim, ref):
         s.close()
+
+
+@pytest.mark.parametrize("n_side,want", [(56, 1), (54, 0)])  # 175,616 and 157,464: the rule's line between
+def test_phase_calls_choose_too(built, n_side, want):
+    """A program of phase calls alone numbers no homes; its pressure passes look by themselves."""
+    sc = with_drop((n_side,) * 3, 0, False, 0.28, 0)
+    say("case: phase calls look,", sc.n)
+    sim = FluidSystem(sc.n, sc.b)
+    sim.load_scene(sc)
+    sim.Run2PhysicalSort()
+    assert crowding(sim)[1] == 0
+    sim.Run2InnerPhysicalLoop(DT)
+    assert crowding(sim)[1] == want
+    sim.Run2PhysicalSort()
+    p = sim.download(F.FPOS)
+    mid = p[:, :3].mean(0)
+    p[:, :3] = mid + (p[:, :3] - mid) * np.float32(0.5 / 0.28)
+    sim.upload(F.FPOS, p)
+    for _ in range(257):
+        sim.Run2PhysicalSort()
+        sim.ComputePressureCL()
+    assert crowding(sim)[1] == 0
+    sim.close()
