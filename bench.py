@@ -33,7 +33,7 @@ def kernels_of_phase(scene, crowded: bool = False) -> dict:
     `crowded` as mg_debug_crowding tells it. A model with bonds splits its force only with bond
     records (cut-off 1)."""
     rows = int(scene.grid.srch) == 3
-    force_rows = rows and (scene.n <= 147456 and float(scene.params.r2) == 1.0 if scene.b else scene.n <= 131072)
+    force_rows = rows and (scene.n <= 147456 and float(scene.params.r2) == 1.0 if scene.b else scene.n <= 122880)
     genes = bool(scene.flags & 1)
     return {"pressure": "k_pressure_rows" if rows and not crowded else "k_pressure",
             "force": "k_force_advance_rows" if force_rows else "k_force_advance",

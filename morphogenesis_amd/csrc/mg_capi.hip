@@ -1081,12 +1081,13 @@ template <int NX, int CAP = BAND_CAP> constexpr size_t band_lds(unsigned threads
  *   force      32,768: 15.7 / 21.6 / 45.6;  110,592: 43 / 53 / 53;  140,608: 53 / 66 / 59;
  *              175,616: 67 / 80 / 63;  262,144: 101 / 110 / 73
  *             [46,656: 25 / 21 / 41;  64,000: 32 / 22 / 42;  110,592: 50 / 37 / 41;  140,608: 63 / 48 / 47]
+ *             (a lattice at rest, three / one lane: 110,592 34 / 34, 120,050 36 / 35, 130,000 44 / 35)
  * Nine wavefronts win while the chip has wavefront slots to spare (49,152 particles are three
  * workgroups per CU); beyond, three rows per wavefront keep more of the chip busy per byte of
  * LDS, until the one-lane form fills it too. The force with bonds has no use for three: its two
  * bond wavefronts then idle longer than the rows take. */
 const int kPressureRows9 = 49152;
-const int kForceRows9 = 147456, kForceRows9NoBonds = 40960, kForceRows3NoBonds = 131072;
+const int kForceRows9 = 147456, kForceRows9NoBonds = 40960, kForceRows3NoBonds = 122880;
 
 /* the pressure and force launches for the handle's SPH kernels */
 void launch_pressure(mg_handle* h, unsigned nb, const DS& d)
