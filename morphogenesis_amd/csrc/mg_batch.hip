@@ -293,8 +293,9 @@ int persist_launch(mg_batch* b, int q)
  * 16,112 (16 instances): 61 / 318 / 155; 201,509 (32): 211 / 664 / 384; 930,148 (64): 750 / 1,800 /
  * 939; 1,884,496 (128): 1,424 / 2,921 / 1,621; 3,721,327 (200): 2,651 / 4,997 / 3,006. One launch
  * per phase for all size classes has one tail instead of one per class, and it takes the sweeps
- * split by rows; larger batches keep the persistent launch as their default and
- * mg_batch_autotune decides. */
+ * split by rows. Larger batches keep the persistent launch as their default although the merged form
+ * is the faster there too (256 instances of 4,581,500 particles: 3,061 / 6,176 / 3,619): their callers
+ * choose it (mg_batch_set_form) or let mg_batch_autotune. */
 const size_t kBatchMerged = 1u << 22;
 
 bool merged_wanted(const mg_batch* b)
@@ -348,8 +349,11 @@ int merged_build(mg_batch* b, float dt, unsigned flags)
 }
 
 /* One fused step of every instance in the merged form. The split by rows follows the single
- * model's rules (launch_pressure, launch_force_advance, launch_diffuse_rows) at the particles of
- * the whole batch: what counts is how far they fill the chip. */
+ * model's sizes (launch_pressure, launch_force_advance, launch_diffuse_rows) at the particles of
+ * the whole batch: what counts is how far they fill the chip. Not its rules for crowded cells and
+ * for models without bonds: one instance without bond slots keeps the force of all in one lane per
+ * particle, and no dense groups are listed. Crowded batches, merged / dispatch at blocks of 256, us:
+ * 64 instances of 8,000 at rows of 111 1,825 / 1,999, 200 of 8,800 at rows of 171 7,001 / 7,327. */
 int merged_launch(mg_batch* b, int q)
 {
     const BatchInst* I = b->RI[q];

@@ -900,11 +900,11 @@ int normalize(mg_handle* h)
  * in the same order: no result changes. */
 const int kRehomeSteps = 2048;
 /* Dense groups are listed when their particles are few: where crowding is common no group outlasts
- * the rest, and splitting 1,024 of 4,096 groups costs more than it gives. 262,144 particles, force
- * and diffusion with lists against a lane per particle, us: spacing 0.42 (rows of 40 on average, some
- * beyond 64) 162 + 223 / 117 + 121; spacing 0.3 (111 on average) a step of 1,460 / 1,098. With few, see
- * dense_listed: 1,014,784 particles 352 + 368 / 444 + 554; 4,194,304 with cells of up to 147: 1,280 +
- * 1,728 / 1,531 + 1,839. */
+ * the rest, and splitting 1,024 of 4,096 groups costs more than it gives. 262,144 particles, force +
+ * diffusion with lists / a lane per particle, us: spacing 0.42 (rows of 40 on average, some beyond 64)
+ * 172 + 231 / 122 + 123; spacing 0.3 (111 on average) 516 + 617 / 397 + 402. With few, see
+ * dense_listed: 1,014,784 particles 350 + 355 / 444 + 554; 4,194,304 with cells of up to 147: 1,283 +
+ * 1,622 / 1,531 + 1,839. */
 const int kDenseShare = 8;
 /* Models of more than kPressureCrowded particles whose rows hold this many candidates on average keep the
  * one-lane pressure (bands beyond the LDS stage: the one-lane sweep has more loads in flight). us, split
@@ -1075,9 +1075,8 @@ template <int NX, int CAP = BAND_CAP> constexpr size_t band_lds(unsigned threads
 /* Which models take the sweeps split by rows (k_*_rows; three cells per axis, the row-structured
  * grid). us per launch by particles, nine wavefronts per 64 particles / three / one lane each (the
  * bonded tissue drifting off the cell faces; in brackets the fluid without bonds):
- *   pressure   32,768: 17.5 /  29.0 /  66.6;  46,656: 27.4 / 30.5 / 66.4;  54,872: 35.5 / 30.8 / 66.4;
- *              110,592: 55 / 40 / 68;  262,144: 112 / 68 / 92;  512,000: 237 / 142 / 183
- *              (with the exact test of candidates; three at 262,144 take 61.5 with rs_test's)
+ *   pressure   32,768: 17.4 / 25.3 / 63.9;  46,656: 26.8 / 26.7 / 64.8;  54,872: 34.9 / 28.2 / 64.5;
+ *              110,592: 54 / 36 / 67;  262,144: 110 / 63 / 85;  512,000: 218 / 125 / 172
  *   force      32,768: 15.7 / 21.6 / 45.6;  110,592: 43 / 53 / 53;  140,608: 53 / 66 / 59;
  *              175,616: 67 / 80 / 63;  262,144: 101 / 110 / 73
  *             [46,656: 25 / 21 / 41;  64,000: 32 / 22 / 42;  110,592: 50 / 37 / 41;  140,608: 63 / 48 / 47]
@@ -1194,8 +1193,8 @@ DiffPlan diff_plan(const mg_handle* h)
 
 /* Models whose diffusion and gene action run split by rows (k_diffuse_rows; for the diffusion also
  * three cells per axis on the row-structured grid): fused with the insert 32,768 particles
- * 24.8 us against 48.8 with a lane per particle, 46,656: 39.9 / 49.3, 54,872: 46.3 / 50.3,
- * 64,000: 53.9 / 50.5. */
+ * 22.5 us against 47.0 with a lane per particle, 46,656: 35.8 / 47.7, 54,872: 41.5 / 48.0,
+ * 64,000: 49.2 / 48.1. */
 template <int PART> void launch_diffuse_rows(mg_handle* h, const DS& d, const DiffPlan& dp)
 {
     hipLaunchKernelGGL(k_diffuse_rows<PART>, dim3(nblk(h->N, 64)), dim3(64 * RS_ROWS), 0, h->st, d, h->p, h->g, h->gen, dp);

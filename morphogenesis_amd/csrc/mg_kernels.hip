@@ -1448,7 +1448,7 @@ __global__ __launch_bounds__(64 * W, RS_OCC) void k_pressure_rows(DS d, MgParams
  * d.dense_row candidates (64, where the hit masks end, and four times the mean); the force and the
  * diffusion take them nine wavefronts each, in a launch of their own, and the one-lane kernels pass
  * them by. A falling column and four
- * drops, 1,014,784 particles: force 444 -> 276 + 85 us, diffusion and genes 554 -> 236 + 142. */
+ * drops, 1,014,784 particles: force 444 -> 274 + 76 us, diffusion and genes 554 -> 237 + 118. */
 __device__ __forceinline__ bool dense_listed(const DS& d, uint32_t bid)
 {
     return d.DL && d.DL[1 + MG_DENSE_MAX + bid * (blockDim.x >> 6) + (threadIdx.x >> 6)] != 0u;
@@ -2396,7 +2396,7 @@ __global__ LAUNCH_BOUNDS_256 void k_insert_next(DS d, MgGrid g)
  *
  * 512 particles 34 -> 17 us, 29,667 44 -> 20 (a lane per particle was one serial chain: sweep,
  * then every gene in turn); with the chip full it loses, as most wavefronts wait while few
- * work (64,000 particles 50 -> 54 us), so larger models keep a lane per particle. */
+ * work (64,000 particles 48 -> 49 us, 110,592 51 -> 71), so larger models keep a lane per particle. */
 #define RS_DIFFUSE 1
 #define RS_GENES 2
 #define RS_INSERT 4
