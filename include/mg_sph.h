@@ -6,7 +6,8 @@
  * (src/fluid.h:138-206): mg_upload / mg_download take host memory laid out exactly like
  * the reference's host mirrors m_Fluid.mcpu[buf_id]. Every function returns MG_OK (0) or
  * a negative MG_ERR_* code; mg_last_error() describes the last failure. Step functions
- * are asynchronous on the handle's stream; mg_download, mg_get_counts and mg_sync wait.
+ * are asynchronous on the handle's stream, but for a short read of the device after a sort, every
+ * 2,048 steps and, above 57,344 particles, every 256; mg_download, mg_get_counts and mg_sync wait.
  * A handle is not thread-safe.
  *
  * Each declaration names the reference interface it replaces.
